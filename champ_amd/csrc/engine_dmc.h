@@ -164,117 +164,200 @@ __global__ void k_dmc_gather(const double *st_src, double *st_dst, int64_t strid
 
 // ---------------------------------------------------------------------------
 // split_join (qmc/dmc/dmc_elec/split_join_mod.f90:3-219) on the device, one
-// workgroup: the same loops and draws as the host routine qmcw_split_join
-// (joins in walker order with one rannyu per joined pair; the split
-// threshold from the sorted weights; splits into the holes last-first, each
-// copy with four 12-bit limbs drawn from the branching stream; compaction).
-// The joins, splits and compaction are sequential in the walker index and
-// the stream, so one lane runs them; the sort of the weights runs on every
-// lane (bitonic, over the next power of two, padded with +inf).
+// workgroup: the same decisions and draws as the host routine
+// qmcw_split_join (joins in walker order with one rannyu per joined pair; the
+// split threshold from the sorted weights; splits into the holes last-first,
+// each copy with four 12-bit limbs drawn from the branching stream;
+// compaction).  Only the walkers that take part in a join or a split are
+// sequential: every lane marks them (a bit per walker, and the weights of a
+// chunk, in LDS) and one lane walks the marked ones.  A lane that walked all
+// walkers through global memory was bound by one load latency per walker
+// (2,008 us for the dimer's 4,096 walkers; a DMC generation of theirs went from
+// 5.45 to 3.64 ms, 1.8 ms of it here).
+// The threshold needs a place in the sorted weights only when the population
+// nears the capacity; below that the reference's index clamps to the first
+// element, the smallest weight, and the sort (bitonic, over the next power of
+// two, padded with +inf) is left out.  The compaction's copies are resolved to
+// their final sources first and then run on every lane.
 // w[roundup(mwalk, 8)]: in, the n weights; out, the new population's
 // weights, padded with 0 to a multiple of 8.  rng[mwalk][4]: the walkers' streams, moved
 // with them.  origin[mwalk]: the old walker each new one copies.  sortbuf:
 // npow2 doubles; under: n ints.  res: {walkers, branching events, status
 // (0 ok, 1 more walkers than mwalk), walkers padded to a multiple of 8}.
+constexpr int kSjChunk = 4096;   // walkers whose marks and weights one pass keeps in LDS
 __global__ __launch_bounds__(1024) void k_split_join(double *w, int n, int mwalk, int *brng, int *rng,
                                                      int *origin, double *sortbuf, int npow2, int *under,
                                                      int *res) {
   const int t = threadIdx.x, nt = blockDim.x;
-  __shared__ int s_nunder, s_nbr;
+  __shared__ unsigned long long s_bits[kSjChunk / 64];
+  __shared__ double s_w[kSjChunk], s_min[16];
+  __shared__ int s_cnt[16];
+  __shared__ int s_nu, s_nbr, s_n2, s_status;
   for (int i = t; i < mwalk; i += nt) origin[i] = i;
-  if (t == 0) {
-    int st4[4] = {brng[0], brng[1], brng[2], brng[3]};
-    int nu = 0, ipair = 0, iw2 = 0, nbr = 0;
-    for (int iw = 0; iw < n; iw++) {
-      const double wi = w[iw];
-      if (!(wi < 0.5)) continue;
-      if (wi == 0.0) {
-        nbr++;
-        under[nu++] = iw;
-      } else if (ipair == 0) {
-        ipair = 1;
-        iw2 = iw;
-      } else {
-        nbr++;
-        ipair = 0;
-        const double wt = wi + w[iw2];
-        if (rannyu(st4) > wi / wt) {
-          w[iw2] = wt;
-          under[nu++] = iw;
-        } else {
-          w[iw] = wt;
-          under[nu++] = iw2;
-        }
-      }
+  // ---- joins
+  int st4[4] = {brng[0], brng[1], brng[2], brng[3]};   // lane 0 advances it
+  int nu = 0, ipair = 0, iw2 = 0, nbr = 0;
+  double wi2 = 0.0;
+  for (int base = 0; base < n; base += kSjChunk) {
+    const int m = min(kSjChunk, n - base);
+    for (int i = t; i < kSjChunk; i += nt) {
+      const double wi = i < m ? w[base + i] : 1.0;
+      s_w[i] = wi;
+      const unsigned long long b = __ballot(wi < 0.5);
+      if ((i & 63) == 0) s_bits[i >> 6] = b;
     }
+    __syncthreads();
+    if (t == 0)
+      for (int q = 0; q < (m + 63) / 64; q++)
+        for (unsigned long long b = s_bits[q]; b; b &= b - 1) {
+          const int il = 64 * q + __ffsll(b) - 1, iw = base + il;
+          const double wi = s_w[il];
+          if (wi == 0.0) {
+            nbr++;
+            under[nu++] = iw;
+          } else if (ipair == 0) {
+            ipair = 1;
+            iw2 = iw;
+            wi2 = wi;
+          } else {
+            nbr++;
+            ipair = 0;
+            const double wt = wi + wi2;
+            if (rannyu(st4) > wi / wt) {
+              w[iw2] = wt;
+              under[nu++] = iw;
+            } else {
+              w[iw] = wt;
+              under[nu++] = iw2;
+            }
+          }
+        }
+    __syncthreads();
+  }
+  if (t == 0) { s_nu = nu; s_nbr = nbr; }
+  __syncthreads();
+  // ---- the split threshold
+  const int first = n - (mwalk - (n - s_nu));   // n - nmax_dupl, a 1-based index into the sorted weights
+  double wmin = __builtin_inf();
+  for (int i = t; i < n; i += nt) wmin = fmin(wmin, w[i]);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) wmin = fmin(wmin, __shfl_xor(wmin, o, 64));
+  if ((t & 63) == 0) s_min[t >> 6] = wmin;
+  __syncthreads();
+  for (int i = 0; i < nt / 64; i++) wmin = fmin(wmin, s_min[i]);
+  if (n == 0) wmin = 0.0;
+  bool sorted = false;
+  auto sort = [&]() {
+    for (int i = t; i < npow2; i += nt) sortbuf[i] = i < n ? w[i] : __builtin_inf();
+    __syncthreads();
+    for (int k = 2; k <= npow2; k <<= 1)
+      for (int j = k >> 1; j > 0; j >>= 1) {
+        for (int i = t; i < npow2; i += nt) {
+          const int l = i ^ j;
+          if (l > i) {
+            const double a = sortbuf[i], b = sortbuf[l];
+            const bool up = (i & k) == 0;
+            if ((a > b) == up) { sortbuf[i] = b; sortbuf[l] = a; }
+          }
+        }
+        __syncthreads();
+      }
+    sorted = true;
+  };
+  // the weight at place i of the sorted weights (clamped below, as the reference's)
+  auto at1 = [&](int i) {
+    if (i <= 1) return wmin;
+    if (!sorted) sort();
+    return sortbuf[i - 1];
+  };
+  double wt_split = fmax(2.0, at1(first));
+  int nmore = 0;
+  for (int i = max(1, first) + t; i <= n; i += nt) {
+    const double r = (first <= 1 ? w[i - 1] : sortbuf[i - 1]) / wt_split;
+    nmore += r >= 8.0 ? 3 : r >= 4.0 ? 2 : r >= 2.0 ? 1 : 0;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) nmore += __shfl_xor(nmore, o, 64);
+  if ((t & 63) == 0) s_cnt[t >> 6] = nmore;
+  __syncthreads();
+  nmore = 0;
+  for (int i = 0; i < nt / 64; i++) nmore += s_cnt[i];
+  wt_split = (first + nmore < n) ? fmax(2.0, at1(first + nmore)) : 1e99;
+  // ---- splits: a copy put into a hole further on is met again
+  int n2 = n, status = 0;
+  for (int base = 0; base < n; base += kSjChunk) {
+    const int m = min(kSjChunk, n - base);
+    __syncthreads();
+    for (int i = t; i < kSjChunk; i += nt) {
+      const double wi = i < m ? w[base + i] : 0.0;
+      s_w[i] = wi;
+      const unsigned long long b = __ballot(wi > wt_split);
+      if ((i & 63) == 0) s_bits[i >> 6] = b;
+    }
+    __syncthreads();
+    if (t == 0)
+      for (int q = 0; q < (m + 63) / 64 && !status; q++)
+        while (s_bits[q]) {
+          const int k = __ffsll(s_bits[q]) - 1, il = 64 * q + k, iw = base + il;
+          s_bits[q] &= s_bits[q] - 1;
+          nbr++;
+          int dst;
+          if (nu > 0) {
+            dst = under[--nu];
+          } else {
+            if (n2 >= mwalk) { status = 1; break; }
+            dst = n2++;
+          }
+          const double wh = s_w[il] * 0.5;
+          w[iw] = wh;
+          w[dst] = wh;
+          origin[dst] = origin[iw];
+          const int dl = dst - base;
+          if (dl > il && dl < m) {
+            s_w[dl] = wh;
+            if (wh > wt_split) s_bits[dl >> 6] |= 1ull << (dl & 63);
+          }
+          for (int c = 0; c < 4; c++) rng[4 * dst + c] = (int)(rannyu(st4) * 4096.0) & 4095;
+          rng[4 * dst + 3] |= 1;
+        }
+  }
+  if (t == 0) {
+    s_nu = nu; s_nbr = nbr; s_n2 = n2; s_status = status;
     brng[0] = st4[0]; brng[1] = st4[1]; brng[2] = st4[2]; brng[3] = st4[3];
-    s_nunder = nu;
-    s_nbr = nbr;
   }
   __syncthreads();
-  for (int i = t; i < npow2; i += nt) sortbuf[i] = i < n ? w[i] : __builtin_inf();
+  // ---- compaction: hole under[nh - 1 - k] takes the record n2 - 1 - k, for
+  // k = 0, 1, ...; a record that an earlier k filled is followed back to
+  // where its content came from (at[]: the k that filled record nf + i)
+  const int nh = s_status ? 0 : s_nu, nf = s_n2 - nh;
+  int *at = reinterpret_cast<int *>(sortbuf);
+  for (int i = t; i < nh; i += nt) at[i] = -1;
   __syncthreads();
-  for (int k = 2; k <= npow2; k <<= 1)
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      for (int i = t; i < npow2; i += nt) {
-        const int l = i ^ j;
-        if (l > i) {
-          const double a = sortbuf[i], b = sortbuf[l];
-          const bool up = (i & k) == 0;
-          if ((a > b) == up) { sortbuf[i] = b; sortbuf[l] = a; }
-        }
-      }
-      __syncthreads();
-    }
-  if (t == 0) {
-    int nu = s_nunder, nbr = s_nbr;
-    const int nafter = n - nu, nmax_dupl = mwalk - nafter;
-    auto at1 = [&](int i) { return n > 0 ? sortbuf[max(1, i) - 1] : 0.0; };   // 1-based, clamped below
-    double wt_split = fmax(2.0, at1(n - nmax_dupl));
-    int nmore = 0;
-    for (int iw = max(1, n - nmax_dupl); iw <= n; iw++) {
-      const double r = sortbuf[iw - 1] / wt_split;
-      if (r >= 8.0) nmore += 3;
-      else if (r >= 4.0) nmore += 2;
-      else if (r >= 2.0) nmore += 1;
-    }
-    wt_split = (n - nmax_dupl + nmore < n) ? fmax(2.0, at1(n - nmax_dupl + nmore)) : 1e99;
-    int st4[4] = {brng[0], brng[1], brng[2], brng[3]};
-    int n2 = n, status = 0;
-    for (int iw = 0; iw < n && !status; iw++) {
-      if (!(w[iw] > wt_split)) continue;
-      nbr++;
-      int dst;
-      if (nu > 0) {
-        dst = under[--nu];
-      } else {
-        if (n2 >= mwalk) { status = 1; break; }
-        dst = n2++;
-      }
-      w[iw] *= 0.5;
-      w[dst] = w[iw];
-      origin[dst] = origin[iw];
-      for (int k = 0; k < 4; k++) rng[4 * dst + k] = (int)(rannyu(st4) * 4096.0) & 4095;
-      rng[4 * dst + 3] |= 1;
-    }
-    while (!status && nu > 0) {
-      const int dst = under[--nu], src = n2 - 1;
-      n2--;
-      if (dst != src) {
-        w[dst] = w[src];
-        origin[dst] = origin[src];
-        for (int k = 0; k < 4; k++) rng[4 * dst + k] = rng[4 * src + k];
-      }
-    }
-    brng[0] = st4[0]; brng[1] = st4[1]; brng[2] = st4[2]; brng[3] = st4[3];
-    const int nl = (n2 + 7) / 8 * 8;     // the buffers hold mwalk rounded up to 8
-    for (int d = n2; d < nl; d++) {       // padding records: copies of the first walker, weight 0
-      origin[d] = origin[0];
-      w[d] = 0.0;
-      for (int k = 0; k < 4; k++) rng[4 * d + k] = rng[k];
-    }
-    res[0] = n2; res[1] = nbr; res[2] = status; res[3] = nl;
+  for (int k = t; k < nh; k += nt) {
+    const int dst = under[nh - 1 - k];
+    if (dst >= nf) at[dst - nf] = k;
   }
+  __syncthreads();
+  for (int k = t; k < nh; k += nt) {
+    const int dst = under[nh - 1 - k];
+    if (dst >= nf) continue;
+    int src = s_n2 - 1 - k, kk = k;
+    for (int f = at[src - nf]; f >= 0 && f < kk; f = at[src - nf]) {
+      kk = f;
+      src = s_n2 - 1 - f;
+    }
+    w[dst] = w[src];
+    origin[dst] = origin[src];
+    for (int c = 0; c < 4; c++) rng[4 * dst + c] = rng[4 * src + c];
+  }
+  __syncthreads();
+  const int nl = (nf + 7) / 8 * 8;      // the buffers hold mwalk rounded up to 8
+  for (int d = nf + t; d < nl; d += nt) {   // padding records: copies of the first walker, weight 0
+    origin[d] = origin[0];
+    w[d] = 0.0;
+    for (int c = 0; c < 4; c++) rng[4 * d + c] = rng[c];
+  }
+  if (t == 0) { res[0] = nf; res[1] = s_nbr; res[2] = s_status; res[3] = nl; }
 }
 
 // ---------------------------------------------------------------------------

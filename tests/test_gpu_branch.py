@@ -48,6 +48,29 @@ def test_device_split_join_matches_host_routine():
     assert nsplit > 5
 
 
+# populations about the 4,096 walkers whose marks one pass of the kernel keeps,
+# with room (no sort of the weights) and near the capacity (sorted), and
+# weights that leave holes after the splits (compaction) or need them all
+@pytest.mark.parametrize("n", [0, 1, 63, 64, 65, 4095, 4096, 4097, 8193])
+@pytest.mark.parametrize("room", [0, 3, None])
+@pytest.mark.parametrize("spread", [0.4, 1.2, 2.2])
+def test_device_split_join_at_chunk_edges(n, room, spread):
+    lib = abi.load_library()
+    g = np.random.default_rng(n + int(10 * spread))
+    w = np.exp(g.normal(0.0, spread, n))
+    w[g.random(n) < 0.05] = 0.0
+    if spread > 2:
+        w[g.random(n) < 0.3] *= 0.01
+    cap = max(1, 2 * n if room is None else n + room)
+    rng = g.integers(0, 4096, (cap, 4), dtype=np.int32)
+    sh, h = _run(lib.qmcw_split_join, w, cap, [7, 11, 13, 17], rng)
+    sg, gp = _run(lib.qmcw_split_join_gpu, w, cap, [7, 11, 13, 17], rng)
+    assert sh == sg
+    if sh == 0:
+        for a, c in zip(h, gp):
+            assert np.array_equal(np.asarray(a), np.asarray(c))
+
+
 def test_dmc_generations_on_the_host_split_join(monkeypatch):
     from test_gpu_dmc import test_dmc_generations_match_oracle
     monkeypatch.setenv("QMCW_HOST_SPLIT_JOIN", "1")
