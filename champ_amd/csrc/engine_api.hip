@@ -58,7 +58,8 @@ struct qmcw_handle {
   // one VMC step captured as a HIP graph (qmcw_vmc_run_device) and its key
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
-  int graph_ok = 0, graph_G = 0, graph_Wl = 0, graph_derivs = 0;
+  int graph_ok = 0, graph_Wl = 0, graph_derivs = 0;
+  int64_t graph_G = 0;
   double graph_delta = 0.0, graph_fbias = 0.0;
   const double *graph_st = nullptr;
   int use_graph = 1;
@@ -96,6 +97,8 @@ struct qmcw_handle {
   int host_split_join = 0;    // QMCW_HOST_SPLIT_JOIN=1: split_join on the host
   int no_gproj_mfma = 0;      // QMCW_NO_GPROJ_MFMA=1: the projection on VALU in k_full_det
   int no_een_tab = 0;         // QMCW_NO_EEN_TAB=1: the move's e-e-n terms summed per pair
+  int nlpp_waves = -1;        // the autotuner's choice for k_full_nlpp_tiles (-1: the rule)
+  int nlpp_tiles_env = -1;    // QMCW_NLPP_TILES: wavefronts per walker of k_full_nlpp_tiles (0: never used)
   int32_t brng[4] = {0, 0, 0, 1};
   // event timing of the device driver
   int prof = 0;
@@ -574,6 +577,27 @@ static void det_lds_inv(const qmcw_handle *h, KArgs &A, size_t &smem) {
   smem = tot;
 }
 
+// Wavefronts per walker of k_full_nlpp_tiles, 0 where k_full_nlpp's lane
+// groups are the faster way.  From this many (electron, centre) pairs on the
+// tiles won at every walker count and precision (lane groups -> tiles, us:
+// 25 electrons, 7 centres, 601 walkers 222 -> 129; 38, 9, 1,024: 541 -> 283;
+// 60, 14, 512: 1,883 -> 474; the 98-electron chain, 50, 2,048: 18,100 ->
+// 6,660, FP64); below it the lane groups fill the GPU when there are many
+// walkers (8, 2, 16,384: 555 against 1,041) and the tiles when there are few
+// (8, 2, 1,024: 235 against 104), which the autotuner finds out.  A block
+// gets as many wavefronts as leave two on every SIMD.
+constexpr int kNlppTilePairs = 160;
+static int nlpp_tile_waves(const qmcw_handle *h) {
+  const DevSys &S = h->A.S;
+  if (S.nloc == 0 || S.nordc < 2 || S.nctype * S.nterms > kMaxCtype * kMaxTerms) return 0;
+  if (h->nlpp_tiles_env >= 0) return std::min(h->nlpp_tiles_env, kNlppWaves);
+  if (h->nlpp_waves >= 0) return h->nlpp_waves;      // the autotuner's choice
+  if (S.N * S.M < kNlppTilePairs) return 0;
+  int nw = 1;
+  while (nw < kNlppWaves && (int64_t)h->Wl * nw < 8 * (int64_t)h->ncu) nw *= 2;
+  return nw;
+}
+
 // The arguments of the full evaluation's kernels for the handle's current
 // state (keep: take the rows the committed moves kept): jas for k_full_jas
 // (and k_deriv_jas), det for k_full_det, k_gproj_mfma and k_full_fin (and
@@ -628,6 +652,7 @@ static void eval_args(const qmcw_handle *h, bool derivs, bool keep, EvalArgs &e)
       e.nlpp.lds_dnlpp = per_lane_d;
       e.dnlpp_smem = blk_d;
     }
+    e.nlpp.nlpp_tiles = nlpp_tile_waves(h);
     // psp_nonloc_orb's contraction on FP64 MFMA after k_deriv_nlpp
     e.nlpp.pnl_mfma = h->no_gproj_mfma ? 0 : 1;
   }
@@ -1235,6 +1260,7 @@ extern "C" int qmcw_create(const qmcw_system *s, int32_t nwalk, int32_t precisio
   if (const char *e = getenv("QMCW_HOST_SPLIT_JOIN")) h->host_split_join = atoi(e) != 0;
   if (const char *e = getenv("QMCW_NO_GPROJ_MFMA")) h->no_gproj_mfma = atoi(e) != 0;
   if (const char *e = getenv("QMCW_NO_EEN_TAB")) h->no_een_tab = atoi(e) != 0;
+  if (const char *e = getenv("QMCW_NLPP_TILES")) h->nlpp_tiles_env = std::max(0, atoi(e));
   {
     int dev = 0, n = 0;
     if (hipGetDevice(&dev) == hipSuccess &&
@@ -1557,7 +1583,8 @@ static void drop_graph(qmcw_handle *h) {
 // value changes.
 static int step_graph(qmcw_handle *h, double delta, double fbias) {
   const int derivs = h->sample_derivs;
-  const int gkey = h->Gk[0] | (h->Gk[1] << 8) | (h->Gk[2] << 16) | (h->Gk[3] << 24);
+  const int64_t gkey = h->Gk[0] | (h->Gk[1] << 8) | (h->Gk[2] << 16) | ((int64_t)h->Gk[3] << 24) |
+                       ((int64_t)(h->nlpp_waves + 1) << 32);
   if (h->graph_ok && h->graph_G == gkey && h->graph_Wl == h->Wl && h->graph_derivs == derivs &&
       h->graph_delta == delta && h->graph_fbias == fbias && h->graph_st == h->A.st)
     return QMCW_OK;
@@ -1651,9 +1678,9 @@ extern "C" int qmcw_vmc_run_device(qmcw_handle *h, int32_t nstep, double delta, 
 // (engine_batch.h).  Argument sets: 0 the first full evaluation (each
 // handle's kept rows as it left them), 1 the steps.  Kernels per set: move,
 // jas, det (also gproj, fin), nlpp, rotqua; block offsets per kernel (move,
-// jas, det, nlpp, rotqua, gproj) and width (8, 16, 32, 64: the systems of
+// jas, det, nlpp, rotqua, gproj, nlpp tiles) and width (8, 16, 32, 64: the systems of
 // each width in their own launch; rotqua and gproj use the first).
-enum { KB_MOVE, KB_JAS, KB_DET, KB_NLPP, KB_ROT, KB_NARGS, KB_GPROJ = KB_NARGS, KB_NOFF };
+enum { KB_MOVE, KB_JAS, KB_DET, KB_NLPP, KB_ROT, KB_NARGS, KB_GPROJ = KB_NARGS, KB_TILES, KB_NOFF };
 constexpr int kBatchWidths[4] = {8, 16, 32, 64};
 static int width_index(int G) { return G == 8 ? 0 : (G == 16 ? 1 : (G == 32 ? 2 : 3)); }
 
@@ -1669,7 +1696,7 @@ struct qmcw_batch {
   int *dnw = nullptr;                        // [n]
   long long **dnacc = nullptr;               // [n]
   int nblk[KB_NOFF][4] = {};
-  size_t smem_move = 0, smem_det = 0, smem_nlpp = 0;
+  size_t smem_move = 0, smem_det = 0, smem_nlpp = 0, smem_tiles = 0;
   std::string err;
 };
 
@@ -1708,14 +1735,18 @@ static int batch_upload(qmcw_batch *b, int set, bool first) {
     A[(size_t)KB_ROT * n + s] = h->A;
     b->smem_det = std::max(b->smem_det, e.det_smem);
     b->smem_nlpp = std::max(b->smem_nlpp, e.nlpp_smem);
+    if (e.nlpp.nlpp_tiles)
+      b->smem_tiles = std::max(b->smem_tiles, sizeof(double) * nlpp_tiles_lds(h->A.S.N * h->A.S.M));
     const int Wl = h->Wl;
     const int gx = (int)(((int64_t)Wl * std::max(h->A.S.ns[0], h->A.S.ns[1]) + 63) / 64);
     const int gy = (h->A.S.NB + 63) / 64;
     const int cnt[KB_NOFF] = {Wl / (kWave / h->Gk[KC_MOVE]), Wl / (kWave / h->Gk[KC_JAS]),
-                              Wl / (kWave / h->Gk[KC_DET]), Wl / (kWave / h->Gk[KC_NLPP]),
-                              (Wl + kWave - 1) / kWave, e.det.gproj_mfma ? gx * gy * 2 : 0};
+                              Wl / (kWave / h->Gk[KC_DET]),
+                              e.nlpp.nlpp_tiles ? 0 : Wl / (kWave / h->Gk[KC_NLPP]),
+                              (Wl + kWave - 1) / kWave, e.det.gproj_mfma ? gx * gy * 2 : 0,
+                              e.nlpp.nlpp_tiles ? Wl : 0};
     const int wi[KB_NOFF] = {width_index(h->Gk[KC_MOVE]), width_index(h->Gk[KC_JAS]),
-                             width_index(h->Gk[KC_DET]), width_index(h->Gk[KC_NLPP]), 0, 0};
+                             width_index(h->Gk[KC_DET]), width_index(h->Gk[KC_NLPP]), 0, 0, 0};
     for (int k = 0; k < KB_NOFF; k++)
       for (int g = 0; g < 4; g++) {
         int *o = boff.data() + ((size_t)k * 4 + g) * (n + 1);
@@ -1787,6 +1818,12 @@ static void batch_eval(const qmcw_batch *b, int set) {
         c.nblocks = b->nblk[KB_NLPP][g];
         K.full_nlpp_batch(c);
       }
+    if (b->nblk[KB_TILES][0] > 0) {
+      c.B = batch_args(b, set, KB_NLPP, KB_TILES);
+      c.nblocks = b->nblk[KB_TILES][0];
+      c.smem = b->smem_tiles;
+      K.full_nlpp_tiles_batch(c);
+    }
   }
   for (int g = 0; g < 4; g++)
     if (b->nblk[KB_DET][g] > 0) {
@@ -1948,6 +1985,10 @@ extern "C" int qmcw_autotune(qmcw_handle *h, int32_t *chosen) {
   double *xin = h->io + (size_t)h->Wp * 8;
   const int prof_save = h->prof;
   drop_graph(h);
+  // the pseudopotential as tiles (k_full_nlpp_tiles) or in lane groups: the
+  // lane groups are not tried where the tiles always won
+  h->nlpp_waves = -1;
+  const bool tiles_only = nlpp_tile_waves(h) > 0 || h->nlpp_tiles_env >= 0;
   // the one-electron move is also timed as three launches (k_move_a/b/c)
   // unless QMCW_SPLIT_MOVE fixed the choice; the other classes once per width
   const int sm0 = h->split_forced ? h->split_move : 0, sm1 = h->split_forced ? h->split_move : 1;
@@ -1981,11 +2022,38 @@ extern "C" int qmcw_autotune(qmcw_handle *h, int32_t *chosen) {
     }
     for (int k = 0; k < 4; k++) {
       if (k != KC_MOVE && sm != sm0) continue;
+      if (k == KC_NLPP && tiles_only && h->nlpp_tiles_env != 0) continue;
       if (t[k] > 0 && t[k] < best[k]) {
         best[k] = t[k];
         bestG[k] = G;
         if (k == KC_MOVE) best_split = sm;
       }
+    }
+  }
+  if (h->nlpp_tiles_env < 0) {
+    h->nlpp_waves = 1;
+    if (nlpp_tile_waves(h) > 0) {        // a pseudopotential the tiles can take
+      int best_waves = tiles_only ? -1 : 0;
+      double tb = tiles_only ? 1e30 : best[KC_NLPP];
+      for (int nw = 1; nw <= kNlppWaves; nw *= 2) {
+        h->nlpp_waves = nw;
+        h->prof = 0;
+        launch_eval(h, false);
+        HIPCHK(h, hipStreamSynchronize(h->stream));
+        h->prof = 1;
+        h->ev_used = 0;
+        launch_eval(h, false);
+        HIPCHK(h, hipStreamSynchronize(h->stream));
+        for (size_t i = 0; i + 1 < h->ev_used; i += 2) {
+          float ms = 0.f;
+          if (h->ev_phase[i] != QMCW_PROF_FULL_NLPP) continue;
+          HIPCHK(h, hipEventElapsedTime(&ms, h->ev[i], h->ev[i + 1]));
+          if (ms > 0 && ms < tb) { tb = ms; best_waves = nw; }
+        }
+      }
+      h->nlpp_waves = best_waves;
+    } else {
+      h->nlpp_waves = -1;
     }
   }
   h->prof = prof_save;
@@ -2013,6 +2081,7 @@ extern "C" int qmcw_set_group_width(qmcw_handle *h, int32_t G) {
   HIPCHK(h, hipStreamSynchronize(h->stream));
   h->G = G;
   for (int k = 0; k < 4; k++) h->Gk[k] = G;
+  h->nlpp_waves = -1;
   return QMCW_OK;
 }
 

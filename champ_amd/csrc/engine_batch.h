@@ -5,7 +5,7 @@
 // counts share a launch; the kernels' lane-group widths and e-e-n order are
 // common to the batch.
 #pragma once
-#include "engine_kernels.h"
+#include "engine_nlpp.h"
 
 namespace qmcw {
 
@@ -62,6 +62,15 @@ void k_full_nlpp_batch(BatchArgs B) {
   const KArgs &A = B.A[s];
   if (A.S.nloc == 0) return;
   full_nlpp_b<T, G, ORD>(A, blockIdx.x - B.boff[s]);
+}
+
+// the systems whose pseudopotential runs one block of kNlppWaves wavefronts
+// per walker (KArgs::nlpp_tiles)
+template <typename T, int ORD>
+__global__ __launch_bounds__(64 * kNlppWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void k_full_nlpp_tiles_batch(BatchArgs B) {
+  const int s = batch_sys(B, blockIdx.x);
+  full_nlpp_tiles_b<T, ORD>(B.A[s], blockIdx.x - B.boff[s]);
 }
 
 #ifndef QMCW_ORD   // launched from the host translation unit only

@@ -1131,8 +1131,9 @@ __device__ __forceinline__ double ecp_radial(const DevSys &S, double r, int l0, 
   int b = cst(S.ecp_off)[ict * QMCW_MAX_LPOT + l0], e = cst(S.ecp_off)[ict * QMCW_MAX_LPOT + l0 + 1];
   for (int q = b; q < e; q++) {
     int pw = cst(S.ecp_power)[q];
-    double p = 1.0;
-    if (pw != 2) p = pow(r, (double)(pw - 2));
+    // r^(pw - 2): the terms of the pseudopotentials have small powers
+    double p = pw == 1 ? 1.0 / r : pw == 3 ? r : 1.0;
+    if (pw < 1 || pw > 3) p = pow(r, (double)(pw - 2));
     v += p * cst(S.ecp_coef)[q] * exp(-cst(S.ecp_expo)[q] * rsq);
   }
   return v;

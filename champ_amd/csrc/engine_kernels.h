@@ -33,6 +33,7 @@ struct KArgs {
   int lds_y_off;     // its offset (doubles) in the dynamic LDS, after the basis values
   int lds_nlpp;      // doubles per lane of k_full_nlpp's point scratch in LDS (0: global)
   int lds_dnlpp;     // doubles per lane of k_deriv_nlpp's point scratch in LDS (0: global)
+  int nlpp_tiles;    // wavefronts per walker of k_full_nlpp_tiles (0: k_full_nlpp)
   int bf16;          // orbital-contraction inputs rounded to bfloat16
   int chunk;         // electrons per basis chunk in the full evaluation
   int pnl_mfma;      // k_deriv_nlpp leaves psp_nonloc_orb's contraction to k_pnl_mfma
@@ -975,14 +976,24 @@ __global__ __launch_bounds__(64) void k_pnl_mfma(KArgs A, int nw) {
 // rotqua (qmc/vmc/rotqua.f90): a random rotation drawn from the stream st4,
 // as the axes (x1, x2, x3), (y1, y2, y3), (z1, z2, z3) that take the
 // reference grid q0 to q = q0x x + q0y y + q0z z.
-__device__ __forceinline__ void rot_axes(int *st4, double *ax) {
-  double x1, x2, x3, xsum;
+// The draws of a rotation and its axes apart: one lane walks a stream, any
+// lane can form the axes.
+__device__ __forceinline__ void rot_draws(int *st4, double *d) {
+  double x1, x2, u1, u2;
   do {
     x1 = 1.0 - 2.0 * rannyu(st4);
     x2 = 1.0 - 2.0 * rannyu(st4);
-    xsum = x1 * x1 + x2 * x2;
-  } while (xsum >= 1.0);
-  double xsum2 = 2.0 * sqrt(fabs(1.0 - xsum));
+  } while (x1 * x1 + x2 * x2 >= 1.0);
+  do {
+    u1 = rannyu(st4) * 2.0 - 1.0;
+    u2 = rannyu(st4) * 2.0 - 1.0;
+  } while (u1 * u1 + u2 * u2 >= 1.0);
+  d[0] = x1; d[1] = x2; d[2] = u1; d[3] = u2;
+}
+__device__ __forceinline__ void rot_from_draws(const double *d, double *ax) {
+  double x1 = d[0], x2 = d[1], u1 = d[2], u2 = d[3];
+  const double xsum = x1 * x1 + x2 * x2, usum = u1 * u1 + u2 * u2;
+  double xsum2 = 2.0 * sqrt(fabs(1.0 - xsum)), x3;
   x1 *= xsum2;
   x2 *= xsum2;
   x3 = 1.0 - 2.0 * xsum;
@@ -995,18 +1006,17 @@ __device__ __forceinline__ void rot_axes(int *st4, double *ax) {
   }
   double yy1 = x3 * cfi, yy2 = x3 * sfi, yy3 = -sthet;
   double zz1 = -sfi, zz2 = cfi, zz3 = 0;
-  double u1, u2, usum;
-  do {
-    u1 = rannyu(st4) * 2.0 - 1.0;
-    u2 = rannyu(st4) * 2.0 - 1.0;
-    usum = u1 * u1 + u2 * u2;
-  } while (usum >= 1.0);
   double uu = sqrt(usum);
   u1 /= uu;
   u2 /= uu;
   ax[0] = x1; ax[1] = x2; ax[2] = x3;
   ax[3] = yy1 * u1 + zz1 * u2; ax[4] = yy2 * u1 + zz2 * u2; ax[5] = yy3 * u1 + zz3 * u2;
   ax[6] = yy1 * u2 - zz1 * u1; ax[7] = yy2 * u2 - zz2 * u1; ax[8] = yy3 * u2 - zz3 * u1;
+}
+__device__ __forceinline__ void rot_axes(int *st4, double *ax) {
+  double d[4];
+  rot_draws(st4, d);
+  rot_from_draws(d, ax);
 }
 
 // Pseudopotential quadrature points of the in-range pairs plist[0..npair)

@@ -45,6 +45,7 @@ struct OrdKernels {
   void (*sweep_batch)(const BatchCtx &, double delta, double fbias);
   void (*full_jas_batch)(const BatchCtx &);
   void (*full_nlpp_batch)(const BatchCtx &);
+  void (*full_nlpp_tiles_batch)(const BatchCtx &);
 };
 
 extern const OrdKernels kOrdKernels2, kOrdKernels3, kOrdKernels4, kOrdKernels5, kOrdKernels6,

@@ -78,7 +78,18 @@ void deriv_nlpp_g(const LaunchCtx &c) {
   }
 
 void full_jas(const LaunchCtx &c) { QMCW_BY_G(full_jas_g, c); }
-void full_nlpp(const LaunchCtx &c) { QMCW_BY_G(full_nlpp_g, c); }
+void full_nlpp(const LaunchCtx &c) {
+  if (c.A.nlpp_tiles) {
+    const dim3 grid(c.Wl), block(kWave * c.A.nlpp_tiles);
+    const size_t lds = sizeof(double) * nlpp_tiles_lds(c.A.S.N * c.A.S.M);
+    if (c.precision == QMCW_FP64)
+      hipLaunchKernelGGL((k_full_nlpp_tiles<double, ORD>), grid, block, lds, c.stream, c.A);
+    else
+      hipLaunchKernelGGL((k_full_nlpp_tiles<float, ORD>), grid, block, lds, c.stream, c.A);
+    return;
+  }
+  QMCW_BY_G(full_nlpp_g, c);
+}
 void ratio(const LaunchCtx &c, int ie, int mode, const double *xn, double delta, double fbias,
            double *out, long long *nacc) {
   QMCW_BY_G(ratio_g, c, ie, mode, xn, delta, fbias, out, nacc);
@@ -159,6 +170,13 @@ void sweep_batch(const BatchCtx &c, double delta, double fbias) {
 }
 void full_jas_batch(const BatchCtx &c) { QMCW_BY_GB(full_jas_batch_g, c); }
 void full_nlpp_batch(const BatchCtx &c) { QMCW_BY_GB(full_nlpp_batch_g, c); }
+void full_nlpp_tiles_batch(const BatchCtx &c) {
+  const dim3 grid(c.nblocks), block(kWave * kNlppWaves);
+  if (c.precision == QMCW_FP64)
+    hipLaunchKernelGGL((k_full_nlpp_tiles_batch<double, ORD>), grid, block, c.smem, c.stream, c.B);
+  else
+    hipLaunchKernelGGL((k_full_nlpp_tiles_batch<float, ORD>), grid, block, c.smem, c.stream, c.B);
+}
 
 }  // namespace
 
@@ -166,7 +184,8 @@ void full_nlpp_batch(const BatchCtx &c) { QMCW_BY_GB(full_nlpp_batch_g, c); }
 extern const OrdKernels QMCW_CAT(kOrdKernels, QMCW_ORD) = {full_jas, full_nlpp, ratio, deriv_jas,
                                                             deriv_nlpp, move_a, tm_ratios,
                                                             ratio_batch, sweep_batch,
-                                                            full_jas_batch, full_nlpp_batch};
+                                                            full_jas_batch, full_nlpp_batch,
+                                                            full_nlpp_tiles_batch};
 #endif
 
 }  // namespace qmcw

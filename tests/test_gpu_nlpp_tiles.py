@@ -1,0 +1,79 @@
+"""The pseudopotential with its points' Jastrow on MFMA (k_full_nlpp_tiles)
+at the sizes where its tiles end: electrons about the 16-column tiles and the
+passes of three and four of them, centres about the steps of four, one to
+four wavefronts per walker, every order of the e-e-n polynomial, g and h
+shells.  FP64 against the oracle (bounds of the molecules' parity tests);
+mixed against the lane-group kernel of the same precision, whose FP32 sums
+run in another order (2^-24 per operation over the few thousand terms of a
+point's Jastrow, times |V_nl| of a few Ha, stays below 1e-4)."""
+import os
+import sys
+
+import numpy as np
+import pytest
+
+import oracle
+from champ_amd import system
+from champ_amd.engine import Engine
+
+sys.path.insert(0, os.path.dirname(__file__))
+pytestmark = pytest.mark.gpu
+
+
+def _mol(nelec, ncent, nordc=4, gh=False):
+    s = system.random_molecule(300 + nelec, nelec=nelec, ncent=ncent, zeff=6.0, gh_shells=gh)
+    if nordc != s.nordc:
+        g = np.random.default_rng(nordc)
+        s.nordc = nordc
+        s.c = system.cusp_exact(g.normal(0, 0.03, (3, system.nterms4(nordc))), nordc)
+    return s
+
+
+CASES = [(2, 1, 4, False), (15, 3, 4, False), (16, 4, 4, False), (17, 5, 4, True),
+         (33, 2, 4, False), (48, 3, 4, False), (49, 4, 4, False), (65, 6, 4, False),
+         (9, 3, 2, False), (9, 3, 3, False), (18, 3, 5, False), (9, 3, 6, False), (9, 3, 7, False)]
+
+
+@pytest.mark.parametrize("nelec,ncent,nordc,gh", CASES)
+@pytest.mark.parametrize("waves", [1, 2, 4])
+def test_tiles_match_oracle(monkeypatch, nelec, ncent, nordc, gh, waves):
+    monkeypatch.setenv("QMCW_NLPP_TILES", str(waves))
+    s = _mol(nelec, ncent, nordc, gh)
+    W = 5
+    x = system.random_walkers(s, W, seed=nelec)
+    x[0] += 2.0                        # a walker with few pairs in range or none
+    e = Engine(s, W)
+    e.set_walkers(x)
+    g = e.psi_at()
+    o9 = oracle.Oracle(s).eval_batch(x)["out9"]
+    assert np.max(np.abs(g["epot"] - o9[:, 4]) / (np.abs(o9[:, 4]) + 1e-8)) < 1e-9
+
+
+@pytest.mark.parametrize("nelec,ncent", [(8, 3), (33, 4), (65, 6)])
+def test_mixed_tiles_match_lane_groups(monkeypatch, nelec, ncent):
+    s = _mol(nelec, ncent)
+    x = system.random_walkers(s, 24, seed=5)
+    out = []
+    for tiles in ("0", "2"):
+        monkeypatch.setenv("QMCW_NLPP_TILES", tiles)
+        e = Engine(s, 24, "mixed")
+        e.set_walkers(x)
+        out.append(e.psi_at()["epot"])
+        e.close()
+    scale = np.abs(out[0]) + 1.0
+    assert np.median(np.abs(out[0] - out[1]) / scale) < 1e-5
+    assert np.max(np.abs(out[0] - out[1]) / scale) < 1e-3
+
+
+@pytest.mark.parametrize("tmoves", [0, 1])
+def test_dmc_generations_on_tiles(monkeypatch, tmoves):
+    from test_gpu_dmc import test_dmc_generations_match_oracle
+    monkeypatch.setenv("QMCW_NLPP_TILES", "2")
+    test_dmc_generations_match_oracle("c2_dimer", 0.3, tmoves)
+
+
+def test_batch_of_tiles_and_lane_groups(monkeypatch):
+    """One launch sequence over systems on either side of the rule."""
+    from test_gpu_batch import test_one_launch_batch_matches_oracle
+    monkeypatch.setenv("QMCW_NLPP_TILES", "4")
+    test_one_launch_batch_matches_oracle(monkeypatch, "0")
