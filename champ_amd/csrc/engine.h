@@ -20,6 +20,18 @@ constexpr int kMaxNs = 512;        // electrons of one spin
 // grid points in num_tab
 constexpr int kNumPar = 12;
 
+// A shell of a centre type and a centre, each one scalar load: the shells of
+// a type are the same at all of its centres up to the place of their basis
+// functions (bas: index from the centre's first function, -1 absent)
+struct TypeShell {
+  int l, a, num, p0, p1;     // angular momentum, power of r, table, primitives [p0, p1) of tprim
+  int bas[kMaxShellM];
+};
+struct TypeCent {
+  double x, y, z;
+  int bas0, ic;              // first basis function, centre
+};
+
 // Flattened system in device memory.  Pointers are device pointers.
 struct DevSys {
   int N, nup, ndn, M, nctype, NB, NO;
@@ -43,6 +55,13 @@ struct DevSys {
   const double *num_par;     // [nnum][kNumPar]
   const double *num_tab;     // [sum of nr][4] grid point x, R, R'' (spline), 0
   int maxshell_per_cent;
+  // the same shells by centre type (point_ratio): the type's shells
+  // tsh[tsh_off[t]..), its centres tcent[tc_off[t]..), and the primitives'
+  // (exponent, coefficient) pairs
+  const int *tsh_off, *tc_off;   // [nctype+1]
+  const TypeShell *tsh;
+  const TypeCent *tcent;
+  const double *tprim;
   const double *coefT;       // [NB][NO] (normalisation folded in)
   const double *coef_occ[2]; // [NB][nocc] coefT of the occupied orbitals of each spin
   // determinants (spin s = 0 up, 1 down)

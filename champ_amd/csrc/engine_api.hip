@@ -631,13 +631,13 @@ static void eval_args(const qmcw_handle *h, bool derivs, bool keep, EvalArgs &e)
   }
   det_lds_inv(h, A, det_smem);
   e.jas = A;
-  // k_full_nlpp's per-lane point scratch (4M distances, N values of U) in
+  // k_full_nlpp's per-lane point scratch (M distances, N values of U) in
   // LDS when all of the launch's blocks stay resident with it
   e.nlpp = A;
   {
     const int M = A.S.M, N = A.S.N;
     const size_t tsz = h->precision == QMCW_FP64 ? sizeof(double) : sizeof(float);
-    const int per_lane = 4 * M + (int)((N * tsz + 7) / 8);
+    const int per_lane = M + (int)((N * tsz + 7) / 8);
     const size_t blk = (size_t)kWave * per_lane * sizeof(double);
     const size_t bpc = ((size_t)h->Wl / (kWave / h->Gk[KC_NLPP]) + h->ncu - 1) / h->ncu;
     const size_t cap = std::min<size_t>(48 * 1024, (160 * 1024) / std::max<size_t>(1, bpc));
@@ -645,8 +645,8 @@ static void eval_args(const qmcw_handle *h, bool derivs, bool keep, EvalArgs &e)
       e.nlpp.lds_nlpp = per_lane;
       e.nlpp_smem = blk;
     }
-    // k_deriv_nlpp: the same plus N doubles per lane
-    const int per_lane_d = per_lane + N;
+    // k_deriv_nlpp: the vectors as well, and N doubles per lane
+    const int per_lane_d = per_lane + 3 * M + N;
     const size_t blk_d = (size_t)kWave * per_lane_d * sizeof(double);
     if (derivs && h->use_lds && blk_d <= cap) {
       e.nlpp.lds_dnlpp = per_lane_d;
@@ -920,6 +920,38 @@ extern "C" int qmcw_create(const qmcw_system *s, int32_t nwalk, int32_t precisio
   UP(sh_cent, S.sh_cent); UP(sh_l, S.sh_l); UP(sh_a, S.sh_a); UP(sh_nm, S.sh_nm);
   UP(sh_prim_off, S.sh_prim_off); UP(sh_m, S.sh_m); UP(sh_bas, S.sh_bas);
   UP(cent_sh_off, S.cent_sh_off); UP(pz, S.prim_zeta); UP(pc, S.prim_coef);
+  {
+    std::vector<int> tso{0}, tco{0}, cb0(s->ncent, 0);
+    std::vector<TypeShell> ts;
+    std::vector<TypeCent> tc;
+    std::vector<double> tp;
+    for (size_t p = 0; p < pz.size(); p++) { tp.push_back(pz[p]); tp.push_back(pc[p]); }
+    for (int ic = 1; ic < s->ncent; ic++) {
+      const int t = s->iwctype[ic - 1];
+      cb0[ic] = cb0[ic - 1] + s->ctype_bas_off[t + 1] - s->ctype_bas_off[t];
+    }
+    for (int t = 0; t < s->nctype; t++) {
+      int first = -1;
+      for (int ic = 0; ic < s->ncent; ic++) {
+        if (s->iwctype[ic] != t) continue;
+        if (first < 0) first = ic;
+        tc.push_back({s->cent[3 * ic], s->cent[3 * ic + 1], s->cent[3 * ic + 2], cb0[ic], ic});
+      }
+      for (int sh = first < 0 ? 0 : cent_sh_off[first]; first >= 0 && sh < cent_sh_off[first + 1]; sh++) {
+        TypeShell d;
+        d.l = sh_l[sh]; d.a = sh_a[sh]; d.num = sh_num[sh];
+        d.p0 = sh_prim_off[sh]; d.p1 = sh_prim_off[sh + 1];
+        for (int q = 0; q < kMaxShellM; q++) {
+          const int b = sh_bas[sh * kMaxShellM + q];
+          d.bas[q] = b < 0 ? -1 : b - cb0[first];
+        }
+        ts.push_back(d);
+      }
+      tso.push_back((int)ts.size());
+      tco.push_back((int)tc.size());
+    }
+    UP(tso, S.tsh_off); UP(tco, S.tc_off); UP(ts, S.tsh); UP(tc, S.tcent); UP(tp, S.tprim);
+  }
   S.has_num = 0;
   for (int v : sh_num) S.has_num |= (v >= 0);
   if (S.has_num) {

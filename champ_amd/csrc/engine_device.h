@@ -970,48 +970,89 @@ __device__ void eval_shell(const DevSys &S, int s, T x, T y, T z, T r, int want,
   }
 }
 
-// sum over the shell's components of gp[basis] * phi_basis at (x, y, z).
-// Shells are complete: slot q holds m = 0, 1, -1, 2, -2, ...; an absent
-// component has basis index -1.
+// sum over all basis functions of gp[b] phi_b at the position xn (value
+// only): the determinant ratio of a quadrature point.  The shells go by
+// centre type, the type's centres two at a time inside a shell, so that one
+// scalar load of a shell's description and of its primitives serves all of
+// the type's centres and the exponentials of two centres are independent.
+// Shell by shell over the centres, each with its own chain of dependent
+// scalar loads, the wavefront waited for those most of the time.
 template <typename T, int L, typename GP>
-__device__ __forceinline__ T shell_dot_l(T x, T y, T z, cptr<int> bas, const GP *gp) {
-  T Sv[2 * L + 1], Sg[2 * L + 1][3];
-  solid_harm<T>(L, x, y, z, Sv, Sg);
+__device__ __forceinline__ T type_shell_dot(const DevSys &S, const TypeShell &d, int c0, int c1,
+                                            const double *xn, const GP *gp) {
+  const cptr<TypeCent> tc = (cptr<TypeCent>)S.tcent;
+  const cptr<double> tp = cst(S.tprim);
+  const bool gauss = (S.basis_type == QMCW_BASIS_GAUSSIAN);
   T acc = 0;
+  for (int c = c0; c < c1; c += 2) {
+    const int cs[2] = {c, c + 1 < c1 ? c + 1 : c};
+    T x[2], y[2], z[2], arg[2], g[2] = {T(0), T(0)};
+    int b0[2];
 #pragma unroll
-  for (int q = 0; q < 2 * L + 1; q++) {
-    int b = bas[q];
-    if (b >= 0) acc += T(gp[b]) * Sv[q];   // gp already rounded in the BF16 engine
+    for (int u = 0; u < 2; u++) {
+      const double dx = xn[0] - tc[cs[u]].x, dy = xn[1] - tc[cs[u]].y, dz = xn[2] - tc[cs[u]].z;
+      b0[u] = tc[cs[u]].bas0;
+      x[u] = (T)dx; y[u] = (T)dy; z[u] = (T)dz;
+      arg[u] = (T)(dx * dx + dy * dy + dz * dz);
+    }
+    if (!gauss || d.num >= 0 || d.a > 0) {
+      // Slater and tabulated functions, and factors r^a, need the distance
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const T r2 = arg[u], r = sqrt(r2);
+        if (d.num >= 0) {
+          g[u] = num_radial_f<T>(S, d.num, L, r);
+        } else {
+          for (int p = d.p0; p < d.p1; p++)
+            g[u] += T(tp[2 * p + 1]) * exp(-T(tp[2 * p]) * (gauss ? r2 : r));
+          for (int q = 0; q < d.a; q++) g[u] *= r;
+        }
+      }
+    } else {
+      for (int p = d.p0; p < d.p1; p++) {
+        const T mz = -T(tp[2 * p]), cf = T(tp[2 * p + 1]);
+#pragma unroll
+        for (int u = 0; u < 2; u++) g[u] += cf * exp(mz * arg[u]);
+      }
+    }
+    if (c + 1 >= c1) g[1] = T(0);
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      T Sv[2 * L + 1], Sg[2 * L + 1][3], a = 0;
+      solid_harm<T>(L, x[u], y[u], z[u], Sv, Sg);
+#pragma unroll
+      for (int q = 0; q < 2 * L + 1; q++)
+        if (d.bas[q] >= 0) a += T(gp[b0[u] + d.bas[q]]) * Sv[q];
+      acc += a * g[u];
+    }
   }
   return acc;
 }
-template <typename T, typename GP = T>
-__device__ T shell_dot(const DevSys &S, int s, T x, T y, T z, T r, const GP *gp) {
-  int l = cst(S.sh_l)[s], a = cst(S.sh_a)[s];
-  const bool gauss = (S.basis_type == QMCW_BASIS_GAUSSIAN);
-  T g = 0;
-  const int kn = S.has_num ? cst(S.sh_num)[s] : -1;
-  if (kn >= 0) {
-    g = num_radial_f<T>(S, kn, l, r);
-  } else {
-    const cptr<double> pz = cst(S.prim_zeta), pc = cst(S.prim_coef);
-    for (int p = cst(S.sh_prim_off)[s]; p < cst(S.sh_prim_off)[s + 1]; p++) {
-      T zeta = T(pz[p]), d = T(pc[p]);
-      g += d * exp(gauss ? -zeta * r * r : -zeta * r);
+template <typename T, typename GP>
+__device__ __forceinline__ double point_ratio(const DevSys &S, const double *xn, const GP *gp) {
+  double rd = 0.0;
+  for (int t = 0; t < S.nctype; t++) {
+    const int c0 = cst(S.tc_off)[t], c1 = cst(S.tc_off)[t + 1];
+    if (c0 == c1) continue;
+    for (int sh = cst(S.tsh_off)[t]; sh < cst(S.tsh_off)[t + 1]; sh++) {
+      const cptr<int> w = cst((const int *)(S.tsh + sh));
+      TypeShell d;
+      d.l = w[0]; d.a = w[1]; d.num = w[2]; d.p0 = w[3]; d.p1 = w[4];
+#pragma unroll
+      for (int q = 0; q < kMaxShellM; q++) d.bas[q] = w[5 + q];
+      T v;
+      switch (d.l) {
+        case 0: v = type_shell_dot<T, 0, GP>(S, d, c0, c1, xn, gp); break;
+        case 1: v = type_shell_dot<T, 1, GP>(S, d, c0, c1, xn, gp); break;
+        case 2: v = type_shell_dot<T, 2, GP>(S, d, c0, c1, xn, gp); break;
+        case 3: v = type_shell_dot<T, 3, GP>(S, d, c0, c1, xn, gp); break;
+        case 4: v = type_shell_dot<T, 4, GP>(S, d, c0, c1, xn, gp); break;
+        default: v = type_shell_dot<T, 5, GP>(S, d, c0, c1, xn, gp); break;
+      }
+      rd += (double)v;
     }
-    for (int q = 0; q < a; q++) g *= r;
   }
-  const cptr<int> bas = cst(S.sh_bas) + s * kMaxShellM;
-  T acc;
-  switch (l) {
-    case 0: acc = shell_dot_l<T, 0, GP>(x, y, z, bas, gp); break;
-    case 1: acc = shell_dot_l<T, 1, GP>(x, y, z, bas, gp); break;
-    case 2: acc = shell_dot_l<T, 2, GP>(x, y, z, bas, gp); break;
-    case 3: acc = shell_dot_l<T, 3, GP>(x, y, z, bas, gp); break;
-    case 4: acc = shell_dot_l<T, 4, GP>(x, y, z, bas, gp); break;
-    default: acc = shell_dot_l<T, 5, GP>(x, y, z, bas, gp); break;
-  }
-  return acc * g;
+  return rd;
 }
 
 // Values of shell s's basis functions at (x, y, z), r, accumulated in FP64:

@@ -1020,7 +1020,7 @@ __device__ __forceinline__ void rot_axes(int *st4, double *ax) {
 }
 
 // Pseudopotential quadrature points of the in-range pairs plist[0..npair)
-// taken by this lane: sum of w exp(dJ) v P_l (Psi_D ratio).  rnew: 4M
+// taken by this lane: sum of w exp(dJ) v P_l (Psi_D ratio).  rnew: M
 // doubles and uq: N values of per-lane scratch (LDS or global), stored
 // lane-interleaved.
 template <typename T, int G, int ORD, bool PAIR>
@@ -1037,7 +1037,6 @@ __device__ __forceinline__ double nlpp_points(const KArgs &A, const double *ws, 
   const double *gp = ss + SL.gproj;
   const double *quad = ws + L.quad;
   const int nq = S.nquad;
-  const LaneArr<double> rvnew = rnew + M;
   double vpsp = 0.0;
   const double *prot = ss + SL.prot;
   for (int t = lane; t < npair * nq; t += G) {
@@ -1063,17 +1062,10 @@ __device__ __forceinline__ double nlpp_points(const KArgs &A, const double *ws, 
     for (int jc = 0; jc < M; jc++) {
       const double dx = xn[0] - cst(S.cent)[3 * jc], dy = xn[1] - cst(S.cent)[3 * jc + 1],
                    dz = xn[2] - cst(S.cent)[3 * jc + 2];
-      rvnew[3 * jc] = dx; rvnew[3 * jc + 1] = dy; rvnew[3 * jc + 2] = dz;
       rnew[jc] = (jc == ic) ? rei : sqrt(dx * dx + dy * dy + dz * dz);
     }
     // determinant ratio of moving electron i to the point
-    double rd = 0.0;
-    const double *gpi = gp + (int64_t)i * S.NB;
-    for (int sh = 0; sh < S.nshell; sh++) {
-      const int jc = cst(S.sh_cent)[sh];
-      rd += (double)shell_dot<T, double>(S, sh, (T)rvnew[3 * jc], (T)rvnew[3 * jc + 1],
-                                         (T)rvnew[3 * jc + 2], (T)rnew[jc], gpi);
-    }
+    const double rd = point_ratio<T, double>(S, xn, gp + (int64_t)i * S.NB);
     // Jastrow value change against the electron's current pair sum: kept
     // per electron for small N; summed here for large N, where the sum's
     // loads overlap the point's other work (measured faster on the chain)
@@ -1196,10 +1188,10 @@ __device__ __forceinline__ void full_nlpp_b(const KArgs &A, int bid_) {
     if (A.dmc_rot && !mover) {
       vpsp = 0.0;
     } else if (A.lds_nlpp) {
-      // the block's 64 lanes interleaved: 4M doubles, then N values
+      // the block's 64 lanes interleaved: M doubles, then N values
       extern __shared__ double dyn_lds[];
       const LaneArr<double> rq{dyn_lds + threadIdx.x, kWave};
-      const LaneArr<T> uq{reinterpret_cast<T *>(dyn_lds + 4 * M * kWave) + threadIdx.x, kWave};
+      const LaneArr<T> uq{reinterpret_cast<T *>(dyn_lds + M * kWave) + threadIdx.x, kWave};
       vpsp = nlpp_points<T, G, ORD, PAIR>(A, ws, ss, npair, plist, rq, uq, tqw, lane);
     } else {
       // the walker's G lanes interleaved in its scratch
@@ -1256,7 +1248,7 @@ void k_tm_ratios(KArgs A, int ie, int cw, const double *pts, const int *cnt, dou
   // read before the next full evaluation rebuilds them all)
   group_gproj<G>(S, ss + SL.gproj, ss + SL.g[0], ss + SL.g[1], A.bf16, lane, ie);
   __syncthreads();
-  const LaneArr<double> rnew{ss + SL.qd + lane, G}, rvnew = rnew + M;
+  const LaneArr<double> rnew{ss + SL.qd + lane, G};
   const LaneArr<T> uq{reinterpret_cast<T *>(ss + SL.uq) + lane, G};
   const double *gpi = ss + SL.gproj + (int64_t)ie * S.NB;
   double fold = fso[ie * N + ie];
@@ -1267,15 +1259,9 @@ void k_tm_ratios(KArgs A, int ie, int cw, const double *pts, const int *cnt, dou
     for (int jc = 0; jc < M; jc++) {
       const double dx = xn[0] - cst(S.cent)[3 * jc], dy = xn[1] - cst(S.cent)[3 * jc + 1],
                    dz = xn[2] - cst(S.cent)[3 * jc + 2];
-      rvnew[3 * jc] = dx; rvnew[3 * jc + 1] = dy; rvnew[3 * jc + 2] = dz;
       rnew[jc] = sqrt(dx * dx + dy * dy + dz * dz);
     }
-    double rd = 0.0;
-    for (int sh = 0; sh < S.nshell; sh++) {
-      const int jc = cst(S.sh_cent)[sh];
-      rd += (double)shell_dot<T, double>(S, sh, (T)rvnew[3 * jc], (T)rvnew[3 * jc + 1],
-                                         (T)rvnew[3 * jc + 2], (T)rnew[jc], gpi);
-    }
+    const double rd = point_ratio<T, double>(S, xn, gpi);
     const double delta = (double)jas_point_val<T, ORD>(S, ie, xn, x, rnew, bt, uq) - fold;
     out[8 * ((int64_t)c * cw + w)] = rd * exp(delta);
   }

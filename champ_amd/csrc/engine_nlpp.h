@@ -352,15 +352,7 @@ __device__ __forceinline__ void full_nlpp_tiles_b(const KArgs &A, int w) {
     tl.el[lane] = i;
     tl.ic[lane] = ic;
     // determinant ratio of moving electron i to the point
-    double rd = 0.0;
-    const double *gpi = gp + (int64_t)i * S.NB;
-    for (int jc = 0; jc < M; jc++) {
-      const double dx = xn[0] - cst(S.cent)[3 * jc], dy = xn[1] - cst(S.cent)[3 * jc + 1],
-                   dz = xn[2] - cst(S.cent)[3 * jc + 2];
-      const double rc = (jc == ic) ? rei : sqrt(dx * dx + dy * dy + dz * dz);
-      for (int sh = cst(S.cent_sh_off)[jc]; sh < cst(S.cent_sh_off)[jc + 1]; sh++)
-        rd += (double)shell_dot<T, double>(S, sh, (T)dx, (T)dy, (T)dz, (T)rc, gpi);
-    }
+    const double rd = point_ratio<T, double>(S, xn, gp + (int64_t)i * S.NB);
     wave_lds_fence();
     const int nsub = (min(64, npt - t0) + 15) / 16;
     for (int sub = 0; sub < nsub; sub++) nlpp_tile<T, ORD>(S, tl, 16 * sub, s_c, x, bt, lane);
