@@ -736,15 +736,19 @@ static void launch_move_bc(qmcw_handle *h, const KArgs &A, size_t smem_b, size_t
 // The one-electron move's arguments at lane-group width G: LDS for the
 // moved electron's basis values (phi_b bytes) and, after them, eval_y's
 // inputs (smem: the whole dynamic LDS of the single-kernel move)
-static KArgs move_args(const qmcw_handle *h, int G, bool split, size_t &phi_b, size_t &smem) {
+static KArgs move_args(const qmcw_handle *h, int G, bool split, size_t &phi_b, size_t &smem,
+                       bool batch = false) {
   KArgs A = h->A;
   // the moved electron's basis values in LDS when they fit (<= 48 KB per
   // block); in the single-kernel move the same region first holds the
   // e-e-n tables of the Jastrow row (one per centre)
   const size_t tsz = h->precision == QMCW_FP64 ? sizeof(double) : sizeof(float);
   const int ordk = std::max(2, A.S.nordc);
+  // (een_sum_stride or een_tab_stride values each; a batch's kernel may take
+  // either, for which the larger holds)
+  const bool sums = !batch && (h->precision == QMCW_FP64 ? een_sums<double>(G, A.S.M) : een_sums<float>(G, A.S.M));
   const int tab = (A.S.nordc > 1 && !split && !h->no_een_tab)
-                      ? A.S.M * (3 * ((ordk + 1) * (ordk + 2) / 2) + 8) : 0;
+                      ? A.S.M * (3 * ((ordk + 1) * (ordk + 2) / 2) + (sums ? 4 : 8)) : 0;
   const int wst = std::max(A.S.NB * 5, tab);
   const size_t lds = (size_t)(kWave / G) * wst * tsz;
   A.lds_phi = (h->use_lds && lds <= 48 * 1024) ? 1 : 0;
@@ -1756,7 +1760,7 @@ static int batch_upload(qmcw_batch *b, int set, bool first) {
   for (int s = 0; s < n; s++) {
     qmcw_handle *h = b->hs[s];
     size_t phi_b = 0, sm = 0;
-    A[(size_t)KB_MOVE * n + s] = move_args(h, h->Gk[KC_MOVE], false, phi_b, sm);
+    A[(size_t)KB_MOVE * n + s] = move_args(h, h->Gk[KC_MOVE], false, phi_b, sm, true);
     b->smem_move = std::max(b->smem_move, sm);
     EvalArgs e;
     const bool keep = first ? (h->orb_valid != 0) : true;
@@ -2064,7 +2068,11 @@ extern "C" int qmcw_autotune(qmcw_handle *h, int32_t *chosen) {
   }
   if (h->nlpp_tiles_env < 0) {
     h->nlpp_waves = 1;
-    if (nlpp_tile_waves(h) > 0) {        // a pseudopotential the tiles can take
+    // a pseudopotential the tiles can take, unless its lane groups already
+    // put two wavefronts on every SIMD (there the tiles never won below
+    // kNlppTilePairs)
+    const int64_t groups = (int64_t)h->Wl / (kWave / bestG[KC_NLPP]);
+    if (nlpp_tile_waves(h) > 0 && (tiles_only || groups < 8 * (int64_t)h->ncu)) {
       int best_waves = tiles_only ? -1 : 0;
       double tb = tiles_only ? 1e30 : best[KC_NLPP];
       for (int nw = 1; nw <= kNlppWaves; nw *= 2) {
@@ -2085,7 +2093,7 @@ extern "C" int qmcw_autotune(qmcw_handle *h, int32_t *chosen) {
       }
       h->nlpp_waves = best_waves;
     } else {
-      h->nlpp_waves = -1;
+      h->nlpp_waves = nlpp_tile_waves(h) > 0 ? 0 : -1;
     }
   }
   h->prof = prof_save;

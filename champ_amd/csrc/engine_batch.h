@@ -31,7 +31,7 @@ __global__ QMCW_HEAVY void k_ratio_1e_batch(BatchArgs B, int ie, double delta, d
   const int s = batch_sys(B, blockIdx.x);
   const KArgs &A = B.A[s];
   if (ie >= A.S.N) return;
-  ratio_1e_b<T, G, ORD>(A, blockIdx.x - B.boff[s], ie, 2, nullptr, delta, fbias, nullptr, B.nacc[s]);
+  ratio_1e_b<T, G, ORD, een_sums<T>(G, kSumCentres)>(A, blockIdx.x - B.boff[s], ie, 2, nullptr, delta, fbias, nullptr, B.nacc[s]);
 }
 
 // The whole sweep of each system in one launch: a block moves its
@@ -44,7 +44,7 @@ __global__ QMCW_HEAVY void k_sweep_1e_batch(BatchArgs B, double delta, double fb
   const KArgs &A = B.A[s];
   const int N = A.S.N;
   for (int ie = 0; ie < N; ie++) {
-    ratio_1e_b<T, G, ORD>(A, blockIdx.x - B.boff[s], ie, 2, nullptr, delta, fbias, nullptr, B.nacc[s]);
+    ratio_1e_b<T, G, ORD, een_sums<T>(G, kSumCentres)>(A, blockIdx.x - B.boff[s], ie, 2, nullptr, delta, fbias, nullptr, B.nacc[s]);
     __syncthreads();
   }
 }

@@ -555,6 +555,187 @@ __device__ void jas_pair_tab(const DevSys &S, bool parallel_spin, T rij, const T
   out.lj = m_hi ? lo : lm;
 }
 
+// The tables of jas_pair_sum, T values per centre: the moved electron's
+// polynomial in (U, B) (een_gamma's layout), the one of its gradient along
+// the vector to the centre (dA/dr / r times the A derivative), the one of its
+// laplacian (second derivative and 2/r times the first), then the vector
+template <int ORD>
+__host__ __device__ constexpr int een_sum_stride() { return 3 * (een_gi<ORD>(ORD, 0) + 1) + 4; }
+
+// The moved electron's tables at its new position (distances rn and vectors
+// rvn to the centres), one centre per lane
+template <typename T, int ORD, int G>
+__device__ __forceinline__ void een_sum_tables(const DevSys &S, const double *rn, const double *rvn, T *tab,
+                                           int lane) {
+  constexpr int NG = een_gi<ORD>(ORD, 0) + 1, TS = een_sum_stride<ORD>();
+  const T k = T(S.scalek);
+  for (int ic = lane; ic < S.M; ic += G) {
+    T A, Ad1, Ad2;
+    const T r = (T)rn[ic];
+    scaled<T>(S.isc, k, r, A, Ad1, Ad2);
+    A = T(1) - k * A;
+    Ad1 = -k * Ad1;
+    Ad2 = -k * Ad2;
+    T *tb = tab + ic * TS;
+    T g[3 * NG];
+    een_gamma3<T, ORD>(A, cst(S.c) + cst(S.iwctype)[ic] * S.nterms, g);
+    const T d = Ad1 / r, l1 = Ad2 + T(2) * d, l2 = Ad1 * Ad1;
+#pragma unroll
+    for (int q = 0; q < NG; q++) {
+      tb[q] = g[q];
+      tb[NG + q] = g[NG + q] * d;
+      tb[2 * NG + q] = g[2 * NG + q] * l2 + g[NG + q] * l1;
+    }
+#pragma unroll
+    for (int q = 0; q < 3; q++) tb[3 * NG + q] = (T)rvn[3 * ic + q];
+  }
+}
+
+// jas_pair_tab for many centres.  The sum over centres of a polynomial in U is
+// a polynomial in U of sums over centres, so the centre loop only adds up, for each power of U, the value,
+// both electrons' gradient vectors and their laplacian parts; U's derivatives
+// and the cross terms (twice grad U . grad A, a product with the gradient
+// vectors) are formed once per pair.  Per (pair, centre) that is about 190
+// operations, against about 250 with the chain rule inside the loop, and the
+// tables are smaller, so that two blocks share a SIMD in FP64 too: a DMC
+// generation of the 98-electron chain (4,096 walkers, FP64) went from 178.8
+// to 161.9 ms.  With two centres the sums only cost registers (the C2-like
+// system's move 115 -> 128 us in FP64).
+template <typename T, int ORD, typename PO>
+__device__ void jas_pair_sum(const DevSys &S, bool parallel_spin, T rij, const T *rvmo, const T *tab,
+                             const PO &po, bool m_hi, PairOut<T> &out) {
+  constexpr int NG = een_gi<ORD>(ORD, 0) + 1, TS = een_sum_stride<ORD>();
+  const T k = T(S.scalek);
+  T sspinn = T(1);
+  int isb = 0;
+  double asymp_b = S.asymp_jasb0;
+  if (parallel_spin) {
+    if (S.nspin2b == 2) isb = 1;
+    else if (S.nocuspb == 0) sspinn = T(0.5);
+    asymp_b = S.asymp_jasb1;
+  }
+  const double *b = S.b + isb * (S.nordb + 1);
+  T u, d1, d2;
+  scaled<T>(S.isc, k, rij, u, d1, d2);
+  T bot = T(1) + T(b[1]) * u;
+  T f = sspinn * T(b[0]) * u / bot;
+  T fu = sspinn * T(b[0]) / (bot * bot);
+  T fuu = T(-2) * fu * T(b[1]) / bot;
+  f -= T(asymp_b);
+  T up = u, upm = T(1);
+  for (int iord = 2; iord <= S.nordb; iord++) {
+    T bb = T(b[iord]);
+    fuu += bb * T(iord * (iord - 1)) * upm;
+    fu += bb * T(iord) * up;
+    upm = up;
+    up *= u;
+    f += bb * up;
+  }
+  const T irij = T(1) / rij;
+  fuu = fuu * d1 * d1 + fu * d2;
+  fu = fu * d1 * irij;
+  T gm[3], go[3];
+#pragma unroll
+  for (int q = 0; q < 3; q++) { gm[q] = fu * rvmo[q]; go[q] = -fu * rvmo[q]; }
+  T lm = fuu + T(2) * fu, lo = lm;
+  if (S.nordc > 1) {
+    // sums over the centres, per power of U: value w, the gradient vectors of
+    // m and o (without U's part) and their laplacians (likewise)
+    T w[ORD + 1], gmk[ORD][3], gok[ORD][3], lmk[ORD], lok[ORD];
+#pragma unroll
+    for (int kk = 0; kk <= ORD; kk++) w[kk] = T(0);
+#pragma unroll
+    for (int kk = 0; kk < ORD; kk++) {
+      lmk[kk] = lok[kk] = T(0);
+#pragma unroll
+      for (int q = 0; q < 3; q++) gmk[kk][q] = gok[kk][q] = T(0);
+    }
+    for (int ic = 0; ic < S.M; ic++) {
+      const T *tb = tab + ic * TS;
+      double rod, rvo[3];
+      po.get(S, ic, rod, rvo);
+      const T ro = (T)rod;
+      T B, Bd1, Bd2;
+      scaled<T>(S.isc, k, ro, B, Bd1, Bd2);
+      B = T(1) - k * B; Bd1 = -k * Bd1; Bd2 = -k * Bd2;
+      const T db = Bd1 / ro, l1 = Bd2 + T(2) * db, l2 = Bd1 * Bd1;
+      const T vm[3] = {tb[3 * NG], tb[3 * NG + 1], tb[3 * NG + 2]};
+      const T vo[3] = {db * (T)rvo[0], db * (T)rvo[1], db * (T)rvo[2]};
+      w[ORD] += tb[een_gi<ORD>(ORD, 0)];
+#pragma unroll
+      for (int kk = 0; kk < ORD; kk++) {
+        // the polynomials in B of this power of U, with the first two B
+        // derivatives of the value
+        T r = 0, rb = 0, rbb = 0, ra = 0, rl = 0;
+#pragma unroll
+        for (int n = ORD - kk; n >= 0; n--) {
+          rbb = rbb * B + T(2) * rb;
+          rb = rb * B + r;
+          r = r * B + tb[een_gi<ORD>(kk, n)];
+          ra = ra * B + tb[NG + een_gi<ORD>(kk, n)];
+          rl = rl * B + tb[2 * NG + een_gi<ORD>(kk, n)];
+        }
+        w[kk] += r;
+        lmk[kk] += rl;
+        lok[kk] += rbb * l2 + rb * l1;
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+          gmk[kk][q] += ra * vm[q];
+          gok[kk][q] += rb * vo[q];
+        }
+      }
+    }
+    T U, Ud1, Ud2;
+    scaled<T>(S.isc, k, rij, U, Ud1, Ud2);
+    U = T(1) - k * U;
+    Ud1 = -k * Ud1;
+    Ud2 = -k * Ud2;
+    // the polynomials in U and their derivatives (Horner)
+    T F = w[ORD], FU = T(0), FUU = T(0);
+#pragma unroll
+    for (int kk = ORD - 1; kk >= 0; kk--) {
+      FUU = FUU * U + T(2) * FU;
+      FU = FU * U + F;
+      F = F * U + w[kk];
+    }
+    const T gU = FU * Ud1 * irij;
+    T lu = T(2) * gU + FUU * Ud1 * Ud1 + FU * Ud2, cm = T(0), co = T(0);
+    f += F;
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      T a = T(0), au = T(0), c = T(0), cu = T(0);
+#pragma unroll
+      for (int kk = ORD - 1; kk >= 0; kk--) {
+        au = au * U + a;
+        a = a * U + gmk[kk][q];
+        cu = cu * U + c;
+        c = c * U + gok[kk][q];
+      }
+      gm[q] += a + gU * rvmo[q];
+      go[q] += c - gU * rvmo[q];
+      cm += au * rvmo[q];
+      co += cu * rvmo[q];
+    }
+    T am = T(0), ao = T(0);
+#pragma unroll
+    for (int kk = ORD - 1; kk >= 0; kk--) {
+      am = am * U + lmk[kk];
+      ao = ao * U + lok[kk];
+    }
+    const T x2 = T(2) * Ud1 * irij;
+    lm += lu + am + x2 * cm;
+    lo += lu + ao - x2 * co;
+  }
+  out.f = f;
+#pragma unroll
+  for (int q = 0; q < 3; q++) {
+    out.gi[q] = m_hi ? gm[q] : go[q];
+    out.gj[q] = m_hi ? go[q] : gm[q];
+  }
+  out.li = m_hi ? lm : lo;
+  out.lj = m_hi ? lo : lm;
+}
+
 // e-e Pade + polynomial of a pair at scaled distance u
 template <typename T>
 __device__ __forceinline__ T jas_b_val(const DevSys &S, bool parallel_spin, T u) {

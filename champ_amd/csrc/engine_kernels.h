@@ -24,7 +24,7 @@ struct KArgs {
   int lds_phi;       // k_ratio_1e keeps the moved electron's basis values in LDS
   int lds_wst;       // T values per walker of that LDS region (at least NB * 5)
   int een_tab;       // k_ratio_1e: the moved electron's e-e-n tables in the same region
-                     // during the Jastrow row (een_tables, jas_pair_tab)
+                     // during the Jastrow row (een_tables or een_sum_tables)
   int lds_det;       // k_full_det keeps a chunk's basis values in LDS
   int keep_state;    // the full evaluation takes the rows the committed moves kept in the state
                      // (distances, Jastrow pairs and, without full_orb, the orbitals)
@@ -1437,7 +1437,21 @@ __device__ __forceinline__ void orbitals_1e(const KArgs &A, int s, int nocc, con
 // walker's rannyu stream) or take xnew (mode 0), then distancese +
 // jastrow4e + orbitals + dete_update + eval_grad into the pending buffers.
 // out[w][8]: ratio, ln|psid_new|, sign, psij_new, grad(3), lap
-template <typename T, int G, int ORD>
+// Whether the move of a system of M centres at lane-group width G takes
+// jas_pair_sum: always in FP32, where it costs nothing with few centres; in
+// FP64 from this many centres on, at the widths such systems run at.  Closing
+// the sums costs about 400 operations a pair, what seven centres save at some
+// 60 each: with two centres the move slowed from 115 to 128 us (registers),
+// with the chain's it quickened from 1,010 to 874.
+constexpr int kSumCentres = 8;
+template <typename T>
+__host__ __device__ constexpr bool een_sums(int G, int M) {
+  return sizeof(T) == 4 || (G >= 32 && M >= kSumCentres);
+}
+
+// SUMS: the e-e-n tables of jas_pair_sum (many centres) instead of
+// jas_pair_tab's
+template <typename T, int G, int ORD, bool SUMS>
 __device__ __forceinline__ void ratio_1e_b(const KArgs &A, int bid_, int ie, int mode,
                                            const double *xnew_in, double delta, double fbias,
                                            double *out, long long *nacc) {
@@ -1507,7 +1521,10 @@ __device__ __forceinline__ void ratio_1e_b(const KArgs &A, int bid_, int ie, int
   extern __shared__ double dyn_lds[];
   T *etab = reinterpret_cast<T *>(dyn_lds) + (int64_t)grp * A.lds_wst;
   if (A.een_tab) {
-    een_tables<T, ORD, G>(S, ren, rven, etab, lane);
+    if (SUMS)
+      een_sum_tables<T, ORD, G>(S, ren, rven, etab, lane);
+    else
+      een_tables<T, ORD, G>(S, ren, rven, etab, lane);
     __syncthreads();
   }
   for (int j = lane; j < N; j += G) {
@@ -1537,7 +1554,10 @@ __device__ __forceinline__ void ratio_1e_b(const KArgs &A, int bid_, int ie, int
     if (A.een_tab) {
       const T rvmo[3] = {hi == ie ? rvij[0] : -rvij[0], hi == ie ? rvij[1] : -rvij[1],
                          hi == ie ? rvij[2] : -rvij[2]};
-      jas_pair_tab<T, ORD>(S, par, (T)ree[j], rvmo, etab, pJ, hi == ie, po);
+      if (SUMS)
+        jas_pair_sum<T, ORD>(S, par, (T)ree[j], rvmo, etab, pJ, hi == ie, po);
+      else
+        jas_pair_tab<T, ORD>(S, par, (T)ree[j], rvmo, etab, pJ, hi == ie, po);
     } else if (hi == ie) {
       jas_pair_g<T, ORD>(S, par, (T)ree[j], rvij, pI, pJ, po);
     } else {
@@ -1671,10 +1691,10 @@ __device__ __forceinline__ void ratio_1e_b(const KArgs &A, int bid_, int ie, int
     if (s_acc[grp]) group_commit<G>(A, ws, mv, ie, lane);
   }
 }
-template <typename T, int G, int ORD>
+template <typename T, int G, int ORD, bool SUMS>
 __global__ QMCW_HEAVY void k_ratio_1e(KArgs A, int ie, int mode, const double *xnew_in,
                                       double delta, double fbias, double *out, long long *nacc) {
-  ratio_1e_b<T, G, ORD>(A, blockIdx.x, ie, mode, xnew_in, delta, fbias, out, nacc);
+  ratio_1e_b<T, G, ORD, SUMS>(A, blockIdx.x, ie, mode, xnew_in, delta, fbias, out, nacc);
 }
 
 // ---------------------------------------------------------------------------

@@ -48,11 +48,14 @@ template <int G>
 void ratio_g(const LaunchCtx &c, int ie, int mode, const double *xn, double delta, double fbias,
              double *out, long long *nacc) {
   const dim3 grid(c.Wl / (kWave / G)), block(kWave);
-  if (c.precision == QMCW_FP64)
-    hipLaunchKernelGGL((k_ratio_1e<double, G, ORD>), grid, block, c.smem_ratio, c.stream, c.A, ie,
+  if (c.precision != QMCW_FP64)
+    hipLaunchKernelGGL((k_ratio_1e<float, G, ORD, true>), grid, block, c.smem_ratio, c.stream, c.A, ie,
                        mode, xn, delta, fbias, out, nacc);
+  else if (een_sums<double>(G, c.A.S.M))
+    hipLaunchKernelGGL((k_ratio_1e<double, G, ORD, (G >= 32)>), grid, block, c.smem_ratio, c.stream, c.A,
+                       ie, mode, xn, delta, fbias, out, nacc);
   else
-    hipLaunchKernelGGL((k_ratio_1e<float, G, ORD>), grid, block, c.smem_ratio, c.stream, c.A, ie,
+    hipLaunchKernelGGL((k_ratio_1e<double, G, ORD, false>), grid, block, c.smem_ratio, c.stream, c.A, ie,
                        mode, xn, delta, fbias, out, nacc);
 }
 template <int G>
