@@ -163,13 +163,12 @@ struct SLayout {
 // Derivative scratch (offsets in doubles from the walker's scratch base),
 // present when the system has parameters to optimise.
 struct DLayout {
-  int64_t raw;               // [nslot][N][5] slot pieces: value, grad, lap
-  int64_t gvalue, gjas, d2g; // [npj], [npj][N][3], [npj]
-  int64_t pbc;               // [N*M][NB] per (electron, centre) weighted basis sums
-  int64_t dpe_raw;           // [N*M][nslot]
-  int64_t dpe_slot, dpe;     // [nslot], [npj]
+  int64_t dj;                // [nslot][2] Jastrow slots: value, -hb (laplacian + 2 v . gradient)
+  int64_t pw;                // [N*M*nquad][2] quadrature points: factor, factor times ratio
+  int64_t pbc;               // [N][NB] weighted basis sums of each electron's points
+  int64_t dpe_slot;          // [nslot] the pseudopotential's slots
   int64_t pnl;               // [N][NO] psp_nonloc_orb
-  int64_t btd, uqd;          // [N][M] e-e-n variable B(r_j,ic), [64][N] per-lane U of a point
+  int64_t tb, tu, uqd;       // [M][N] e-e-n variable B(r_j,ic), [4][N][N] pair tables, [64][N] U of a point
   int64_t B;                 // [N][NO] orbital-resolved local energy
   int64_t tfull[2], dt[2];   // [ns][NO]
   int64_t aib;               // [ns][NO]

@@ -543,7 +543,7 @@ static void launch_fin(qmcw_handle *h, const KArgs &A) {
 template <int G>
 static void launch_derivs_asm(qmcw_handle *h, const KArgs &A) {
   const dim3 grid(h->Wl / (kWave / G)), block(kWave);
-  hipLaunchKernelGGL((k_derivs<G>), grid, block, 0, h->stream, A, h->der);
+  hipLaunchKernelGGL((k_derivs<G, false>), grid, block, 0, h->stream, A, h->der);
 }
 
 #define DISPATCH_GW(gw, fn, ...)                  \
@@ -645,12 +645,14 @@ static void eval_args(const qmcw_handle *h, bool derivs, bool keep, EvalArgs &e)
       e.nlpp.lds_nlpp = per_lane;
       e.nlpp_smem = blk;
     }
-    // k_deriv_nlpp: the vectors as well, and N doubles per lane
-    const int per_lane_d = per_lane + 3 * M + N;
-    const size_t blk_d = (size_t)kWave * per_lane_d * sizeof(double);
-    if (derivs && h->use_lds && blk_d <= cap) {
-      e.nlpp.lds_dnlpp = per_lane_d;
-      e.dnlpp_smem = blk_d;
+    // k_deriv_nlpp: its tile of basis values, and N values of U per lane
+    // after it while the block stays small
+    e.dnlpp_smem = h->precision == QMCW_FP64 ? deriv_tile_bytes<double>() : deriv_tile_bytes<float>();
+    const size_t blk_d = (size_t)kWave * N * sizeof(double);
+    e.nlpp.lds_dnlpp = 0;
+    if (derivs && h->use_lds && e.dnlpp_smem + blk_d <= 48 * 1024) {
+      e.nlpp.lds_dnlpp = N;
+      e.dnlpp_smem += blk_d;
     }
     e.nlpp.nlpp_tiles = nlpp_tile_waves(h);
     // psp_nonloc_orb's contraction on FP64 MFMA after k_deriv_nlpp
@@ -663,6 +665,13 @@ static void eval_args(const qmcw_handle *h, bool derivs, bool keep, EvalArgs &e)
   A.orb_mfma = (derivs && A.S.nparm > 0 && !h->no_gproj_mfma) ? 1 : 0;
   e.det = A;
   e.det_smem = det_smem;
+}
+
+// Lane-group width of k_deriv_jas, whose lanes take whole electrons: the
+// narrowest that holds them, so that few lanes idle
+static int deriv_jas_width(const qmcw_handle *h) {
+  const int N = h->A.S.N;
+  return N <= 8 ? 8 : N <= 16 ? 16 : N <= 32 ? 32 : 64;
 }
 
 static void launch_eval(qmcw_handle *h, bool derivs) {
@@ -681,11 +690,6 @@ static void launch_eval(qmcw_handle *h, bool derivs) {
   prof_begin(h, QMCW_PROF_FULL_JAS);
   K.full_jas(cj);
   prof_end(h);
-  if (derivs) {
-    prof_begin(h, QMCW_PROF_DERIV_JAS);
-    K.deriv_jas(cj);
-    prof_end(h);
-  }
   prof_begin(h, QMCW_PROF_FULL_DET);
   DISPATCH_GW(gd, launch_det, h, A, det_smem);
   if (A.orb_mfma)
@@ -716,8 +720,19 @@ static void launch_eval(qmcw_handle *h, bool derivs) {
   DISPATCH_GW(gd, launch_fin, h, A);
   prof_end(h);
   if (derivs) {
+    // after the determinants: the slots need each electron's whole velocity
+    LaunchCtx cd = cj;
+    cd.G = deriv_jas_width(h);
+    prof_begin(h, QMCW_PROF_DERIV_JAS);
+    K.deriv_jas(cd);
+    prof_end(h);
     prof_begin(h, QMCW_PROF_DERIVS);
-    DISPATCH_GW(gd, launch_derivs_asm, h, A);
+    // its intermediates in LDS while four blocks fit a compute unit's 160 KB
+    const size_t lds = sizeof(double) * derivs_lds_doubles(A.S);
+    if (h->use_lds && lds <= 40 * 1024)
+      hipLaunchKernelGGL((k_derivs<64, true>), dim3(h->Wl), dim3(kWave), lds, h->stream, A, h->der);
+    else
+      DISPATCH_GW(gd, launch_derivs_asm, h, A);
     prof_end(h);
     h->der_valid = 1;
   }
@@ -1237,11 +1252,10 @@ extern "C" int qmcw_create(const qmcw_system *s, int32_t nwalk, int32_t precisio
   if (S.nparm > 0) {
     DLayout &DL = h->A.DL;
     int64_t NM = (int64_t)N * M;
-    DL.raw = take((int64_t)S.nslot * N * 5);
-    DL.gvalue = take(S.npj); DL.gjas = take((int64_t)S.npj * N * 3); DL.d2g = take(S.npj);
-    DL.pbc = take(NM * NB); DL.dpe_raw = take(NM * S.nslot);
-    DL.dpe_slot = take(S.nslot); DL.dpe = take(S.npj); DL.pnl = take((int64_t)N * NO);
-    DL.btd = take(NM); DL.uqd = take((int64_t)kWave * N);
+    DL.dj = take(2 * (int64_t)S.nslot); DL.pw = take(S.nloc > 0 ? 2 * NM * S.nquad : 1);
+    DL.pbc = take((int64_t)N * NB);
+    DL.dpe_slot = take(S.nslot); DL.pnl = take((int64_t)N * NO);
+    DL.tb = take(NM); DL.tu = take(4 * (int64_t)N * N); DL.uqd = take((int64_t)kWave * N);
     DL.B = take((int64_t)N * NO);
     for (int sp = 0; sp < 2; sp++) {
       DL.tfull[sp] = take((int64_t)D.ns[sp] * NO); DL.dt[sp] = take((int64_t)D.ns[sp] * NO);

@@ -8,519 +8,534 @@
 
 namespace qmcw {
 
-// Per-slot derivative pieces go to base[slot * rs + c], c = 0 value,
-// 1..3 gradient, 4 laplacian.
-struct SlotAcc {
-  double *base;
-  int64_t rs;
-  __device__ __forceinline__ void add(int slot, int c, double v) const { base[slot * rs + c] += v; }
-  // all five pieces of a slot: the old values are read together before the
-  // stores, one memory round trip instead of five
-  __device__ __forceinline__ void add5(int slot, double v, double g0, double g1, double g2,
-                                       double l) const {
-    double *p = base + slot * rs;
-    const double o0 = p[0], o1 = p[1], o2 = p[2], o3 = p[3], o4 = p[4];
-    p[0] = o0 + v; p[1] = o1 + g0; p[2] = o2 + g1; p[3] = o3 + g2; p[4] = o4 + l;
+// The slot pieces are sums: over the electrons and their pairs for the
+// Jastrow's own derivatives (k_deriv_jas), over the quadrature points for the
+// pseudopotential's (k_deriv_nlpp).  Both keep the sums of a slot group in
+// registers over a lane's whole share and add the lanes up at the end; an
+// update in memory per (pair, centre, slot) took 640 and 1,090 us of a
+// derivative evaluation of 8,192 C2-like walkers (here 130 and 489), and 1,138
+// and 2,589 of one of 601 walkers of a 25-electron molecule, whose call went
+// from 5.3 to 2.5 ms.
+
+// number of e-e-n terms with power k of U (all of them: k = -1)
+template <int ORD>
+__host__ __device__ constexpr int een_count(int kk) {
+  int n = 0;
+  for (int k = 0; k <= ORD; k++)
+    for (int m = 0; 2 * m <= ORD - k; m++)
+      for (int l = 0; l <= ORD - k - 2 * m; l++)
+        if (QMCW_EEN_TERM(k, l, m) && (kk < 0 || k == kk)) n++;
+  return n;
+}
+// index of the first term with power k of U
+template <int ORD>
+__host__ __device__ constexpr int een_first(int kk) {
+  int n = 0;
+  for (int k = 0; k < kk; k++) n += een_count<ORD>(k);
+  return n;
+}
+
+// Derivatives of an e-n (or e-e) Pade + polynomial term with respect to its
+// coefficients, at scaled distance u, with their first two u derivatives, for
+// coefficient iw = 1, 2, ... (1 and 2 the Pade form's; qmc/vmc/
+// deriv_jastrow4.f90:95-220, 880-1090).  The powers advance with iw.
+struct PadeSlots {
+  double u, c0, c1, s, ar, bt, bta;     // coefficients of the form, spin factor, scaled distance at infinity
+  double up, arp, um1, um2;
+  __device__ __forceinline__ PadeSlots(double u_, double c0_, double c1_, double s_, double ar_)
+      : u(u_), c0(c0_), c1(c1_), s(s_), ar(ar_), bt(1.0 / (1.0 + c1_ * u_)), bta(1.0 / (1.0 + c1_ * ar_)),
+        up(u_), arp(ar_), um1(1.0), um2(0.0) {}
+  __device__ __forceinline__ void get(int iw, double &g, double &g1, double &g2) {
+    if (iw == 1) {
+      g = s * (u * bt - ar * bta);
+      g1 = s * bt * bt;
+      g2 = -2.0 * c1 * g1 * bt;
+    } else if (iw == 2) {
+      g = s * c0 * (ar * ar * bta * bta - u * u * bt * bt);
+      g1 = -2.0 * s * c0 * u * bt * bt * bt;
+      g2 = -2.0 * s * c0 * (1.0 - 2.0 * c1 * u) * bt * bt * bt * bt;
+    } else {
+      const int io = iw - 1;
+      um2 = um1;
+      um1 = up;
+      up *= u;
+      arp *= ar;
+      g = up - arp;
+      g1 = io * um1;
+      g2 = io * (io - 1) * um2;
+    }
   }
 };
 
-// a-coefficient pieces of the e-n terms of one electron (distances r[M],
-// vectors rv[3M]), qmc/vmc/deriv_jastrow4.f90:880-1090.  cv scales the value
-// pieces (0: none); FULL adds the gradient and the laplacian.
-template <bool FULL, typename RA, typename RVA>
-__device__ void en_slots(const DevSys &S, RA r, RVA rv, double cv, const SlotAcc &acc) {
-  const double k = S.scalek, ar = S.asymp_r;
-  const int na = S.norda + 1;
-  for (int ic = 0; ic < S.M; ic++) {
-    const int it = cst(S.iwctype)[ic];
-    const double ri = r[ic];
-    double rr, d7, d9;
-    scaled<double>(S.isc, k, ri, rr, d7, d9);
-    const double *a = S.a4 + it * na;
-    double rp = rr, arp = ar, rpm1 = 1.0, rpm2 = 0.0;   // rr^iord, ar^iord, rr^(iord-1), rr^(iord-2)
-    for (int iw = 1; iw <= na; iw++) {
-      double gen, geni, genii;
-      if (iw == 1) {
-        double bt = 1.0 + a[1] * rr, bta = 1.0 + a[1] * ar;
-        gen = rr / bt - ar / bta;
-        geni = 1.0 / (bt * bt);
-        genii = -2.0 * a[1] * geni / bt;
-      } else if (iw == 2) {
-        double t = -a[0] * rr * rr, ti = -2.0 * a[0] * rr, tii = -2.0 * a[0];
-        double bot0 = 1.0 + a[1] * rr, bt = bot0 * bot0, bt2 = bt * bt;
-        double bta = 1.0 + a[1] * ar;
-        gen = t / bt + a[0] * ar * ar / (bta * bta);
-        geni = ti / (bt * bot0);
-        genii = tii * (1.0 - 2.0 * a[1] * rr) / bt2;
-      } else {
-        // iord = iw - 1 >= 2: advance the powers to iord
-        rpm2 = rpm1;
-        rpm1 = rp;
-        rp *= rr;
-        arp *= ar;
-        const int iord = iw - 1;
-        gen = rp - arp;
-        geni = iord * rpm1;
-        genii = iord * (iord - 1) * rpm2;
-      }
-      const int slot = it * na + iw - 1;
-      if (FULL) {
-        genii = genii * d7 * d7 + geni * d9;
-        geni = geni * d7 / ri;
-        acc.add5(slot, cv != 0.0 ? cv * gen : 0.0, geni * rv[3 * ic], geni * rv[3 * ic + 1],
-                 geni * rv[3 * ic + 2], genii + 2.0 * geni);
-      } else if (cv != 0.0) {
-        acc.add(slot, 0, cv * gen);
-      }
-    }
-  }
+// e-e coefficients and spin factor of a pair
+__device__ __forceinline__ int b_spin(const DevSys &S, bool par, double &sspinn) {
+  sspinn = 1.0;
+  if (!par) return 0;
+  if (S.nspin2b == 2) return 1;
+  if (S.nocuspb == 0) sspinn = 0.5;
+  return 0;
 }
 
-// e-e-n term pieces of one (pair, centre): term values U^k (A^(l+m) B^m +
-// A^m B^(l+m)) and, with FULL, their gradient wrt r_i and the part of the
-// laplacian that belongs to electron i (qmc/vmc/deriv_jastrow4.f90:330-720).
-template <bool FULL, int ORD>
-__device__ __forceinline__ void een_slots(double U, double A, double B, double Ud1, double Ud2,
-                                          double Ad1, double Ad2, double rij, double ri,
-                                          const double *rvij, const double *rvi, double u2pst,
-                                          double cv, const SlotAcc &acc, int slot0) {
-  double up[ORD + 1], ap[ORD + 1], bp[ORD + 1];
-  up[0] = ap[0] = bp[0] = 1.0;
-#pragma unroll
-  for (int q = 1; q <= ORD; q++) { up[q] = up[q - 1] * U; ap[q] = ap[q - 1] * A; bp[q] = bp[q - 1] * B; }
-  int idx = 0;
-#pragma unroll
-  for (int k = 0; k <= ORD; k++)
-#pragma unroll
-    for (int m = 0; 2 * m <= ORD - k; m++)
-#pragma unroll
-      for (int l = 0; l <= ORD - k - 2 * m; l++)
-        if (QMCW_EEN_TERM(k, l, m)) {
-          const int lm = l + m;
-          const int slot = slot0 + idx;
-          idx++;
-          const double P = ap[lm] * bp[m] + ap[m] * bp[lm];
-          if (!FULL && cv != 0.0) acc.add(slot, 0, cv * up[k] * P);
-          if (FULL) {
-            double PA = (lm ? lm * ap[lm > 0 ? lm - 1 : 0] * bp[m] : 0.0) +
-                        (m ? m * ap[m > 0 ? m - 1 : 0] * bp[lm] : 0.0);
-            double PAA = (lm > 1 ? lm * (lm - 1) * ap[lm > 1 ? lm - 2 : 0] * bp[m] : 0.0) +
-                         (m > 1 ? m * (m - 1) * ap[m > 1 ? m - 2 : 0] * bp[lm] : 0.0);
-            double Uk = up[k];
-            double Uk1 = k ? k * up[k > 0 ? k - 1 : 0] : 0.0;
-            double Uk2 = k > 1 ? k * (k - 1) * up[k > 1 ? k - 2 : 0] : 0.0;
-            double gu = Uk1 * P, guu = Uk2 * P, gi = Uk * PA, gii = Uk * PAA, gui = Uk1 * PA;
-            guu = guu * Ud1 * Ud1 + gu * Ud2;
-            gu = gu * Ud1 / rij;
-            gui = gui * Ud1 * Ad1;
-            gii = gii * Ad1 * Ad1 + gi * Ad2;
-            gi = gi * Ad1 / ri;
-            acc.add5(slot, cv != 0.0 ? cv * up[k] * P : 0.0, gi * rvi[0] + gu * rvij[0],
-                     gi * rvi[1] + gu * rvij[1], gi * rvi[2] + gu * rvij[2],
-                     2.0 * (gu + gi) + guu + gii + gui * u2pst / (ri * rij));
-          }
-        }
-}
-
-// b-coefficient and e-e-n term pieces of the pair (i, j) seen from electron
-// i: rij, rvij = r_i - r_j, the distances of i and j to the centres and i's
-// vectors to them (qmc/vmc/deriv_jastrow4.f90:95-720).  cv scales the value
-// pieces (0: none); FULL adds the gradient wrt r_i and i's laplacian part.
-template <bool FULL>
-__device__ void b_slots(const DevSys &S, bool par, double rij, const double *rvij, double cv,
-                        const SlotAcc &acc) {
-  const double k = S.scalek, ar = S.asymp_r;
-  double sspinn = 1.0;
-  int isb = 0;
-  if (par) {
-    if (S.nspin2b == 2) isb = 1;
-    else if (S.nocuspb == 0) sspinn = 0.5;
-  }
-  const int nb = S.nordb + 1;
-  const double *b = S.b + isb * nb;
-  double u, dd1, dd2;
-  scaled<double>(S.isc, k, rij, u, dd1, dd2);
-  double up_ = u, arp = ar, upm1 = 1.0, upm2 = 0.0;
-  for (int iw = 1; iw <= nb; iw++) {
-    double gee, geeu, geeuu;
-    if (iw == 1) {
-      double bt = 1.0 + b[1] * u, bta = 1.0 + b[1] * ar;
-      gee = sspinn * u / bt - sspinn * ar / bta;
-      geeu = sspinn / (bt * bt);
-      geeuu = -2.0 * b[1] * geeu / bt;
-    } else if (iw == 2) {
-      double t = -sspinn * b[0] * u * u, tu = -sspinn * 2.0 * b[0] * u, tuu = -sspinn * 2.0 * b[0];
-      double bot0 = 1.0 + b[1] * u, bt = bot0 * bot0, bt2 = bt * bt;
-      double bta = 1.0 + b[1] * ar;
-      gee = t / bt + sspinn * b[0] * ar * ar / (bta * bta);
-      geeu = tu / (bt * bot0);
-      geeuu = tuu * (1.0 - 2.0 * b[1] * u) / bt2;
-    } else {
-      upm2 = upm1;
-      upm1 = up_;
-      up_ *= u;
-      arp *= ar;
-      const int iord = iw - 1;
-      gee = up_ - arp;
-      geeu = iord * upm1;
-      geeuu = iord * (iord - 1) * upm2;
-    }
-    const int slot = S.slot_b0 + isb * nb + iw - 1;
-    if (FULL) {
-      geeuu = geeuu * dd1 * dd1 + geeu * dd2;
-      geeu = geeu * dd1 / rij;
-      acc.add5(slot, cv != 0.0 ? cv * gee : 0.0, geeu * rvij[0], geeu * rvij[1], geeu * rvij[2],
-               geeuu + 2.0 * geeu);
-    } else if (cv != 0.0) {
-      acc.add(slot, 0, cv * gee);
-    }
-  }
-}
-
-template <bool FULL, int ORD>
-__device__ void pair_slots(const DevSys &S, bool par, double rij, const double *rvij,
-                           const double *ri_v, const double *rj_v, const double *rvi, double cv,
-                           const SlotAcc &acc) {
-  const double k = S.scalek;
-  b_slots<FULL>(S, par, rij, rvij, cv, acc);
-  if (S.nordc <= 1) return;
-  double U, Ud1, Ud2;
-  scaled<double>(S.isc, k, rij, U, Ud1, Ud2);
-  U = 1.0 - k * U; Ud1 = -k * Ud1; Ud2 = -k * Ud2;
-  for (int ic = 0; ic < S.M; ic++) {
-    const int it = cst(S.iwctype)[ic];
-    const double ri = ri_v[ic], rj = rj_v[ic];
-    double A, Ad1, Ad2, B, Bd1, Bd2;
-    scaled<double>(S.isc, k, ri, A, Ad1, Ad2);
-    scaled<double>(S.isc, k, rj, B, Bd1, Bd2);
-    A = 1.0 - k * A; Ad1 = -k * Ad1; Ad2 = -k * Ad2;
-    B = 1.0 - k * B;
-    (void)Bd1; (void)Bd2;
-    const double u2pst = rij * rij + ri * ri - rj * rj;
-    een_slots<FULL, ORD>(U, A, B, Ud1, Ud2, Ad1, Ad2, rij, ri, rvij,
-                         FULL ? rvi + 3 * ic : nullptr, u2pst, cv, acc,
-                         S.slot_c0 + it * S.nterms);
-  }
-}
-
-// Value pieces, weighted by cv, of the b-coefficient and e-e-n terms of all
-// pairs (i, j), electron i at xn (distances ri_v to the centres) and every
-// other electron where it is (btd[j * M + ic] = 1 - k scaled(r_j,ic);
-// uqd: per-lane scratch of N values).  Summed over j, the term values of a
-// centre are A^(l+m) S(k, m) + A^m S(k, l+m) with S(k, n) = sum_j U_j^k B_j^n,
-// so each slot takes one addition per call.
-template <int ORD, typename RA, typename UA>
-__device__ void point_pair_slots(const DevSys &S, int i, const double *xn, const double *x,
-                                 RA ri_v, const double *btd, UA uqd, double cv, const SlotAcc &acc) {
+// One power K of U of the e-e-n slots of centre type it (k_deriv_jas): over
+// this lane's electrons i, the type's centres and the other electrons j,
+// with S_n = sum_j U^K B^n, X_n its part of i's laplacian plus twice its
+// gradient along v_i and R_n its gradient along the vector to the centre
+// (see k_deriv_jas), each term takes two entries of each.
+template <int G, int ORD, int K>
+__device__ __forceinline__ void deriv_een_power(const KArgs &A, const double *ws, const double *ss, int it,
+                                                double *dj, int lane) {
+  const DevSys &S = A.S;
   const int N = S.N, M = S.M;
-  const double k = S.scalek, ar = S.asymp_r;
-  // b-coefficient pieces summed over the other electrons in registers
-  // (b_slots' value terms), one update per slot afterwards
-  const int nb = S.nordb + 1;
-  double ab0[QMCW_MAX_ORD + 1], ab1[QMCW_MAX_ORD + 1];
+  constexpr int NN = ORD - K + 1, NT = een_count<ORD>(K);
+  if constexpr (NT > 0) {
+    const double *x = ws + A.L.x, *ren = ws + A.L.r_en, *rven = ws + A.L.rvec_en;
+    const double *vj = ss + A.SL.vj, *vd = ss + A.SL.vd;
+    const double *tu = ss + A.DL.tu, *tb = ss + A.DL.tb;
+    const int64_t NN2 = (int64_t)N * N;
+    const double k = S.scalek, hb = S.hb;
+    double av[NT], ae[NT];
 #pragma unroll
-  for (int q = 0; q <= QMCW_MAX_ORD; q++) ab0[q] = ab1[q] = 0.0;
-  for (int jj = 0; jj < N; jj++) {
-    if (jj == i) continue;
-    const double dx = xn[0] - x[3 * jj], dy = xn[1] - x[3 * jj + 1], dz = xn[2] - x[3 * jj + 2];
-    const double rij = sqrt(dx * dx + dy * dy + dz * dz);
-    double u, d1, d2;
-    scaled<double>(S.isc, k, rij, u, d1, d2);
-    uqd[jj] = 1.0 - k * u;
-    double sspinn = 1.0;
-    int isb = 0;
-    if ((i < S.nup) == (jj < S.nup)) {
-      if (S.nspin2b == 2) isb = 1;
-      else if (S.nocuspb == 0) sspinn = 0.5;
-    }
-    const cptr<double> b = cst(S.b) + isb * nb;
-    double up_ = u, arp = ar;
+    for (int q = 0; q < NT; q++) av[q] = ae[q] = 0.0;
+    for (int i = lane; i < N; i += G) {
+      const double vi[3] = {vj[3 * i] + vd[3 * i], vj[3 * i + 1] + vd[3 * i + 1], vj[3 * i + 2] + vd[3 * i + 2]};
+      for (int c = cst(S.tc_off)[it]; c < cst(S.tc_off)[it + 1]; c++) {
+        const int ic = ((cptr<TypeCent>)S.tcent)[c].ic;
+        const double ri = ren[i * M + ic];
+        const double rv[3] = {rven[(i * M + ic) * 3], rven[(i * M + ic) * 3 + 1], rven[(i * M + ic) * 3 + 2]};
+        double s0[NN], x0[NN], r0[NN];
 #pragma unroll
-    for (int iw = 1; iw <= QMCW_MAX_ORD + 1; iw++) {
-      if (iw > nb) continue;
-      double gee;
-      if (iw == 1) {
-        const double bt = 1.0 + b[1] * u, bta = 1.0 + b[1] * ar;
-        gee = sspinn * u / bt - sspinn * ar / bta;
-      } else if (iw == 2) {
-        const double t = -sspinn * b[0] * u * u;
-        const double bot0 = 1.0 + b[1] * u, bt = bot0 * bot0, bta = 1.0 + b[1] * ar;
-        gee = t / bt + sspinn * b[0] * ar * ar / (bta * bta);
-      } else {
-        up_ *= u;
-        arp *= ar;
-        gee = up_ - arp;
-      }
-      if (isb) ab1[iw - 1] += cv * gee;
-      else ab0[iw - 1] += cv * gee;
-    }
-  }
-  {
-    double *bs = acc.base + (int64_t)S.slot_b0 * acc.rs;
-    const int nsb = S.nspin2b == 2 ? 2 : 1;
-    double o0[QMCW_MAX_ORD + 1], o1[QMCW_MAX_ORD + 1];
+        for (int n = 0; n < NN; n++) s0[n] = x0[n] = r0[n] = 0.0;
+        for (int j = 0; j < N; j++) {
+          if (j == i) continue;
+          const double U = tu[j * N + i], B = tb[ic * N + j];
+          double uk2 = 1.0;                     // U^(K-2)
 #pragma unroll
-    for (int q = 0; q <= QMCW_MAX_ORD; q++) {
-      o0[q] = q < nb ? bs[(int64_t)q * acc.rs] : 0.0;
-      o1[q] = (nsb == 2 && q < nb) ? bs[(int64_t)(nb + q) * acc.rs] : 0.0;
-    }
-#pragma unroll
-    for (int q = 0; q <= QMCW_MAX_ORD; q++) {
-      if (q < nb) bs[(int64_t)q * acc.rs] = o0[q] + ab0[q];
-      if (nsb == 2 && q < nb) bs[(int64_t)(nb + q) * acc.rs] = o1[q] + ab1[q];
-    }
-  }
-  if (S.nordc <= 1) return;
-  constexpr int NG = een_gi<ORD>(ORD, 0) + 1;
-  for (int ic = 0; ic < M; ic++) {
-    double sg[NG];
-#pragma unroll
-    for (int q = 0; q < NG; q++) sg[q] = 0.0;
-    for (int jj = 0; jj < N; jj++) {
-      if (jj == i) continue;
-      const double U = uqd[jj], B = btd[jj * M + ic];
-      double uk = 1.0;
-#pragma unroll
-      for (int kk = 0; kk <= ORD; kk++) {
-        double t = uk;
-#pragma unroll
-        for (int n = 0; n <= ORD - kk; n++) {
-          sg[een_gi<ORD>(kk, n)] += t;
-          t *= B;
-        }
-        uk *= U;
-      }
-    }
-    double A, t1, t2;
-    scaled<double>(S.isc, k, ri_v[ic], A, t1, t2);
-    A = 1.0 - k * A;
-    double ap[ORD + 1];
-    ap[0] = 1.0;
-#pragma unroll
-    for (int q = 1; q <= ORD; q++) ap[q] = ap[q - 1] * A;
-    const int slot0 = S.slot_c0 + cst(S.iwctype)[ic] * S.nterms;
-    int idx = 0;
-#pragma unroll
-    for (int kk = 0; kk <= ORD; kk++)
-#pragma unroll
-      for (int m = 0; 2 * m <= ORD - kk; m++)
-#pragma unroll
-        for (int l = 0; l <= ORD - kk - 2 * m; l++)
-          if (QMCW_EEN_TERM(kk, l, m)) {
-            acc.add(slot0 + idx, 0, cv * (ap[l + m] * sg[een_gi<ORD>(kk, m)] +
-                                          ap[m] * sg[een_gi<ORD>(kk, l + m)]));
-            idx++;
+          for (int q = 0; q < K - 2; q++) uk2 *= U;
+          const double uk1 = K >= 2 ? uk2 * U : 1.0, uk = K >= 1 ? uk1 * U : 1.0;
+          double s = uk, xx = 0.0, r = 0.0;
+          if (K >= 1) {
+            // gu = Ud1 / rij, l1 = Ud2 + 2 Ud1 / rij, l2 = Ud1^2
+            const double gu = tu[NN2 + j * N + i], l1 = tu[2 * NN2 + j * N + i], l2 = tu[3 * NN2 + j * N + i];
+            const double d[3] = {x[3 * i] - x[3 * j], x[3 * i + 1] - x[3 * j + 1], x[3 * i + 2] - x[3 * j + 2]};
+            const double fu = K * uk1, gd = fu * gu;
+            xx = fu * l1 + (K >= 2 ? K * (K - 1) * uk2 * l2 : 0.0) +
+                 2.0 * gd * (d[0] * vi[0] + d[1] * vi[1] + d[2] * vi[2]);
+            r = gd * (d[0] * rv[0] + d[1] * rv[1] + d[2] * rv[2]);
           }
+#pragma unroll
+          for (int n = 0; n < NN; n++) {
+            s0[n] += s;
+            s *= B;
+            if (K >= 1) {
+              x0[n] += xx;
+              r0[n] += r;
+              xx *= B;
+              r *= B;
+            }
+          }
+        }
+        double A0, Ad1, Ad2;
+        scaled<double>(S.isc, k, ri, A0, Ad1, Ad2);
+        A0 = 1.0 - k * A0; Ad1 = -k * Ad1; Ad2 = -k * Ad2;
+        double ap[ORD + 1];
+        ap[0] = 1.0;
+#pragma unroll
+        for (int q = 1; q <= ORD; q++) ap[q] = ap[q - 1] * A0;
+        const double da = Ad1 / ri, l2 = Ad1 * Ad1;
+        const double l1 = Ad2 + 2.0 * da * (1.0 + rv[0] * vi[0] + rv[1] * vi[1] + rv[2] * vi[2]);
+        int idx = 0;
+#pragma unroll
+        for (int m = 0; 2 * m <= ORD - K; m++)
+#pragma unroll
+          for (int l = 0; l <= ORD - K - 2 * m; l++)
+            if (QMCW_EEN_TERM(K, l, m)) {
+              const int p = l + m;
+              // every ordered pair is met from both sides: half the value each
+              av[idx] += 0.5 * (ap[p] * s0[m] + ap[m] * s0[p]);
+              double e = ap[p] * x0[m] + ap[m] * x0[p];
+              if (p >= 1) e += p * ap[p >= 1 ? p - 1 : 0] * (l1 * s0[m] + 2.0 * da * r0[m]);
+              if (m >= 1) e += m * ap[m >= 1 ? m - 1 : 0] * (l1 * s0[p] + 2.0 * da * r0[p]);
+              if (p >= 2) e += p * (p - 1) * ap[p >= 2 ? p - 2 : 0] * l2 * s0[m];
+              if (m >= 2) e += m * (m - 1) * ap[m >= 2 ? m - 2 : 0] * l2 * s0[p];
+              ae[idx] += e;
+              idx++;
+            }
+      }
+    }
+    const int s1 = S.slot_c0 + it * S.nterms + een_first<ORD>(K);
+#pragma unroll
+    for (int q = 0; q < NT; q++) {
+      const double v = gsum<G>(av[q]), e = gsum<G>(ae[q]);
+      if (lane == 0) { dj[2 * (s1 + q)] = v; dj[2 * (s1 + q) + 1] = -hb * e; }
+    }
   }
+}
+template <int G, int ORD, int K>
+__device__ __forceinline__ void deriv_een_powers(const KArgs &A, const double *ws, const double *ss, int it,
+                                                 double *dj, int lane) {
+  deriv_een_power<G, ORD, K>(A, ws, ss, it, dj, lane);
+  if constexpr (K < ORD) deriv_een_powers<G, ORD, K + 1>(A, ws, ss, it, dj, lane);
 }
 
 // ---------------------------------------------------------------------------
-// Jastrow parameter derivatives of the current configuration: gvalue(p),
-// g(p, i) = d grad_i ln J / dp and d2g(p) = d lap ln J / dp
-// (qmc/vmc/deriv_jastrow4.f90).  Each lane takes whole electrons: it visits
-// every pair (i, j) from i's side, so its rows of the slot pieces are its own.
+// Jastrow parameter derivatives of the current configuration, per slot
+// (qmc/vmc/deriv_jastrow4.f90): dj[slot] = {d ln J / dc,
+// -hb (d lap ln J / dc + 2 sum_i v_i . d grad_i ln J / dc)} with v_i the
+// electron's whole velocity (k_full_det has run): what d ln Psi/dp and
+// dE_L/dp need of them, so no gradient per electron and slot is kept.  Each
+// lane takes whole electrons i and every pair (i, j) from i's side.  For a
+// power k of U and a centre, the sums over j of U^k B^n (and of its gradient
+// and laplacian parts) serve all terms of that power.
 template <int G, int ORD>
 __global__ QMCW_HEAVY void k_deriv_jas(KArgs A) {
   QMCW_GROUP_SETUP
-  const int N = S.N, M = S.M, nsl = S.nslot;
+  const int N = S.N, M = S.M;
   const WLayout &L = A.L;
-  const DLayout &DL = A.DL;
-  const double *ren = ws + L.r_en, *rven = ws + L.rvec_en, *ree = ws + L.r_ee, *rvee = ws + L.rvec_ee;
-  double *raw = ss + DL.raw;
-  for (int t = lane; t < nsl * N * 5; t += G) raw[t] = 0.0;
-  __syncthreads();
-  for (int i = lane; i < N; i += G) {
-    const SlotAcc acc{raw + 5 * i, (int64_t)N * 5};
-    en_slots<true>(S, ren + i * M, rven + i * M * 3, 1.0, acc);
-    for (int j = 0; j < N; j++) {
-      if (j == i) continue;
-      const int hi = i > j ? i : j, lo = i > j ? j : i;
-      const double sg = i > j ? 1.0 : -1.0;   // rvec_ee(hi, lo) = r_hi - r_lo
-      const double *rv = rvee + 3 * (hi * N + lo);
-      const double rvij[3] = {sg * rv[0], sg * rv[1], sg * rv[2]};
-      const bool par = (hi < S.nup) || (lo >= S.nup);
-      pair_slots<true, ORD>(S, par, ree[hi * N + lo], rvij, ren + i * M, ren + j * M,
-                       rven + i * M * 3, j < i ? 1.0 : 0.0, acc);
+  const double *x = ws + L.x, *ren = ws + L.r_en, *rven = ws + L.rvec_en;
+  const double *vj = ss + A.SL.vj, *vd = ss + A.SL.vd;
+  double *tu = ss + A.DL.tu, *tb = ss + A.DL.tb, *dj = ss + A.DL.dj;
+  const double k = S.scalek, ar = S.asymp_r, hb = S.hb;
+  constexpr int MW = QMCW_MAX_ORD + 1;
+  // ---- a-coefficients, a centre type at a time
+  const int na = S.norda + 1;
+  for (int it = 0; it < S.nctype; it++) {
+    double av[MW], ae[MW];
+#pragma unroll
+    for (int q = 0; q < MW; q++) av[q] = ae[q] = 0.0;
+    for (int i = lane; i < N; i += G) {
+      const double vi[3] = {vj[3 * i] + vd[3 * i], vj[3 * i + 1] + vd[3 * i + 1], vj[3 * i + 2] + vd[3 * i + 2]};
+      for (int c = cst(S.tc_off)[it]; c < cst(S.tc_off)[it + 1]; c++) {
+        const int p = i * M + ((cptr<TypeCent>)S.tcent)[c].ic;
+        const double ri = ren[p];
+        double u, d7, d9;
+        scaled<double>(S.isc, k, ri, u, d7, d9);
+        const double gd = d7 / ri * (1.0 + rven[3 * p] * vi[0] + rven[3 * p + 1] * vi[1] + rven[3 * p + 2] * vi[2]);
+        PadeSlots ps(u, cst(S.a4)[it * na], cst(S.a4)[it * na + 1], 1.0, ar);
+#pragma unroll
+        for (int iw = 1; iw <= MW; iw++) {
+          if (iw > na) continue;
+          double g, g1, g2;
+          ps.get(iw, g, g1, g2);
+          av[iw - 1] += g;
+          ae[iw - 1] += g2 * d7 * d7 + g1 * (d9 + 2.0 * gd);
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < MW; q++) {
+      if (q >= na) continue;
+      const double v = gsum<G>(av[q]), e = gsum<G>(ae[q]);
+      if (lane == 0) { dj[2 * (it * na + q)] = v; dj[2 * (it * na + q) + 1] = -hb * e; }
     }
   }
-  __syncthreads();
-  double *gv = ss + DL.gvalue, *gj = ss + DL.gjas, *d2g = ss + DL.d2g;
-  for (int t = lane; t < S.npj * N; t += G) {
-    const int p = t / N, i = t % N;
-    double g0 = 0.0, g1 = 0.0, g2 = 0.0;
-    for (int q = cst(S.pj_off)[p]; q < cst(S.pj_off)[p + 1]; q++) {
-      const double w = cst(S.pj_w)[q];
-      const double *r = raw + ((int64_t)cst(S.pj_slot)[q] * N + i) * 5;
-      g0 += w * r[1]; g1 += w * r[2]; g2 += w * r[3];
-    }
-    gj[3 * t] = g0; gj[3 * t + 1] = g1; gj[3 * t + 2] = g2;
+  // ---- b-coefficients, and the pair tables of the e-e-n terms: per (j, i)
+  // U, Ud1 / rij, Ud2 + 2 Ud1 / rij and Ud1^2, per (centre, j) B
+  const int nb = S.nordb + 1;
+  const int64_t NN2 = (int64_t)N * N;
+  for (int p = lane; p < N * M; p += G) {
+    double b, t1, t2;
+    scaled<double>(S.isc, k, ren[p], b, t1, t2);
+    tb[(p % M) * N + p / M] = 1.0 - k * b;
   }
-  for (int p = lane; p < S.npj; p += G) {
-    double v = 0.0, d = 0.0;
-    for (int q = cst(S.pj_off)[p]; q < cst(S.pj_off)[p + 1]; q++) {
-      const double w = cst(S.pj_w)[q];
-      const double *r = raw + (int64_t)cst(S.pj_slot)[q] * N * 5;
-      double sv = 0.0, sd = 0.0;
-      for (int i = 0; i < N; i++) { sv += r[5 * i]; sd += r[5 * i + 4]; }
-      v += w * sv;
-      d += w * sd;
+  for (int isb = 0; isb < (S.nspin2b == 2 ? 2 : 1); isb++) {
+    double av[MW], ae[MW];
+#pragma unroll
+    for (int q = 0; q < MW; q++) av[q] = ae[q] = 0.0;
+    for (int i = lane; i < N; i += G) {
+      const double vi[3] = {vj[3 * i] + vd[3 * i], vj[3 * i + 1] + vd[3 * i + 1], vj[3 * i + 2] + vd[3 * i + 2]};
+      for (int j = 0; j < N; j++) {
+        if (j == i) continue;
+        const double d[3] = {x[3 * i] - x[3 * j], x[3 * i + 1] - x[3 * j + 1], x[3 * i + 2] - x[3 * j + 2]};
+        const double rij = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
+        double u, d1, d2;
+        scaled<double>(S.isc, k, rij, u, d1, d2);
+        const double dr = d1 / rij;
+        if (isb == 0) {
+          tu[j * N + i] = 1.0 - k * u;
+          tu[NN2 + j * N + i] = -k * dr;
+          tu[2 * NN2 + j * N + i] = -k * (d2 + 2.0 * dr);
+          tu[3 * NN2 + j * N + i] = k * k * d1 * d1;
+        }
+        double sp;
+        if (b_spin(S, (i < S.nup) == (j < S.nup), sp) != isb) continue;
+        const double gd = dr * (1.0 + d[0] * vi[0] + d[1] * vi[1] + d[2] * vi[2]);
+        PadeSlots ps(u, cst(S.b)[isb * nb], cst(S.b)[isb * nb + 1], sp, ar);
+#pragma unroll
+        for (int iw = 1; iw <= MW; iw++) {
+          if (iw > nb) continue;
+          double g, g1, g2;
+          ps.get(iw, g, g1, g2);
+          av[iw - 1] += 0.5 * g;
+          ae[iw - 1] += g2 * d1 * d1 + g1 * (d2 + 2.0 * gd);
+        }
+      }
     }
-    gv[p] = v;
-    d2g[p] = d;
+#pragma unroll
+    for (int q = 0; q < MW; q++) {
+      if (q >= nb) continue;
+      const double v = gsum<G>(av[q]), e = gsum<G>(ae[q]);
+      const int sl = S.slot_b0 + isb * nb + q;
+      if (lane == 0) { dj[2 * sl] = v; dj[2 * sl + 1] = -hb * e; }
+    }
+  }
+  if (S.nordc <= 1) return;
+  __syncthreads();
+  for (int it = 0; it < S.nctype; it++) deriv_een_powers<G, ORD, 0>(A, ws, ss, it, dj, lane);
+}
+
+// Quadrature point, or (t >= npt) pair taken at the electron's current
+// position, that lane entry t of k_deriv_nlpp stands for: position,
+// electron and the weight of its slot pieces
+__device__ __forceinline__ void nlpp_entry(const KArgs &A, const double *ws, const double *pw, const int *plist,
+                                           int npt, int t, double *xn, int &i, double &wt) {
+  const DevSys &S = A.S;
+  const int nq = S.nquad, M = S.M;
+  const double *x = ws + A.L.x, *quad = ws + A.L.quad;
+  if (t < npt) {
+    const int iq = t % nq, p = plist[t / nq], ic = p % M;
+    i = p / M;
+    const double r = ws[A.L.r_en + p];
+#pragma unroll
+    for (int q = 0; q < 3; q++) xn[q] = r * quad[q * nq + iq] + cst(S.cent)[3 * ic + q];
+    wt = pw[2 * t + 1];
+  } else {
+    const int kp = t - npt;
+    i = plist[kp] / M;
+    xn[0] = x[3 * i]; xn[1] = x[3 * i + 1]; xn[2] = x[3 * i + 2];
+    wt = 0.0;
+    for (int iq = 0; iq < nq; iq++) wt -= pw[2 * (kp * nq + iq) + 1];
   }
 }
 
-// The (electron, centre) pairs plist[kp] taken by this lane, whole: the
-// weighted basis sums (pbc rows) and the slot pieces of dpe (dpe_raw rows)
-// over the pair's quadrature points.  rnew: 4M doubles, uq: N values of the
-// kernel's T, uqd: N doubles of per-lane scratch (LDS or global), stored
-// lane-interleaved.
-template <typename T, int G, int ORD>
-__device__ __forceinline__ void deriv_nlpp_pairs(const KArgs &A, const double *ws, double *ss, int npair,
-                                                 const int *plist, LaneArr<double> rnew, LaneArr<T> uq,
-                                                 LaneArr<double> uqd, int lane) {
-  const DevSys &S = A.S;
-  const WLayout &L = A.L;
-  const SLayout &SL = A.SL;
-  const DLayout &DL = A.DL;
-  const int N = S.N, M = S.M, NB = S.NB, nsl = S.nslot, nq = S.nquad;
-  const double *x = ws + L.x, *ren = ws + L.r_en, *rven = ws + L.rvec_en, *fso = ws + L.fso;
-  const double *vnl = ss + SL.vnl, *quad = ws + L.quad, *gp = ss + SL.gproj, *btd = ss + DL.btd;
-  const T *bt = reinterpret_cast<const T *>(ss + SL.bt);    // filled by k_full_nlpp
-  double *pbc = ss + DL.pbc, *draw = ss + DL.dpe_raw;
-  const LaneArr<double> rvnew = rnew + M;
-  for (int kp = lane; kp < npair; kp += G) {
-    const int p = plist[kp];
-    double *pbrow = pbc + (int64_t)p * NB;
-    double *drow = draw + (int64_t)p * nsl;
-    const double *v = vnl + p * (QMCW_MAX_LPOT + 1);
-    for (int b = 0; b < NB; b++) pbrow[b] = 0.0;
-    const int i = p / M, ic = p % M, ict = cst(S.iwctype)[ic];
-    const double *gpi = gp + (int64_t)i * NB;
-    const double rei = ren[p];
-    const SlotAcc acc{drow, 1};
-    double fold = fso[i * N + i];
-    for (int jj = 0; jj < N; jj++)
-      if (jj != i) fold += fso[jj < i ? i * N + jj : jj * N + i];
-    double wsum = 0.0;
-    for (int iq = 0; iq < nq; iq++) {
-      const double qx = quad[iq], qy = quad[nq + iq], qz = quad[2 * nq + iq];
-      const double *rv0 = rven + 3 * p;
-      const double costh = (rv0[0] * qx + rv0[1] * qy + rv0[2] * qz) / rei;
-      const double xn[3] = {rei * qx + cst(S.cent)[3 * ic], rei * qy + cst(S.cent)[3 * ic + 1],
-                            rei * qz + cst(S.cent)[3 * ic + 2]};
-      for (int jc = 0; jc < M; jc++) {
-        const double dx = xn[0] - cst(S.cent)[3 * jc], dy = xn[1] - cst(S.cent)[3 * jc + 1],
-                     dz = xn[2] - cst(S.cent)[3 * jc + 2];
-        rvnew[3 * jc] = dx; rvnew[3 * jc + 1] = dy; rvnew[3 * jc + 2] = dz;
-        rnew[jc] = (jc == ic) ? rei : sqrt(dx * dx + dy * dy + dz * dz);
-      }
-      // Jastrow factor and channel sum first, then one pass over the shells
-      // forms both the determinant ratio and the weighted basis sums
-      const double delta = (double)jas_point_val<T, ORD>(S, i, xn, x, rnew, bt, uq) - fold;
-      double vpot = 0.0;
-      for (int l = 1; l <= cst(S.npotd)[ict]; l++)
-        if (l != cst(S.lpotp1)[ict]) vpot += v[l - 1] * legendre_w(l, costh);
-      const double fac = cst(S.q0)[3 * nq + iq] * exp(delta) * vpot;
-      double rat = 0.0;
-      for (int sh = 0; sh < S.nshell; sh++) {
-        const int jc = cst(S.sh_cent)[sh];
-        shell_val_axpy<T>(S, sh, (T)rvnew[3 * jc], (T)rvnew[3 * jc + 1], (T)rvnew[3 * jc + 2],
-                          (T)rnew[jc], gpi, fac, pbrow, rat);
-      }
-      const double wr = fac * rat;
-      wsum += wr;
-      en_slots<false>(S, rnew, rvnew, wr, acc);
-      point_pair_slots<ORD>(S, i, xn, x, rnew, btd, uqd, wr, acc);
-    }
-    // the same terms at the current position, weighted by the summed weight
-    en_slots<false>(S, ren + i * M, rven + i * M * 3, -wsum, acc);
-    point_pair_slots<ORD>(S, i, x + 3 * i, x, ren + i * M, btd, uqd, -wsum, acc);
-  }
+constexpr int kPhiCols = 32;       // basis functions per pass of k_deriv_nlpp's weighted sums
+// LDS bytes of its tile: kPhiCols values (one column of padding) and the
+// factor and electron of each of the block's 64 points
+template <typename T>
+__host__ __device__ constexpr size_t deriv_tile_bytes() {
+  return 64 * ((kPhiCols + 1) * sizeof(T) + sizeof(double) + sizeof(int));
 }
 
 // ---------------------------------------------------------------------------
 // Pseudopotential pieces of the derivatives (qmc/vmc/nonloc.f90:184-197,
-// qmc/fit/deriv_nonloc_pot.f90:59-64): psp_nonloc_orb(i, q) over all
-// orbitals and dpe(p) = sum over quadrature points of
-// w exp(dJ) v P_l (Psi_D ratio) d(dJ)/dp.  Each lane takes whole
-// (electron, centre) pairs and owns their rows; k_full_nlpp has filled the
-// channel values (SLayout::vnl) of the current configuration.
-// psp_nonloc_orb is linear in the orbitals, psp_nonloc_orb(i, q) =
-// sum_b coef(b, q) sum_points fac phi_b(point), so per point only the
-// weighted basis values are accumulated (NB terms) and the contraction with
-// the coefficients runs once per electron; the determinant ratio at a point
-// is sum_b gproj_i[b] phi_b(point).
+// qmc/fit/deriv_nonloc_pot.f90:59-64).  k_full_nlpp has left, per quadrature
+// point of the pairs in range, fac = w exp(dJ) v P_l and fac times the
+// determinant ratio (DLayout::pw).  psp_nonloc_orb is linear in the orbitals,
+// psp_nonloc_orb(i, q) = sum_b coef(b, q) sum_points fac phi_b(point): here the
+// weighted basis sums pbc[i][b] (the contraction runs once per electron,
+// k_pnl_mfma).  A lane evaluates the basis functions of its point into LDS, a
+// group of shells at a time, then the lanes take a function each and add its
+// values over the points.  dpe_slot[slot] = sum over points of fac ratio
+// d(dJ)/dslot: a point's slot pieces, weighted, less the same pieces at the
+// electron's current position; summed over the other electrons, the term
+// values of a centre are A^(l+m) S(k, m) + A^m S(k, l+m) with
+// S(k, n) = sum_j U_j^k B_j^n.
 template <typename T, int G, int ORD>
 __global__ QMCW_HEAVY void k_deriv_nlpp(KArgs A) {
   QMCW_GROUP_SETUP
-  const int N = S.N, M = S.M, NO = S.NO, NB = S.NB, nsl = S.nslot;
+  const int N = S.N, M = S.M, NO = S.NO, NB = S.NB, nq = S.nquad;
   const WLayout &L = A.L;
   const SLayout &SL = A.SL;
   const DLayout &DL = A.DL;
-  const double *ren = ws + L.r_en;
-  const double *vnl = ss + SL.vnl;
-  double *pbc = ss + DL.pbc, *draw = ss + DL.dpe_raw;
-  double *btd = ss + DL.btd;
+  const double *x = ws + L.x, *ren = ws + L.r_en;
+  const double *pw = ss + DL.pw;
+  double *pbc = ss + DL.pbc, *btd = ss + DL.tb, *dsl = ss + DL.dpe_slot;
+  const int *plist = reinterpret_cast<const int *>(ss + SL.plist);
+  const int npair = (int)ss[SL.phs + 57], npt = npair * nq;
   for (int p = lane; p < N * M; p += G) {
     double bu, t1, t2;
     scaled<double>(S.isc, S.scalek, ren[p], bu, t1, t2);
-    btd[p] = 1.0 - S.scalek * bu;
-    double *drow = draw + (int64_t)p * nsl;
-    for (int q = 0; q < nsl; q++) drow[q] = 0.0;
+    btd[(p % M) * N + p / M] = 1.0 - S.scalek * bu;
   }
-  // whole pairs in range per lane
-  int *plist = reinterpret_cast<int *>(ss + SL.plist);
-  const int npair = group_compact<G>(vnl + QMCW_MAX_LPOT, QMCW_MAX_LPOT + 1, N * M, plist, lane);
-  __syncthreads();
-  // per-lane distances of the points and e-e-n variables of the other
-  // electrons: LDS when the launch reserved it
-  if (A.lds_dnlpp) {
-    // the block's 64 lanes interleaved: 4M doubles, N values of T, N doubles
-    extern __shared__ double dyn_lds[];
-    const LaneArr<double> rq{dyn_lds + threadIdx.x, kWave};
-    const LaneArr<T> uq{reinterpret_cast<T *>(dyn_lds + 4 * M * kWave) + threadIdx.x, kWave};
-    const LaneArr<double> uqd{dyn_lds + (int64_t)(A.lds_dnlpp - N) * kWave + threadIdx.x, kWave};
-    deriv_nlpp_pairs<T, G, ORD>(A, ws, ss, npair, plist, rq, uq, uqd, lane);
-  } else {
-    // the walker's G lanes interleaved in its scratch
-    const LaneArr<double> rq{ss + SL.qd + lane, G};
-    const LaneArr<T> uq{reinterpret_cast<T *>(ss + SL.uq) + lane, G};
-    const LaneArr<double> uqd{ss + DL.uqd + lane, G};
-    deriv_nlpp_pairs<T, G, ORD>(A, ws, ss, npair, plist, rq, uq, uqd, lane);
+  for (int q = lane; q < N * NB; q += G) pbc[q] = 0.0;
+  // ---- the weighted basis sums
+  extern __shared__ double dyn_lds[];
+  double *s_f = dyn_lds + grp * G;                                  // the group's points
+  int *s_el = reinterpret_cast<int *>(dyn_lds + 64) + grp * G;
+  T *s_phi = reinterpret_cast<T *>(dyn_lds + 96) + (int64_t)grp * G * (kPhiCols + 1);
+  int maxpt = npt;                                                  // of the block's walkers
+#pragma unroll
+  for (int o = G; o < 64; o <<= 1) maxpt = max(maxpt, __shfl_xor(maxpt, o, 64));
+  for (int t0 = 0; t0 < maxpt; t0 += G) {
+    const int nin = max(0, min(G, npt - t0));
+    double xn[3] = {0.0, 0.0, 0.0}, wt;
+    int el = 0;
+    if (lane < nin) nlpp_entry(A, ws, pw, plist, npt, t0 + lane, xn, el, wt);
+    __syncthreads();
+    s_f[lane] = lane < nin ? pw[2 * (t0 + lane)] : 0.0;
+    s_el[lane] = el;
+    // shells of one centre after another, up to kPhiCols functions a pass
+    int ic = 0, sh = 0;
+    while (ic < M) {
+      const int ic_0 = ic, sh_0 = sh;
+      int nf = 0;
+      while (ic < M) {
+        if (sh == cst(S.cent_sh_off)[ic + 1]) { ic++; continue; }
+        const int nm = 2 * cst(S.sh_l)[sh] + 1;
+        if (nf + nm > kPhiCols) break;
+        nf += nm;
+        sh++;
+      }
+      T *ph = s_phi + lane * (kPhiCols + 1);
+      for (int q = sh_0, f = 0, c = ic_0; q < sh; q++) {
+        while (q >= cst(S.cent_sh_off)[c + 1]) c++;
+        const double dx = xn[0] - cst(S.cent)[3 * c], dy = xn[1] - cst(S.cent)[3 * c + 1],
+                     dz = xn[2] - cst(S.cent)[3 * c + 2];
+        shell_slots<T>(S, q, (T)dx, (T)dy, (T)dz, (T)sqrt(dx * dx + dy * dy + dz * dz), ph + f);
+        f += 2 * cst(S.sh_l)[q] + 1;
+      }
+      __syncthreads();
+      for (int f = lane; f < nf; f += G) {
+        // the function of column f
+        int q = sh_0, g = f;
+        while (g > 2 * cst(S.sh_l)[q]) { g -= 2 * cst(S.sh_l)[q] + 1; q++; }
+        const int b = S.sh_bas[q * kMaxShellM + g];
+        if (b < 0) continue;
+        double a = 0.0;
+        int cur = s_el[0];
+        for (int p = 0; p < nin; p++) {
+          if (s_el[p] != cur) {
+            pbc[cur * NB + b] += a;
+            a = 0.0;
+            cur = s_el[p];
+          }
+          a += s_f[p] * (double)s_phi[p * (kPhiCols + 1) + f];
+        }
+        if (nin > 0) pbc[cur * NB + b] += a;
+      }
+      __syncthreads();
+    }
   }
-  __syncthreads();
-  // per-electron basis sums over the centres in range, kept in the row of
-  // centre 0 (each lane reads and writes only its own (i, b) column)
-  for (int t = lane; t < N * NB; t += G) {
-    const int i = t / NB, b = t % NB;
-    double a = 0.0;
-    for (int ic = 0; ic < M; ic++)
-      if (vnl[(i * M + ic) * (QMCW_MAX_LPOT + 1) + QMCW_MAX_LPOT] != 0.0)
-        a += pbc[(int64_t)(i * M + ic) * NB + b];
-    pbc[(int64_t)i * M * NB + b] = a;
+  // ---- the slots: quadrature points and, after them, the pairs at the
+  // electrons' current positions
+  const int nent = npt + npair;
+  const double k = S.scalek, ar = S.asymp_r;
+  constexpr int MW = QMCW_MAX_ORD + 1;
+  const int na = S.norda + 1, nb = S.nordb + 1;
+  for (int isb = 0; isb < (S.nspin2b == 2 ? 2 : 1); isb++) {
+    double av[MW];
+#pragma unroll
+    for (int q = 0; q < MW; q++) av[q] = 0.0;
+    for (int t = lane; t < nent; t += G) {
+      double xn[3], wt;
+      int i;
+      nlpp_entry(A, ws, pw, plist, npt, t, xn, i, wt);
+      for (int j = 0; j < N; j++) {
+        if (j == i) continue;
+        double sp;
+        if (b_spin(S, (i < S.nup) == (j < S.nup), sp) != isb) continue;
+        const double dx = xn[0] - x[3 * j], dy = xn[1] - x[3 * j + 1], dz = xn[2] - x[3 * j + 2];
+        double u, d1, d2;
+        scaled<double>(S.isc, k, sqrt(dx * dx + dy * dy + dz * dz), u, d1, d2);
+        PadeSlots ps(u, cst(S.b)[isb * nb], cst(S.b)[isb * nb + 1], sp, ar);
+#pragma unroll
+        for (int iw = 1; iw <= MW; iw++) {
+          if (iw > nb) continue;
+          double g, g1, g2;
+          ps.get(iw, g, g1, g2);
+          av[iw - 1] += wt * g;
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < MW; q++) {
+      if (q >= nb) continue;
+      const double v = gsum<G>(av[q]);
+      if (lane == 0) dsl[S.slot_b0 + isb * nb + q] = v;
+    }
   }
-  double *dsl = ss + DL.dpe_slot;
-  for (int sl = lane; sl < nsl; sl += G) {
-    double a = 0.0;
-    for (int p = 0; p < N * M; p++) a += draw[(int64_t)p * nsl + sl];
-    dsl[sl] = a;
+  constexpr int NG = een_gi<ORD>(ORD, 0) + 1, NT = een_count<ORD>(-1);
+  const LaneArr<double> uq = A.lds_dnlpp
+      ? LaneArr<double>{dyn_lds + deriv_tile_bytes<T>() / 8 + threadIdx.x, kWave}
+      : LaneArr<double>{ss + DL.uqd + lane, G};
+  for (int it = 0; it < S.nctype; it++) {
+    double av[MW], ac[NT];
+#pragma unroll
+    for (int q = 0; q < MW; q++) av[q] = 0.0;
+#pragma unroll
+    for (int q = 0; q < NT; q++) ac[q] = 0.0;
+    for (int t = lane; t < nent; t += G) {
+      double xn[3], wt;
+      int i;
+      nlpp_entry(A, ws, pw, plist, npt, t, xn, i, wt);
+      if (S.nordc > 1)
+        for (int j = 0; j < N; j++) {
+          const double dx = xn[0] - x[3 * j], dy = xn[1] - x[3 * j + 1], dz = xn[2] - x[3 * j + 2];
+          double u, d1, d2;
+          scaled<double>(S.isc, k, sqrt(dx * dx + dy * dy + dz * dz), u, d1, d2);
+          uq[j] = 1.0 - k * u;
+        }
+      for (int c = cst(S.tc_off)[it]; c < cst(S.tc_off)[it + 1]; c++) {
+        const cptr<TypeCent> tc = (cptr<TypeCent>)S.tcent + c;
+        const double dx = xn[0] - tc->x, dy = xn[1] - tc->y, dz = xn[2] - tc->z;
+        double u, d1, d2;
+        scaled<double>(S.isc, k, sqrt(dx * dx + dy * dy + dz * dz), u, d1, d2);
+        PadeSlots ps(u, cst(S.a4)[it * na], cst(S.a4)[it * na + 1], 1.0, ar);
+#pragma unroll
+        for (int iw = 1; iw <= MW; iw++) {
+          if (iw > na) continue;
+          double g, g1, g2;
+          ps.get(iw, g, g1, g2);
+          av[iw - 1] += wt * g;
+        }
+        if (S.nordc <= 1) continue;
+        double sg[NG];
+#pragma unroll
+        for (int q = 0; q < NG; q++) sg[q] = 0.0;
+        const double *bj = btd + tc->ic * N;
+        for (int j = 0; j < N; j++) {
+          if (j == i) continue;
+          const double U = uq[j], B = bj[j];
+          double uk = 1.0;
+#pragma unroll
+          for (int kk = 0; kk <= ORD; kk++) {
+            double v = uk;
+#pragma unroll
+            for (int n = 0; n <= ORD - kk; n++) {
+              sg[een_gi<ORD>(kk, n)] += v;
+              v *= B;
+            }
+            uk *= U;
+          }
+        }
+        double ap[ORD + 1];
+        ap[0] = wt;
+#pragma unroll
+        for (int q = 1; q <= ORD; q++) ap[q] = ap[q - 1] * (1.0 - k * u);
+        int idx = 0;
+#pragma unroll
+        for (int kk = 0; kk <= ORD; kk++)
+#pragma unroll
+          for (int m = 0; 2 * m <= ORD - kk; m++)
+#pragma unroll
+            for (int l = 0; l <= ORD - kk - 2 * m; l++)
+              if (QMCW_EEN_TERM(kk, l, m)) {
+                ac[idx] += ap[l + m] * sg[een_gi<ORD>(kk, m)] + ap[m] * sg[een_gi<ORD>(kk, l + m)];
+                idx++;
+              }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < MW; q++) {
+      if (q >= na) continue;
+      const double v = gsum<G>(av[q]);
+      if (lane == 0) dsl[it * na + q] = v;
+    }
+    if (S.nordc > 1) {
+#pragma unroll
+      for (int q = 0; q < NT; q++) {
+        const double v = gsum<G>(ac[q]);
+        if (lane == 0) dsl[S.slot_c0 + it * S.nterms + q] = v;
+      }
+    }
   }
-  __syncthreads();
-  double *pnl = ss + DL.pnl;
   // (k_pnl_mfma forms pnl after this kernel when A.pnl_mfma)
-  for (int t = A.pnl_mfma ? N * NO : lane; t < N * NO; t += G) {
+  if (A.pnl_mfma) return;
+  double *pnl = ss + DL.pnl;
+  for (int t = lane; t < N * NO; t += G) {
     const int i = t / NO, q = t % NO;
-    const double *row = pbc + (int64_t)i * M * NB;
     double a = 0.0;
-    for (int b = 0; b < NB; b++) a += cst(S.coefT)[(int64_t)b * NO + q] * row[b];
+    for (int b = 0; b < NB; b++) a += cst(S.coefT)[(int64_t)b * NO + q] * pbc[i * NB + b];
     pnl[t] = a;
-  }
-  double *dpe = ss + DL.dpe;
-  for (int p = lane; p < S.npj; p += G) {
-    double a = 0.0;
-    for (int q = cst(S.pj_off)[p]; q < cst(S.pj_off)[p + 1]; q++) a += cst(S.pj_w)[q] * dsl[cst(S.pj_slot)[q]];
-    dpe[p] = a;
   }
 }
 
@@ -531,7 +546,18 @@ __global__ QMCW_HEAVY void k_deriv_nlpp(KArgs A) {
 // (qmc/deriv_fast_mod.f90:174-823), dpsi_orb_bld / deloc_orb_bld
 // (qmc/deriv_orb_mod.f90:1486-1630) and the Jastrow denergy of
 // qmc/vmc/hpsi.f90:366-374.  out[w * 2P + p] = dpsi, out[w * 2P + P + p] = deloc.
-template <int G>
+// With LDS the intermediates (derivs_lds_doubles of them) stay in LDS, a
+// wavefront per walker: each of the dozen dependent phases then waits for LDS
+// instead of L2, which bounded the kernel (37 of 600 VALU instructions per
+// SIMD and us): 469 -> 246 us for 8,192 C2-like walkers.
+__host__ __device__ inline int derivs_lds_doubles(const DevSys &S) {
+  const int nsm = S.ns[0] > S.ns[1] ? S.ns[0] : S.ns[1], nom = S.nocc[0] > S.nocc[1] ? S.nocc[0] : S.nocc[1];
+  int n = (2 * S.N + nsm) * S.NO + nom * nsm;
+  for (int s = 0; s < 2; s++)
+    n += 2 * S.ns[s] * S.NO + S.ndetu[s] * (3 + S.kmax2) + 2 * S.nocc[s] * S.ns[s];
+  return n;
+}
+template <int G, bool LDS>
 __global__ QMCW_HEAVY void k_derivs(KArgs A, double *out) {
   QMCW_GROUP_SETUP
   const int N = S.N, NO = S.NO, P = S.nparm;
@@ -542,7 +568,29 @@ __global__ QMCW_HEAVY void k_derivs(KArgs A, double *out) {
   const double *orb = ss + SL.orb;
   const double *vj = ss + SL.vj, *vd = ss + SL.vd, *red = ss + SL.phs;
   const double *pnl = ss + DL.pnl;
-  double *B = ss + DL.B;
+  // the orbital values (component 0 of orb, or their copy in LDS)
+  extern __shared__ double dyn_lds[];
+  constexpr int OS = LDS ? 1 : 5;
+  double *nxt = dyn_lds + (LDS ? N * NO : 0);
+  auto part = [&](int64_t at, int n) {
+    if (!LDS) return ss + at;
+    double *p = nxt;
+    nxt += n;
+    return p;
+  };
+  const double *ob = LDS ? dyn_lds : orb;
+  double *B = part(DL.B, N * NO), *tfs[2], *dts[2], *dels[2], *c0s[2], *c1s[2], *ids[2], *dys[2], *dgs[2];
+  for (int s = 0; s < 2; s++) {
+    tfs[s] = part(DL.tfull[s], S.ns[s] * NO);
+    dts[s] = part(DL.dt[s], S.ns[s] * NO);
+    dels[s] = part(DL.del[s], S.ndetu[s]);
+    c0s[s] = part(DL.c0[s], S.ndetu[s]);
+    c1s[s] = part(DL.c1[s], S.ndetu[s]);
+    ids[s] = part(DL.idti[s], S.ndetu[s] * S.kmax2);
+    dys[s] = part(DL.dy[s], S.nocc[s] * S.ns[s]);
+    dgs[s] = part(DL.dg[s], S.nocc[s] * S.ns[s]);
+  }
+  double *aib = part(DL.aib, max(S.ns[0], S.ns[1]) * NO), *aux = part(DL.aux4, 0);
   const double vpsp = S.nloc > 0 ? red[56] : 0.0;
   const double epl = ws[L.epot] - vpsp;          // local part of the potential
   double vj2 = 0.0;
@@ -557,6 +605,7 @@ __global__ QMCW_HEAVY void k_derivs(KArgs A, double *out) {
     double b = -hb * (o[4] + 2.0 * dv + ddjas * o[0]) + epl * o[0] / N;
     if (S.nloc > 0) b += pnl[t];
     B[t] = b;
+    if (LDS) dyn_lds[t] = o[0];
   }
   __syncthreads();
   // ---- full T, dt_bld, alpha_deloc_bld and the k x k inverse products
@@ -564,13 +613,13 @@ __global__ QMCW_HEAVY void k_derivs(KArgs A, double *out) {
     const int ns = S.ns[s], off = s ? S.nup : 0;
     if (ns == 0) continue;
     const double *ai = w_ai(L, ws, s);
-    double *tf = ss + DL.tfull[s], *dt = ss + DL.dt[s], *aib = ss + DL.aib;
+    double *tf = tfs[s], *dt = dts[s];
     for (int e = lane; e < ns * NO; e += G) {
       const int k = e / NO, q = e % NO;
       double a1 = 0.0, a2 = 0.0;
       for (int i = 0; i < ns; i++) {
         const double aki = ai[k + ns * i];
-        a1 += aki * orb[((int64_t)(off + i) * NO + q) * 5];
+        a1 += aki * ob[((int64_t)(off + i) * NO + q) * OS];
         a2 += aki * B[(off + i) * NO + q];
       }
       tf[e] = a1;
@@ -585,7 +634,7 @@ __global__ QMCW_HEAVY void k_derivs(KArgs A, double *out) {
     }
     __syncthreads();
     const double *inv = w_inv(L, ws, s);
-    double *del = ss + DL.del[s], *idti = ss + DL.idti[s];
+    double *del = dels[s], *idti = ids[s];
     for (int u = lane; u < S.ndetu[s]; u += G) {
       const int k = cst(S.ord[s])[u];
       const double *iv = inv + u * S.kmax2;
@@ -612,7 +661,7 @@ __global__ QMCW_HEAVY void k_derivs(KArgs A, double *out) {
   // ---- coefficient sums per unique det and esum
   const double chii = 1.0 / ws[L.chi];
   const double *dv0 = w_detv(L, ws, 0), *dv1 = w_detv(L, ws, 1);
-  const double *del0 = ss + DL.del[0], *del1 = ss + DL.del[1];
+  const double *del0 = dels[0], *del1 = dels[1];
   // over the dets that contain unique det u (the CSR lists of eval_y, in
   // ascending det order)
   for (int t = lane; t < S.ndetu[0] + S.ndetu[1]; t += G) {
@@ -628,13 +677,13 @@ __global__ QMCW_HEAVY void k_derivs(KArgs A, double *out) {
       c0 += cf;
       c1 += cf * ((S.ns[0] ? del0[iu] : 0.0) + (S.ns[1] ? del1[id] : 0.0));
     }
-    (ss + DL.c0[s])[u] = c0;
-    (ss + DL.c1[s])[u] = c1;
+    c0s[s][u] = c0;
+    c1s[s][u] = c1;
   }
   double es = 0.0;
   for (int s = 0; s < 2; s++) {
     const int ns = S.ns[s], nocc = S.nocc[s];
-    const double *y = w_y(L, ws, s), *dt = ss + DL.dt[s];
+    const double *y = w_y(L, ws, s), *dt = dts[s];
     for (int e = lane; e < nocc * ns; e += G) {
       const int j = e / ns, i = e % ns;
       es += y[e] * dt[i * NO + cst(S.occ[s])[j]];
@@ -645,9 +694,9 @@ __global__ QMCW_HEAVY void k_derivs(KArgs A, double *out) {
   // ---- dy_bld
   for (int s = 0; s < 2; s++) {
     const int ns = S.ns[s], nocc = S.nocc[s];
-    const double *inv = w_inv(L, ws, s), *idti = ss + DL.idti[s], *y = w_y(L, ws, s);
-    const double *c0 = ss + DL.c0[s], *c1 = ss + DL.c1[s];
-    double *dy = ss + DL.dy[s];
+    const double *inv = w_inv(L, ws, s), *idti = ids[s], *y = w_y(L, ws, s);
+    const double *c0 = c0s[s], *c1 = c1s[s];
+    double *dy = dys[s];
     // contributions to entry e (the Y-entry CSR lists of eval_y, ascending u)
     const cptr<int> yoff = cst(S.yent_off[s]), yu = cst(S.yent_u[s]), yp = cst(S.yent_pos[s]);
     for (int e = lane; e < nocc * ns; e += G) {
@@ -666,9 +715,9 @@ __global__ QMCW_HEAVY void k_derivs(KArgs A, double *out) {
   for (int s = 0; s < 2; s++) {
     const int ns = S.ns[s], nocc = S.nocc[s], off = s ? S.nup : 0;
     if (ns == 0) continue;
-    const double *tf = ss + DL.tfull[s], *dt = ss + DL.dt[s], *dy = ss + DL.dy[s];
+    const double *tf = tfs[s], *dt = dts[s], *dy = dys[s];
     const double *y = w_y(L, ws, s), *g = ss + SL.g[s], *ai = w_ai(L, ws, s);
-    double *aux = ss + DL.aux4, *dg = ss + DL.dg[s];
+    double *dg = dgs[s];
     for (int e = lane; e < nocc * ns; e += G) aux[e] = 0.0;
     __syncthreads();
     for (int e = lane; e < ns * ns; e += G) {
@@ -712,13 +761,18 @@ __global__ QMCW_HEAVY void k_derivs(KArgs A, double *out) {
     o1[ip] = dd;
     o2[ip] = de;
   }
-  const double *gv = ss + DL.gvalue, *gj = ss + DL.gjas, *d2g = ss + DL.d2g, *dpe = ss + DL.dpe;
+  // the Jastrow's parameters from their slots (k_deriv_jas, and the
+  // pseudopotential's part from k_deriv_nlpp)
+  const double *dj = ss + DL.dj, *dsl = ss + DL.dpe_slot;
   for (int ip = lane; ip < S.npj; ip += G) {
-    double de = -hb * d2g[ip] + (S.nloc > 0 ? dpe[ip] : 0.0);
-    for (int i = 0; i < N; i++)
-      for (int k = 0; k < 3; k++)
-        de -= 2.0 * hb * gj[(ip * N + i) * 3 + k] * (vj[3 * i + k] + vd[3 * i + k]);
-    o1[S.npcsf + ip] = gv[ip];
+    double dv = 0.0, de = 0.0;
+    for (int q = cst(S.pj_off)[ip]; q < cst(S.pj_off)[ip + 1]; q++) {
+      const int sl = S.pj_slot[q];
+      const double w = S.pj_w[q];
+      dv += w * dj[2 * sl];
+      de += w * (dj[2 * sl + 1] + (S.nloc > 0 ? dsl[sl] : 0.0));
+    }
+    o1[S.npcsf + ip] = dv;
     o2[S.npcsf + ip] = de;
   }
   for (int ip = lane; ip < S.nporb; ip += G) {
@@ -731,11 +785,11 @@ __global__ QMCW_HEAVY void k_derivs(KArgs A, double *out) {
         const int ns = S.ns[s], off = s ? S.nup : 0;
         const int pa = cst(S.iocc_lab[s])[a];
         if (ns == 0 || pa < 0) continue;
-        const double *g = ss + SL.g[s], *dg = ss + DL.dg[s];
+        const double *g = ss + SL.g[s], *dg = dgs[s];
         for (int k = 0; k < ns; k++) {
-          const double ob = orb[((int64_t)(off + k) * NO + b) * 5];
-          dp += sg * g[pa * ns + k] * ob;
-          de += sg * (g[pa * ns + k] * B[(off + k) * NO + b] + dg[pa * ns + k] * ob);
+          const double o = ob[((int64_t)(off + k) * NO + b) * OS];
+          dp += sg * g[pa * ns + k] * o;
+          de += sg * (g[pa * ns + k] * B[(off + k) * NO + b] + dg[pa * ns + k] * o);
         }
       }
     }

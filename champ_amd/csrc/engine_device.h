@@ -1236,31 +1236,17 @@ __device__ __forceinline__ double point_ratio(const DevSys &S, const double *xn,
   return rd;
 }
 
-// Values of shell s's basis functions at (x, y, z), r, accumulated in FP64:
-// rat += sum gp[b] phi_b and pb[b] += fac phi_b (the pseudopotential's
-// determinant ratio and weighted basis sums in one pass, no stored values).
+// Values of shell s's basis functions at (x, y, z), distance r, into
+// ph[0..2l] (slot order m = 0, 1, -1, 2, -2, ...).
 template <typename T, int L>
-__device__ __forceinline__ void shell_axpy_l(T x, T y, T z, T g, cptr<int> bas, const double *gp,
-                                             double fac, double *pb, double &rat) {
+__device__ __forceinline__ void shell_slots_l(T x, T y, T z, T g, T *ph) {
   T Sv[2 * L + 1], Sg[2 * L + 1][3];
   solid_harm<T>(L, x, y, z, Sv, Sg);
-  // the shell's sums first (its components are distinct), then the stores
-  double old[2 * L + 1];
 #pragma unroll
-  for (int q = 0; q < 2 * L + 1; q++) old[q] = bas[q] >= 0 ? pb[bas[q]] : 0.0;
-#pragma unroll
-  for (int q = 0; q < 2 * L + 1; q++) {
-    const int b = bas[q];
-    if (b >= 0) {
-      const double v = (double)(Sv[q] * g);
-      rat += gp[b] * v;
-      pb[b] = old[q] + fac * v;
-    }
-  }
+  for (int q = 0; q < 2 * L + 1; q++) ph[q] = Sv[q] * g;
 }
 template <typename T>
-__device__ __forceinline__ void shell_val_axpy(const DevSys &S, int s, T x, T y, T z, T r,
-                                               const double *gp, double fac, double *pb, double &rat) {
+__device__ __forceinline__ void shell_slots(const DevSys &S, int s, T x, T y, T z, T r, T *ph) {
   const int l = cst(S.sh_l)[s], a = cst(S.sh_a)[s];
   const bool gauss = (S.basis_type == QMCW_BASIS_GAUSSIAN);
   T g = 0;
@@ -1268,21 +1254,20 @@ __device__ __forceinline__ void shell_val_axpy(const DevSys &S, int s, T x, T y,
   if (kn >= 0) {
     g = num_radial_f<T>(S, kn, l, r);
   } else {
-    const cptr<double> pz = cst(S.prim_zeta), pc = cst(S.prim_coef);
+    const cptr<double> tp = cst(S.tprim);
     for (int p = cst(S.sh_prim_off)[s]; p < cst(S.sh_prim_off)[s + 1]; p++) {
-      const T zeta = T(pz[p]), d = T(pc[p]);
+      const T zeta = T(tp[2 * p]), d = T(tp[2 * p + 1]);
       g += d * exp(gauss ? -zeta * r * r : -zeta * r);
     }
     for (int q = 0; q < a; q++) g *= r;
   }
-  const cptr<int> bas = cst(S.sh_bas) + s * kMaxShellM;
   switch (l) {
-    case 0: shell_axpy_l<T, 0>(x, y, z, g, bas, gp, fac, pb, rat); break;
-    case 1: shell_axpy_l<T, 1>(x, y, z, g, bas, gp, fac, pb, rat); break;
-    case 2: shell_axpy_l<T, 2>(x, y, z, g, bas, gp, fac, pb, rat); break;
-    case 3: shell_axpy_l<T, 3>(x, y, z, g, bas, gp, fac, pb, rat); break;
-    case 4: shell_axpy_l<T, 4>(x, y, z, g, bas, gp, fac, pb, rat); break;
-    default: shell_axpy_l<T, 5>(x, y, z, g, bas, gp, fac, pb, rat); break;
+    case 0: shell_slots_l<T, 0>(x, y, z, g, ph); break;
+    case 1: shell_slots_l<T, 1>(x, y, z, g, ph); break;
+    case 2: shell_slots_l<T, 2>(x, y, z, g, ph); break;
+    case 3: shell_slots_l<T, 3>(x, y, z, g, ph); break;
+    case 4: shell_slots_l<T, 4>(x, y, z, g, ph); break;
+    default: shell_slots_l<T, 5>(x, y, z, g, ph); break;
   }
 }
 

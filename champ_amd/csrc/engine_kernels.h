@@ -32,7 +32,7 @@ struct KArgs {
   int lds_y;         // doubles per group of the LDS staging of eval_y in the move kernels (0: none)
   int lds_y_off;     // its offset (doubles) in the dynamic LDS, after the basis values
   int lds_nlpp;      // doubles per lane of k_full_nlpp's point scratch in LDS (0: global)
-  int lds_dnlpp;     // doubles per lane of k_deriv_nlpp's point scratch in LDS (0: global)
+  int lds_dnlpp;     // values of U per lane of k_deriv_nlpp in LDS (0: in global scratch)
   int nlpp_tiles;    // wavefronts per walker of k_full_nlpp_tiles (0: k_full_nlpp)
   int bf16;          // orbital-contraction inputs rounded to bfloat16
   int chunk;         // electrons per basis chunk in the full evaluation
@@ -507,7 +507,8 @@ __device__ void group_g(const DevSys &S, int s, const double *ai,
 // determinants; pseudopotential; local energy) so that each carries fewer
 // live registers; scalars pass through the walker's reduction scratch:
 // phs[50] pe_en, [51] pe_ee, [52] ln J, [53] lap ln J, [54] lap ln D,
-// [55] local pseudopotential, [56] nonlocal pseudopotential (SLayout::phs).
+// [55] local pseudopotential, [56] nonlocal pseudopotential, [57] pairs in
+// range (SLayout::phs).
 template <typename T, int G, int ORD>
 __device__ __forceinline__ void full_jas_b(const KArgs &A, int bid_) {
   QMCW_GROUP_SETUP_B(bid_)
@@ -914,13 +915,12 @@ __global__ __launch_bounds__(64) void k_orb_mfma(KArgs A, int nw) {
 // psp_nonloc_orb of the derivatives on FP64 MFMA: pnl[i][q] = sum_b
 // coef(b, q) pbc_i[b] for every walker w < nw and electron i, one GEMM
 // [nw*N x NB] x [NB x NO] with rows = (walker, electron) pairs in walker
-// order (pbc_i: the electron's weighted basis sums, in the row of centre 0
-// of its pairs) and the coefficients shared by every walker; block
-// blockIdx.x takes 64 rows and blockIdx.y 64 orbitals, in the tiles of
-// k_gproj_mfma.
+// order (pbc_i: the electron's weighted basis sums) and the coefficients
+// shared by every walker; block blockIdx.x takes 64 rows and blockIdx.y 64
+// orbitals, in the tiles of k_gproj_mfma.
 __global__ __launch_bounds__(64) void k_pnl_mfma(KArgs A, int nw) {
   const DevSys &S = A.S;
-  const int N = S.N, M = S.M, NB = S.NB, NO = S.NO;
+  const int N = S.N, NB = S.NB, NO = S.NO;
   const int64_t rows = (int64_t)nw * N, row0 = (int64_t)blockIdx.x * 64;
   if (row0 >= rows) return;
   const int64_t stride = A.SL.stride;
@@ -934,7 +934,7 @@ __global__ __launch_bounds__(64) void k_pnl_mfma(KArgs A, int nw) {
     const int64_t rho = row0 + 16 * t + r;
     va[t] = rho < rows;
     const int64_t w = va[t] ? rho / N : 0, i = va[t] ? rho % N : 0;
-    ga[t] = A.sc + w * stride + A.DL.pbc + i * M * NB;
+    ga[t] = A.sc + w * stride + A.DL.pbc + i * NB;
   }
   gp_d4 acc[4][4];
 #pragma unroll
@@ -1024,7 +1024,7 @@ __device__ __forceinline__ void rot_axes(int *st4, double *ax) {
 // doubles and uq: N values of per-lane scratch (LDS or global), stored
 // lane-interleaved.
 template <typename T, int G, int ORD, bool PAIR>
-__device__ __forceinline__ double nlpp_points(const KArgs &A, const double *ws, const double *ss,
+__device__ __forceinline__ double nlpp_points(const KArgs &A, const double *ws, double *ss,
                                               int npair, const int *plist, LaneArr<double> rnew,
                                               LaneArr<T> uq, double *tqw, int lane) {
   const DevSys &S = A.S;
@@ -1081,7 +1081,13 @@ __device__ __forceinline__ double nlpp_points(const KArgs &A, const double *ws, 
     double vpot = 0.0;
     for (int l = 1; l <= cst(S.npotd)[ict]; l++)
       if (l != cst(S.lpotp1)[ict]) vpot += v[l - 1] * legendre_w(l, costh);
-    vpsp += cst(S.q0)[3 * nq + iq] * exp(delta) * vpot * rd;
+    const double fac = cst(S.q0)[3 * nq + iq] * exp(delta) * vpot;
+    vpsp += fac * rd;
+    if (A.full_orb) {      // for k_deriv_nlpp
+      double *pw = ss + A.DL.pw + 2 * t;
+      pw[0] = fac;
+      pw[1] = fac * rd;
+    }
     if (tqw) {
       // kept for T-moves: the point and the Psi ratio there (rank j of the
       // pair among electron i's pairs in range)
@@ -1113,7 +1119,7 @@ __device__ __forceinline__ void full_nlpp_b(const KArgs &A, int bid_) {
   // V_nl = sum_G psp_nonloc_orb is linear in the orbitals, so per quadrature
   // point only the determinant ratio sum_j G(j,i) phi_occj = sum_b gp_i[b]
   // phi_b is needed, with gp_i = G(:,i)^T coef_occ formed once per electron.
-  double vpsp = 0.0, ploc = 0.0;
+  double vpsp = 0.0, ploc = 0.0, npairs = 0.0;
   if (S.nloc > 0) {
     double *vnl = ss + SL.vnl;        // [N*M][QMCW_MAX_LPOT + 1] (last: in range)
     T *bt = reinterpret_cast<T *>(ss + SL.bt);
@@ -1158,6 +1164,7 @@ __device__ __forceinline__ void full_nlpp_b(const KArgs &A, int bid_) {
     // quadrature points only of the pairs in range, spread evenly over the lanes
     int *plist = reinterpret_cast<int *>(ss + SL.plist);
     const int npair = group_compact<G>(vnl + QMCW_MAX_LPOT, QMCW_MAX_LPOT + 1, N * M, plist, lane);
+    npairs = npair;
     // DMC (qmc/vmc/nonloc.f90:89): every pair in range rotates the grid anew,
     // drawing from the walker's stream in pair order.  rotqua's rejection
     // loops make the number of draws vary, so one lane walks the stream and
@@ -1201,7 +1208,7 @@ __device__ __forceinline__ void full_nlpp_b(const KArgs &A, int bid_) {
     }
     vpsp = gsum<G>(vpsp);
   }
-  if (lane == 0) { red[55] = ploc; red[56] = vpsp; }
+  if (lane == 0) { red[55] = ploc; red[56] = vpsp; red[57] = npairs; }
 }
 // FP32 instances are held to 128 VGPRs (four waves per SIMD); PAIR: the
 // point Jastrow two centres at a time (systems of many centres)

@@ -255,7 +255,6 @@ __device__ __forceinline__ void full_nlpp_tiles_b(const KArgs &A, int w) {
 #pragma unroll
         for (int l = 0; l < QMCW_MAX_LPOT; l++) v[l] = vl[l];
       }
-      if (A.full_orb) v[QMCW_MAX_LPOT] = inr ? 1.0 : 0.0;   // k_deriv_nlpp reads the flags
       T bu, t1, t2;
       scaled<T>(S.isc, (T)S.scalek, (T)ren[p], bu, t1, t2);
       bt[ic * N + p / M] = T(1) - (T)S.scalek * bu;
@@ -363,7 +362,13 @@ __device__ __forceinline__ void full_nlpp_tiles_b(const KArgs &A, int w) {
       for (int l = 1; l <= cst(S.npotd)[ict]; l++)
         if (l != cst(S.lpotp1)[ict]) vpot += v[l - 1] * legendre_w(l, costh);
       const double ej = exp(delta);
-      vpsp += cst(S.q0)[3 * nq + iq] * ej * vpot * rd;
+      const double fac = cst(S.q0)[3 * nq + iq] * ej * vpot;
+      vpsp += fac * rd;
+      if (A.full_orb) {      // for k_deriv_nlpp
+        double *pw = ss + A.DL.pw + 2 * t;
+        pw[0] = fac;
+        pw[1] = fac * rd;
+      }
       if (tqw) {
         const int j = (int)prot[10 * (t / nq) + 9];
         if (j >= 0) {
@@ -384,6 +389,7 @@ __device__ __forceinline__ void full_nlpp_tiles_b(const KArgs &A, int w) {
     double *red = ss + SL.phs;
     red[55] = a;
     red[56] = b;
+    red[57] = npair;
   }
 }
 
