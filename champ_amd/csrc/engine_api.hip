@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "engine_derivs.h"
+#include "engine_det_small.h"
 #include "engine_accum.h"
 #include "engine_dmc.h"
 #include "engine_launch.h"
@@ -96,6 +97,7 @@ struct qmcw_handle {
   int npow2 = 1;
   int host_split_join = 0;    // QMCW_HOST_SPLIT_JOIN=1: split_join on the host
   int no_gproj_mfma = 0;      // QMCW_NO_GPROJ_MFMA=1: the projection on VALU in k_full_det
+  int no_det_small = 0;       // QMCW_NO_DET_SMALL=1: small determinants in k_full_det as well
   int no_een_tab = 0;         // QMCW_NO_EEN_TAB=1: the move's e-e-n terms summed per pair
   int nlpp_waves = -1;        // the autotuner's choice for k_full_nlpp_tiles (-1: the rule)
   int nlpp_tiles_env = -1;    // QMCW_NLPP_TILES: wavefronts per walker of k_full_nlpp_tiles (0: never used)
@@ -536,6 +538,11 @@ static void launch_det(qmcw_handle *h, const KArgs &A, size_t smem) {
     hipLaunchKernelGGL((k_full_det<float, G>), grid, block, smem, h->stream, A);
 }
 template <int G>
+static void launch_det_small(qmcw_handle *h, const KArgs &A, size_t smem) {
+  const dim3 grid(h->Wl / (kWave / G)), block(kWave);
+  hipLaunchKernelGGL((k_det_small<G>), grid, block, smem, h->stream, A);
+}
+template <int G>
 static void launch_fin(qmcw_handle *h, const KArgs &A) {
   const dim3 grid(h->Wl / (kWave / G)), block(kWave);
   hipLaunchKernelGGL((k_full_fin<G>), grid, block, 0, h->stream, A);
@@ -596,6 +603,18 @@ static int nlpp_tile_waves(const qmcw_handle *h) {
   int nw = 1;
   while (nw < kNlppWaves && (int64_t)h->Wl * nw < 8 * (int64_t)h->ncu) nw *= 2;
   return nw;
+}
+
+// LDS of a block of k_det_small at lane-group width G, 0 where k_full_det
+// does the determinants: spins it stages itself (16 electrons and more), or
+// more LDS than leaves four blocks to a compute unit.  k_full_det ->
+// k_det_small, us: 165 -> 70 (8 electrons, 16,384 walkers), 68 -> 32 (4,096),
+// 16 -> 8.7 (4 electrons, 1,024)
+static size_t det_small_lds(const qmcw_handle *h, int G) {
+  const DevSys &S = h->A.S;
+  if (!h->use_lds || h->no_det_small || std::max(S.ns[0], S.ns[1]) > kDetSmallNs) return 0;
+  const size_t b = (size_t)(kWave / G) * det_small_doubles(S) * sizeof(double);
+  return b <= 40 * 1024 ? b : 0;
 }
 
 // The arguments of the full evaluation's kernels for the handle's current
@@ -691,7 +710,17 @@ static void launch_eval(qmcw_handle *h, bool derivs) {
   K.full_jas(cj);
   prof_end(h);
   prof_begin(h, QMCW_PROF_FULL_DET);
-  DISPATCH_GW(gd, launch_det, h, A, det_smem);
+  const size_t small = det_small_lds(h, gd);
+  if (small) {
+    if (!A.keep_state || A.full_orb) {       // the orbitals' rows first
+      KArgs B = A;
+      B.orb_only = 1;
+      DISPATCH_GW(gd, launch_det, h, B, det_smem);
+    }
+    DISPATCH_GW(gd, launch_det_small, h, A, small);
+  } else {
+    DISPATCH_GW(gd, launch_det, h, A, det_smem);
+  }
   if (A.orb_mfma)
     hipLaunchKernelGGL(k_orb_mfma,
                        dim3((unsigned)(((int64_t)h->Wl * A.S.N * 5 + 63) / 64), (A.S.NO + 63) / 64),
@@ -1310,6 +1339,7 @@ extern "C" int qmcw_create(const qmcw_system *s, int32_t nwalk, int32_t precisio
   if (const char *e = getenv("QMCW_HOST_SPLIT_JOIN")) h->host_split_join = atoi(e) != 0;
   if (const char *e = getenv("QMCW_NO_GPROJ_MFMA")) h->no_gproj_mfma = atoi(e) != 0;
   if (const char *e = getenv("QMCW_NO_EEN_TAB")) h->no_een_tab = atoi(e) != 0;
+  if (const char *e = getenv("QMCW_NO_DET_SMALL")) h->no_det_small = atoi(e) != 0;
   if (const char *e = getenv("QMCW_NLPP_TILES")) h->nlpp_tiles_env = std::max(0, atoi(e));
   {
     int dev = 0, n = 0;
@@ -1592,7 +1622,10 @@ static void launch_reinvert(qmcw_handle *h) {
   size_t smem = 0;
   det_lds_inv(h, A, smem);
   prof_begin(h, QMCW_PROF_FULL_DET);
-  DISPATCH_GW(h->Gk[KC_DET], launch_det, h, A, smem);
+  if (const size_t small = det_small_lds(h, h->Gk[KC_DET]))
+    DISPATCH_GW(h->Gk[KC_DET], launch_det_small, h, A, small)
+  else
+    DISPATCH_GW(h->Gk[KC_DET], launch_det, h, A, smem);
   prof_end(h);
   h->moves_since_inv = 0;
 }

@@ -13,9 +13,9 @@ namespace qmcw {
 // pseudopotential's (k_deriv_nlpp).  Both keep the sums of a slot group in
 // registers over a lane's whole share and add the lanes up at the end; an
 // update in memory per (pair, centre, slot) took 640 and 1,090 us of a
-// derivative evaluation of 8,192 C2-like walkers (here 130 and 489), and 1,138
-// and 2,589 of one of 601 walkers of a 25-electron molecule, whose call went
-// from 5.3 to 2.5 ms.
+// derivative evaluation of 8,192 C2-like walkers (here 60 and 488), and 1,138
+// and 2,589 of one of 601 walkers of a 25-electron molecule (the latter here
+// 785), whose call went from 5.3 to 2.5 ms.
 
 // number of e-e-n terms with power k of U (all of them: k = -1)
 template <int ORD>

@@ -25,6 +25,7 @@ struct KArgs {
   int lds_wst;       // T values per walker of that LDS region (at least NB * 5)
   int een_tab;       // k_ratio_1e: the moved electron's e-e-n tables in the same region
                      // during the Jastrow row (een_tables or een_sum_tables)
+  int orb_only;      // k_full_det ends after the orbitals (k_det_small does the determinants)
   int lds_det;       // k_full_det keeps a chunk's basis values in LDS
   int keep_state;    // the full evaluation takes the rows the committed moves kept in the state
                      // (distances, Jastrow pairs and, without full_orb, the orbitals)
@@ -656,6 +657,7 @@ __device__ __forceinline__ void full_det_b(const KArgs &A, int bid_) {
     full_orbitals<T, G>(A, ws, ss, reinterpret_cast<T *>(dyn_lds) + (int64_t)grp * A.chunk * S.NB * 5, lane);
   else
     full_orbitals<T, G>(A, ws, ss, reinterpret_cast<T *>(ss + SL.phi), lane);
+  if (A.orb_only) return;
   __syncthreads();
   // ---- determinants (t_bld, alpha_bld, y_bld, g_bld)
   double *tmp = ss + SL.red;  // >= max(ns^2, nocc*ns) doubles
