@@ -97,6 +97,8 @@ struct qmcw_handle {
   int npow2 = 1;
   int host_split_join = 0;    // QMCW_HOST_SPLIT_JOIN=1: split_join on the host
   int no_gproj_mfma = 0;      // QMCW_NO_GPROJ_MFMA=1: the projection on VALU in k_full_det
+  int no_move_small = 0;      // QMCW_NO_MOVE_SMALL=1: the fused moves keep their pending record in global scratch
+  int tuning = 0;             // the autotuner times the launches of the fused moves
   int no_det_small = 0;       // QMCW_NO_DET_SMALL=1: small determinants in k_full_det as well
   int no_een_tab = 0;         // QMCW_NO_EEN_TAB=1: the move's e-e-n terms summed per pair
   int nlpp_waves = -1;        // the autotuner's choice for k_full_nlpp_tiles (-1: the rule)
@@ -814,10 +816,56 @@ static KArgs move_args(const qmcw_handle *h, int G, bool split, size_t &phi_b, s
   return A;
 }
 
+// The arguments of k_move_small at lane-group width G, or false where the
+// move keeps its pending record in global scratch (k_ratio_1e): more
+// electrons than lanes, widths beyond 16, or a block's record beyond 64 KB.
+// Measured k_ratio_1e -> k_move_small (us per launch, FP64): 4 electrons,
+// 16,384 walkers 39.2 -> 32.0; 8, 16,384: 119.6 -> 82.6; 8, 1,024: 44.3 ->
+// 41.1; 16, 2,048: 42.8 -> 37.7 at 16 lanes; at 64 lanes, whose few walkers per
+// unit wait less and whose records are larger, 38 electrons went from 55.5 to
+// 68.7, so the wide groups keep k_ratio_1e.  The basis values
+// go in one pass where the blocks of the launch still fit the compute units'
+// LDS together, else a few centres at a time in the space the other users of
+// the region need anyway.
+static bool small_move_args(const qmcw_handle *h, int G, KArgs &A, SmallMove &sm, size_t &smem) {
+  const DevSys &S = h->A.S;
+  if (!h->use_lds || h->no_move_small || S.N > G || G > 16) return false;
+  A = h->A;
+  const int ts = h->precision == QMCW_FP64 ? (int)sizeof(double) : (int)sizeof(float);
+  const int ordk = std::max(2, S.nordc);
+  A.een_tab = (S.nordc > 1 && !h->no_een_tab) ? 1 : 0;
+  const int tab = A.een_tab ? S.M * (3 * ((ordk + 1) * (ordk + 2) / 2) + 8) : 0;
+  const size_t bpc = ((size_t)h->Wl / (kWave / G) + h->ncu - 1) / h->ncu;
+  const size_t cap = std::min<size_t>(64 * 1024, (160 * 1024) / std::max<size_t>(1, bpc));
+  small_move_layout(S, S.NB, tab, ts, A.ML, sm);
+  smem = (size_t)(kWave / G) * sm.stride * sizeof(double);
+  if (smem > cap) {
+    const int y = S.single_det ? 0 : y_lds_doubles(S.ndetu[0], S.ndetu[1], S.kmax2);
+    const int room = std::max(y * 8 / (5 * ts), tab / 5);
+    small_move_layout(S, std::min(S.NB, std::max(S.cent_bas_max, room)), tab, ts, A.ML, sm);
+    smem = (size_t)(kWave / G) * sm.stride * sizeof(double);
+  }
+  return smem <= 64 * 1024;
+}
+
 static void launch_ratio(qmcw_handle *h, int ie, int mode, const double *xn, double delta,
                          double fbias, double *out, long long *nacc = nullptr) {
   const int G = h->Gk[KC_MOVE];
   size_t phi_b = 0, smem = 0;
+  if ((mode >= 2 || h->tuning) && !h->split_move) {
+    // decided in this launch (or timed for that): nothing pending is kept
+    KArgs B;
+    SmallMove sm;
+    if (small_move_args(h, G, B, sm, smem)) {
+      LaunchCtx c = make_ctx(h, B, G);
+      c.sm = sm;
+      c.smem_ratio = smem;
+      prof_begin(h, QMCW_PROF_RATIO);
+      ord_kernels(B.S.nordc).move_small(c, ie, mode, xn, delta, fbias, nacc);
+      prof_end(h);
+      return;
+    }
+  }
   const KArgs A = move_args(h, G, h->split_move != 0, phi_b, smem);
   LaunchCtx c = make_ctx(h, A, G);
   c.smem_ratio = smem;
@@ -967,6 +1015,20 @@ extern "C" int qmcw_create(const qmcw_system *s, int32_t nwalk, int32_t precisio
   S.NB = nbas; S.nshell = (int)sh_l.size(); S.maxshell_per_cent = maxsh;
   UP(sh_cent, S.sh_cent); UP(sh_l, S.sh_l); UP(sh_a, S.sh_a); UP(sh_nm, S.sh_nm);
   UP(sh_prim_off, S.sh_prim_off); UP(sh_m, S.sh_m); UP(sh_bas, S.sh_bas);
+  {
+    std::vector<int> cb{0};
+    S.cent_bas_max = 1;
+    for (int ic = 0; ic < s->ncent; ic++) {
+      const int n = s->ctype_bas_off[s->iwctype[ic] + 1] - s->ctype_bas_off[s->iwctype[ic]];
+      cb.push_back(cb.back() + n);
+      S.cent_bas_max = std::max(S.cent_bas_max, n);
+    }
+    UP(cb, S.cent_bas);
+    std::vector<int> byl(sh_l.size());
+    for (size_t q = 0; q < byl.size(); q++) byl[q] = (int)q;
+    std::stable_sort(byl.begin(), byl.end(), [&](int a, int b) { return sh_l[a] < sh_l[b]; });
+    UP(byl, S.sh_by_l);
+  }
   UP(cent_sh_off, S.cent_sh_off); UP(pz, S.prim_zeta); UP(pc, S.prim_coef);
   {
     std::vector<int> tso{0}, tco{0}, cb0(s->ncent, 0);
@@ -1339,6 +1401,7 @@ extern "C" int qmcw_create(const qmcw_system *s, int32_t nwalk, int32_t precisio
   if (const char *e = getenv("QMCW_HOST_SPLIT_JOIN")) h->host_split_join = atoi(e) != 0;
   if (const char *e = getenv("QMCW_NO_GPROJ_MFMA")) h->no_gproj_mfma = atoi(e) != 0;
   if (const char *e = getenv("QMCW_NO_EEN_TAB")) h->no_een_tab = atoi(e) != 0;
+  if (const char *e = getenv("QMCW_NO_MOVE_SMALL")) h->no_move_small = atoi(e) != 0;
   if (const char *e = getenv("QMCW_NO_DET_SMALL")) h->no_det_small = atoi(e) != 0;
   if (const char *e = getenv("QMCW_NLPP_TILES")) h->nlpp_tiles_env = std::max(0, atoi(e));
   {
@@ -2065,6 +2128,11 @@ extern "C" int qmcw_autotune(qmcw_handle *h, int32_t *chosen) {
   double best[4] = {1e30, 1e30, 1e30, 1e30};
   int bestG[4] = {h->Gk[0], h->Gk[1], h->Gk[2], h->Gk[3]};
   int best_split = h->split_move;
+  struct Tuning {            // ends with the call, also on an error
+    qmcw_handle *h;
+    ~Tuning() { h->tuning = 0; }
+  } tuning{h};
+  h->tuning = 1;
   double *xin = h->io + (size_t)h->Wp * 8;
   const int prof_save = h->prof;
   drop_graph(h);

@@ -5,10 +5,9 @@
 // in the walker's record in global memory, about sixty dependent passes over
 // matrices of a few dozen values: each pass waited for a store to reach L2
 // and come back (85% of the 164 us of 16,384 C2-like walkers, mixed; 70 us
-// here).  Now
-// the orbital values are read once, both spins are worked on side by side (half
-// of the walker's lanes each), every pass exchanges values through LDS, and
-// the results go out once.  The operations and their order are
+// here).  Now the orbital values are read once, both spins are worked on side
+// by side (half of the walker's lanes each), every pass exchanges values
+// through LDS, and the results go out once.  The operations and their order are
 // k_full_det's.
 #pragma once
 #include "engine_kernels.h"

@@ -153,6 +153,21 @@ __device__ __forceinline__ void contract5(cptr<double> coefT, int NO, int NB, in
   o[0] = a0; o[1] = a1; o[2] = a2; o[3] = a3; o[4] = a4;
 }
 
+// contract5 of NB more functions onto o, in the same order as one call would add them
+template <typename T>
+__device__ __forceinline__ void contract5_add(cptr<double> coef, int NO, int NB, int lab,
+                                              const T *__restrict__ ph, double *o) {
+  double a0 = o[0], a1 = o[1], a2 = o[2], a3 = o[3], a4 = o[4];
+#pragma unroll 4
+  for (int b = 0; b < NB; b++) {
+    const double cf = coef[(int64_t)b * NO + lab];
+    const T *p = ph + 5 * b;
+    a0 += cf * (double)p[0]; a1 += cf * (double)p[1]; a2 += cf * (double)p[2];
+    a3 += cf * (double)p[3]; a4 += cf * (double)p[4];
+  }
+  o[0] = a0; o[1] = a1; o[2] = a2; o[3] = a3; o[4] = a4;
+}
+
 // ---------------------------------------------------------------------------
 // In-place inverse of the column-major n x n block `a` by a group (CHAMP's
 // matinv pivoting, rows in parallel).  tmp: n*n scratch.  Returns det (all
@@ -1343,7 +1358,7 @@ __device__ void group_grad_1e(const KArgs &A, const double *ws, int ie,
   // grad(c) = sum_k ai(k,e) d_c(ref_k) + sum_i sum_j y(j,i) ai(i,e) v_c(j)
   //   v_c(j) = d_c(occ_j) - sum_k d_c(ref_k) T(k, occ_j)
   double acc[4] = {0, 0, 0, 0};
-  const int *iref = S.iref[s];
+  const cptr<int> iref = cst(S.iref[s]);
   for (int k = lane; k < ns; k += G) {
     double a = ai[k + ns * e];
     const double *o = orbv + iref[k] * 5;

@@ -5,6 +5,7 @@
 // system's nordc, so every kernel carries only the registers of its order.
 #pragma once
 #include "engine_batch.h"
+#include "engine_move_small.h"
 
 namespace qmcw {
 
@@ -17,7 +18,8 @@ struct LaunchCtx {
   int precision;        // QMCW_FP64 / QMCW_MIXED / QMCW_MIXED_BF16
   size_t smem_ratio;    // dynamic LDS of k_ratio_1e (0 when A.lds_phi == 0)
   size_t smem_nlpp;     // dynamic LDS of k_full_nlpp (0 when A.lds_nlpp == 0)
-  size_t smem_dnlpp;    // dynamic LDS of k_deriv_nlpp (0 when A.lds_dnlpp == 0)
+  size_t smem_dnlpp;    // dynamic LDS of k_deriv_nlpp
+  SmallMove sm;         // k_move_small's LDS record (A.ML adjusted to it)
 };
 
 // What a batch launcher needs (engine_batch.h): the device arrays of the
@@ -36,6 +38,8 @@ struct OrdKernels {
   void (*full_nlpp)(const LaunchCtx &);
   void (*ratio)(const LaunchCtx &, int ie, int mode, const double *xn, double delta,
                 double fbias, double *out, long long *nacc);
+  void (*move_small)(const LaunchCtx &, int ie, int mode, const double *xn, double delta, double fbias,
+                     long long *nacc);
   void (*deriv_jas)(const LaunchCtx &);
   void (*deriv_nlpp)(const LaunchCtx &);
   void (*move_a)(const LaunchCtx &, int ie, int mode, const double *xn, double delta, double fbias);

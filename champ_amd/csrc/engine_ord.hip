@@ -59,6 +59,17 @@ void ratio_g(const LaunchCtx &c, int ie, int mode, const double *xn, double delt
                        mode, xn, delta, fbias, out, nacc);
 }
 template <int G>
+void move_small_g(const LaunchCtx &c, int ie, int mode, const double *xn, double delta, double fbias,
+                  long long *nacc) {
+  const dim3 grid(c.Wl / (kWave / G)), block(kWave);
+  if (c.precision == QMCW_FP64)
+    hipLaunchKernelGGL((k_move_small<double, G, ORD>), grid, block, c.smem_ratio, c.stream, c.A, c.sm, ie,
+                       mode, xn, delta, fbias, nacc);
+  else
+    hipLaunchKernelGGL((k_move_small<float, G, ORD>), grid, block, c.smem_ratio, c.stream, c.A, c.sm, ie,
+                       mode, xn, delta, fbias, nacc);
+}
+template <int G>
 void deriv_jas_g(const LaunchCtx &c) {
   const dim3 grid(c.Wl / (kWave / G)), block(kWave);
   hipLaunchKernelGGL((k_deriv_jas<G, ORD>), grid, block, 0, c.stream, c.A);
@@ -96,6 +107,11 @@ void full_nlpp(const LaunchCtx &c) {
 void ratio(const LaunchCtx &c, int ie, int mode, const double *xn, double delta, double fbias,
            double *out, long long *nacc) {
   QMCW_BY_G(ratio_g, c, ie, mode, xn, delta, fbias, out, nacc);
+}
+void move_small(const LaunchCtx &c, int ie, int mode, const double *xn, double delta, double fbias,
+                long long *nacc) {
+  if (c.G == 8) move_small_g<8>(c, ie, mode, xn, delta, fbias, nacc);
+  else move_small_g<16>(c, ie, mode, xn, delta, fbias, nacc);
 }
 template <int G>
 void move_a_g(const LaunchCtx &c, int ie, int mode, const double *xn, double delta, double fbias) {
@@ -184,7 +200,7 @@ void full_nlpp_tiles_batch(const BatchCtx &c) {
 }  // namespace
 
 #ifndef __HIP_DEVICE_COMPILE__   // a host table of host launchers
-extern const OrdKernels QMCW_CAT(kOrdKernels, QMCW_ORD) = {full_jas, full_nlpp, ratio, deriv_jas,
+extern const OrdKernels QMCW_CAT(kOrdKernels, QMCW_ORD) = {full_jas, full_nlpp, ratio, move_small, deriv_jas,
                                                             deriv_nlpp, move_a, tm_ratios,
                                                             ratio_batch, sweep_batch,
                                                             full_jas_batch, full_nlpp_batch,
