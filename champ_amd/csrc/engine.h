@@ -44,7 +44,7 @@ struct DevSys {
   // real solid harmonics S_lm (m listed in sh_m) that multiply it
   int nshell;                // over all centres
   const int *cent_sh_off;    // [M+1]
-  const int *sh_by_l;        // [nshell] the shells in order of l
+  const int *sh_by_l;        // [nshell] the shells in order of l, then of their primitives
   const int *cent_bas;       // [M+1] first basis function of each centre
   int cent_bas_max;          // most basis functions of one centre
   const int *sh_cent, *sh_l, *sh_a, *sh_nm, *sh_prim_off;

@@ -795,11 +795,13 @@ static KArgs move_args(const qmcw_handle *h, int G, bool split, size_t &phi_b, s
   const bool sums = !batch && (h->precision == QMCW_FP64 ? een_sums<double>(G, A.S.M) : een_sums<float>(G, A.S.M));
   const int tab = (A.S.nordc > 1 && !split && !h->no_een_tab)
                       ? A.S.M * (3 * ((ordk + 1) * (ordk + 2) / 2) + (sums ? 4 : 8)) : 0;
-  const int wst = std::max(A.S.NB * 5, tab);
+  // (sm_update's vectors take the region after the basis values)
+  const int smv = (int)((3 * std::max(A.S.ns[0], A.S.ns[1]) + std::max(A.S.nocc[0], A.S.nocc[1])) * sizeof(double) / tsz);
+  const int phi = std::max(A.S.NB * 5, smv), wst = (std::max(phi, tab) + 1) / 2 * 2;
   const size_t lds = (size_t)(kWave / G) * wst * tsz;
   A.lds_phi = (h->use_lds && lds <= 48 * 1024) ? 1 : 0;
   A.een_tab = (A.lds_phi && tab > 0) ? 1 : 0;
-  A.lds_wst = A.een_tab ? wst : A.S.NB * 5;
+  A.lds_wst = A.een_tab ? wst : (phi + 1) / 2 * 2;
   phi_b = A.lds_phi ? ((size_t)(kWave / G) * A.lds_wst * tsz + 7) / 8 * 8 : 0;
   // eval_y's determinant values and alpha inverses staged in LDS after the
   // basis values, when the two together stay within 48 KB per block and
@@ -1026,7 +1028,8 @@ extern "C" int qmcw_create(const qmcw_system *s, int32_t nwalk, int32_t precisio
     UP(cb, S.cent_bas);
     std::vector<int> byl(sh_l.size());
     for (size_t q = 0; q < byl.size(); q++) byl[q] = (int)q;
-    std::stable_sort(byl.begin(), byl.end(), [&](int a, int b) { return sh_l[a] < sh_l[b]; });
+    const auto key = [&](int q) { return std::make_pair(sh_l[q], sh_prim_off[q + 1] - sh_prim_off[q]); };
+    std::stable_sort(byl.begin(), byl.end(), [&](int a, int b) { return key(a) < key(b); });
     UP(byl, S.sh_by_l);
   }
   UP(cent_sh_off, S.cent_sh_off); UP(pz, S.prim_zeta); UP(pc, S.prim_coef);

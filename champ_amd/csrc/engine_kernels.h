@@ -22,7 +22,7 @@ struct KArgs {
   int derivs;        // compute Jastrow/NLPP parameter derivative pieces
   int full_orb;      // evaluate all NO orbitals (orbital-rotation derivatives)
   int lds_phi;       // k_ratio_1e keeps the moved electron's basis values in LDS
-  int lds_wst;       // T values per walker of that LDS region (at least NB * 5)
+  int lds_wst;       // T values per walker of that LDS region (even; at least NB * 5, and sm_update's)
   int een_tab;       // k_ratio_1e: the moved electron's e-e-n tables in the same region
                      // during the Jastrow row (een_tables or een_sum_tables)
   int orb_only;      // k_full_det ends after the orbitals (k_det_small does the determinants)
@@ -139,12 +139,35 @@ __device__ __forceinline__ float bf16r(float x) {
 // of its rows near a node: bfloat16 inputs there gave local-energy errors of
 // tens of Ha, so the BF16 mode does not round them (it rounds only the
 // pseudopotential projection, group_gproj).
+// The coefficients come from L2 (a lane an orbital): the next eight are on
+// their way while eight are used; with four loaded and waited for at a time
+// this loop was half of the orbitals' 31,000 cycles of a 38-electron move.
 template <typename T>
 __device__ __forceinline__ void contract5(cptr<double> coefT, int NO, int NB, int lab,
                                           const T *__restrict__ ph, double *o) {
+  constexpr int U = 8;
   double a0 = 0, a1 = 0, a2 = 0, a3 = 0, a4 = 0;
-#pragma unroll 4
-  for (int b = 0; b < NB; b++) {
+  int b = 0;
+  if (NB >= U) {
+    double c[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) c[u] = coefT[(int64_t)u * NO + lab];
+    for (; b + U <= NB; b += U) {
+      double n[U];
+      const int64_t nx = b + 2 * U <= NB ? b + U : b;      // (the last round loads its own again)
+#pragma unroll
+      for (int u = 0; u < U; u++) n[u] = coefT[(nx + u) * NO + lab];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const T *p = ph + 5 * (b + u);
+        a0 += c[u] * (double)p[0]; a1 += c[u] * (double)p[1]; a2 += c[u] * (double)p[2];
+        a3 += c[u] * (double)p[3]; a4 += c[u] * (double)p[4];
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) c[u] = n[u];
+    }
+  }
+  for (; b < NB; b++) {
     const double cf = coefT[(int64_t)b * NO + lab];
     const T *p = ph + 5 * b;
     a0 += cf * (double)p[0]; a1 += cf * (double)p[1]; a2 += cf * (double)p[2];
@@ -1421,24 +1444,66 @@ __device__ __forceinline__ void sm_vectors(double *__restrict__ vi1, double *__r
   }
 }
 
-// rank-1 updates A^-1_new = A^-1 + u vi1^T, T_new = T + u vi2^T with
-// u(k) = -A^-1(k, e) / ratio
+// dete_update of one walker by its group: the ratio (returned), and the
+// rank-1 updates A^-1_new = A^-1 + u vi1^T and T_new = T + u vi2^T with
+// u(k) = -A^-1(k, e) / ratio, into the candidates.  v: 3 ns + nocc doubles (the
+// reference orbitals' values, u, vi1, vi2), in LDS where the launch has it.
+// A lane's loads are a batch ahead of their use and u is formed once: reading
+// the orbitals through their index and dividing per element took 64,000
+// cycles of a 98-electron move.  Ends with a barrier.
 template <int G>
-__device__ __forceinline__ void sm_rank1(double *__restrict__ ain, double *__restrict__ tn,
-                                         const double *__restrict__ ai, const double *__restrict__ tocc,
-                                         const double *__restrict__ vi1, const double *__restrict__ vi2,
-                                         int ns, int nocc, int e, double rat, int lane, bool no_t = false) {
-#pragma unroll 4
-  for (int q = lane; q < ns * ns; q += G) {
-    const int k = q % ns, i = q / ns;
-    ain[q] = ai[q] + (-ai[k + ns * e] / rat) * vi1[i];
+__device__ __forceinline__ double sm_update(double *__restrict__ v, double *__restrict__ ain,
+                                            double *__restrict__ tn, const double *__restrict__ orbe,
+                                            const double *__restrict__ ai, const double *__restrict__ tocc,
+                                            cptr<int> iref, int ns, int nocc, int e, int lane, bool no_t) {
+  double *ref = v, *u = v + ns, *vi1 = v + 2 * ns, *vi2 = v + 3 * ns;
+  double rat = 0.0;
+  for (int k = lane; k < ns; k += G) {
+    const double o = orbe[5 * iref[k]], a = ai[k + ns * e];
+    ref[k] = o;
+    u[k] = -a;
+    rat += o * a;
   }
-  if (no_t) return;
-#pragma unroll 4
-  for (int q = lane; q < ns * nocc; q += G) {
-    const int k = q / nocc, j = q % nocc;
-    tn[q] = tocc[q] + (-ai[k + ns * e] / rat) * vi2[j];
+  rat = gsum<G>(rat);
+  for (int k = lane; k < ns; k += G) u[k] = u[k] / rat;
+  __syncthreads();
+  for (int i = lane; i < ns; i += G) {
+    double acc = 0.0;
+#pragma unroll 8
+    for (int k = 0; k < ns; k++) acc += ref[k] * ai[k + ns * i];
+    vi1[i] = acc - (i == e ? 1.0 : 0.0);
   }
+  for (int j = no_t ? nocc : lane; j < nocc; j += G) {
+    double acc = 0.0;
+#pragma unroll 8
+    for (int k = 0; k < ns; k++) acc += ref[k] * tocc[k * nocc + j];
+    vi2[j] = acc - orbe[5 * j];
+  }
+  __syncthreads();
+  {
+    const int dk = G % ns, di = G / ns;
+    int k = lane % ns, i = lane / ns;
+#pragma unroll 8
+    for (int q = lane; q < ns * ns; q += G) {
+      ain[q] = ai[q] + u[k] * vi1[i];
+      k += dk;
+      i += di;
+      if (k >= ns) { k -= ns; i++; }
+    }
+  }
+  if (!no_t) {
+    const int dj = G % nocc, dk = G / nocc;
+    int j = lane % nocc, k = lane / nocc;
+#pragma unroll 8
+    for (int q = lane; q < ns * nocc; q += G) {
+      tn[q] = tocc[q] + u[k] * vi2[j];
+      j += dj;
+      k += dk;
+      if (j >= nocc) { j -= nocc; k++; }
+    }
+  }
+  __syncthreads();
+  return rat;
 }
 
 // basis values (value, gradient, laplacian) of one position into phi, then
@@ -1447,11 +1512,27 @@ template <typename T, int G>
 __device__ __forceinline__ void orbitals_1e(const KArgs &A, int s, int nocc, const double *ren,
                                             const double *rven, T *phi, double *orbe, int lane) {
   const DevSys &S = A.S;
-  for (int sh = lane; sh < S.nshell; sh += G) {
-    const int ic = cst(S.sh_cent)[sh];
+  // shells of like l side by side: the lanes of a pass take one branch
+  for (int q = lane; q < S.nshell; q += G) {
+    const int sh = cst(S.sh_by_l)[q], ic = cst(S.sh_cent)[sh];
     eval_shell<T>(S, sh, (T)rven[3 * ic], (T)rven[3 * ic + 1], (T)rven[3 * ic + 2], (T)ren[ic], 1, phi);
   }
   __syncthreads();
+  // half as many orbitals as lanes, or fewer: the lanes share the basis too
+  const int parts = nocc <= G / 4 ? 4 : nocc <= G / 2 ? 2 : 1;
+  if (G >= 32 && parts > 1) {
+    const int wd = G / parts, j = lane % wd, nb = (S.NB + parts - 1) / parts;
+    const int b0 = min(S.NB, (lane / wd) * nb), b1 = min(S.NB, b0 + nb);
+    double o[5] = {0, 0, 0, 0, 0};
+    if (j < nocc) contract5<T>(cst(S.coef_occ[s]) + (int64_t)b0 * nocc, nocc, b1 - b0, j, phi + 5 * b0, o);
+    for (int d = wd; d < G; d *= 2)
+#pragma unroll
+      for (int c = 0; c < 5; c++) o[c] += __shfl_xor(o[c], d);
+    if (lane < nocc)
+#pragma unroll
+      for (int c = 0; c < 5; c++) orbe[5 * j + c] = o[c];
+    return;
+  }
   for (int j = lane; j < nocc; j += G)
     contract5<T>(cst(S.coef_occ[s]), nocc, S.NB, j, phi, orbe + 5 * j);
 }
@@ -1572,6 +1653,19 @@ __device__ __forceinline__ void ratio_1e_b(const KArgs &A, int bid_, int ie, int
     PairOut<T> po;
     bool par = (hi < S.nup) || (lo >= S.nup);
     // moved electron's arrays go to whichever slot (hi or lo) it occupies
+    // the pair's old values: on their way during the row's arithmetic in FP32
+    // (in FP64 it leaves no registers for them)
+    double f_old, gi_old[3], gj_old[3], fj_old[3];
+    const auto load_old = [&]() {
+      f_old = fso[hi * N + lo];
+#pragma unroll
+      for (int q = 0; q < 3; q++) {
+        gi_old[q] = fijo[3 * (ie * N + j) + q];
+        gj_old[q] = fijo[3 * (j * N + ie) + q];
+        fj_old[q] = fjo[3 * j + q];
+      }
+    };
+    if (sizeof(T) == 4) load_old();
     // the other electron's distances formed from its position (see EnFromX)
     const EnRows pI{rI, rvI};
     const EnFromX pJ{x[3 * j], x[3 * j + 1], x[3 * j + 2]};
@@ -1588,10 +1682,7 @@ __device__ __forceinline__ void ratio_1e_b(const KArgs &A, int bid_, int ie, int
       jas_pair_g<T, ORD>(S, par, (T)ree[j], rvij, pJ, pI, po);
     }
     // old pair values before the stores to the pending buffers below
-    const double f_old = fso[hi * N + lo];
-    const double gi_old[3] = {fijo[3 * (ie * N + j)], fijo[3 * (ie * N + j) + 1], fijo[3 * (ie * N + j) + 2]};
-    const double gj_old[3] = {fijo[3 * (j * N + ie)], fijo[3 * (j * N + ie) + 1], fijo[3 * (j * N + ie) + 2]};
-    const double fj_old[3] = {fjo[3 * j], fjo[3 * j + 1], fjo[3 * j + 2]};
+    if (sizeof(T) == 8) load_old();
     // per-component selects keep po in registers
     const bool mi = hi == ie;
     const T g_ie[3] = {mi ? po.gi[0] : po.gj[0], mi ? po.gi[1] : po.gj[1], mi ? po.gi[2] : po.gj[2]};
@@ -1636,19 +1727,14 @@ __device__ __forceinline__ void ratio_1e_b(const KArgs &A, int bid_, int ie, int
   const double *tocc = w_tocc(L, ws, s);
   // candidates into the other slots of the state (the commit flips them)
   double *ain = w_ai(L, ws, s, 1), *tn = w_tocc(L, ws, s, 1);
-  double rat = 0.0;
-  for (int k = lane; k < ns; k += G) rat += orbe[5 * cst(S.iref[s])[k]] * ai[k + ns * e];
-  rat = gsum<G>(rat);
-  // vi1(i) = sum_k orbe(ref_k) ai(k, i) - delta(i, e); ui(k) = -ai(k,e)/rat
-  double *vi1 = mv + ML.misc + 8;            // [ns]
-  double *vi2 = vi1 + ns;                    // [nocc]
   // a single determinant needs only A^-1: T stays the fixed permutation
   // and the excited-determinant blocks, Y and chi do not change
   const bool single = S.single_det;
-  sm_vectors<G>(vi1, vi2, orbe, ai, tocc, S.iref[s], ns, nocc, e, lane, single);
-  __syncthreads();
-  sm_rank1<G>(ain, tn, ai, tocc, vi1, vi2, ns, nocc, e, rat, lane, single);
-  __syncthreads();
+  double rat;
+  if (A.lds_phi)               // where the basis values were
+    rat = sm_update<G>(reinterpret_cast<double *>(etab), ain, tn, orbe, ai, tocc, cst(S.iref[s]), ns, nocc, e, lane, single);
+  else
+    rat = sm_update<G>(ss + SL.phi, ain, tn, orbe, ai, tocc, cst(S.iref[s]), ns, nocc, e, lane, single);
   double *invn = w_inv(L, ws, s, 1), *detn = w_detv(L, ws, s, 1);
   for (int u = single ? S.ndetu[s] : lane; u < S.ndetu[s]; u += G) {
     int k = cst(S.ord[s])[u];
@@ -1865,9 +1951,9 @@ __global__ QMCW_MOVE void k_move_b(KArgs A, int ie) {
   // two calls keep the LDS pointer visible as such to the compiler)
   extern __shared__ double dyn_lds[];
   double *orbe = mv + ML.orbe;
+  T *phi = reinterpret_cast<T *>(dyn_lds) + (int64_t)grp * A.lds_wst;
   if (A.lds_phi)
-    orbitals_1e<T, G>(A, s, nocc, ren, rven, reinterpret_cast<T *>(dyn_lds) + (int64_t)grp * S.NB * 5,
-                      orbe, lane);
+    orbitals_1e<T, G>(A, s, nocc, ren, rven, phi, orbe, lane);
   else
     orbitals_1e<T, G>(A, s, nocc, ren, rven, reinterpret_cast<T *>(ss + SL.phi), orbe, lane);
   __syncthreads();
@@ -1876,16 +1962,11 @@ __global__ QMCW_MOVE void k_move_b(KArgs A, int ie) {
   const double *tocc = w_tocc(L, ws, s);
   // candidates into the other slots of the state (the commit flips them)
   double *ain = w_ai(L, ws, s, 1), *tn = w_tocc(L, ws, s, 1);
-  double rat = 0.0;
-  for (int k = lane; k < ns; k += G) rat += orbe[5 * cst(S.iref[s])[k]] * ai[k + ns * e];
-  rat = gsum<G>(rat);
-  // vi1(i) = sum_k orbe(ref_k) ai(k, i) - delta(i, e); ui(k) = -ai(k,e)/rat
-  double *vi1 = mv + ML.misc + 8;            // [ns]
-  double *vi2 = vi1 + ns;                    // [nocc]
-  sm_vectors<G>(vi1, vi2, orbe, ai, tocc, S.iref[s], ns, nocc, e, lane);
-  __syncthreads();
-  sm_rank1<G>(ain, tn, ai, tocc, vi1, vi2, ns, nocc, e, rat, lane);
-  __syncthreads();
+  double rat;
+  if (A.lds_phi)
+    rat = sm_update<G>(reinterpret_cast<double *>(phi), ain, tn, orbe, ai, tocc, cst(S.iref[s]), ns, nocc, e, lane, false);
+  else
+    rat = sm_update<G>(ss + SL.phi, ain, tn, orbe, ai, tocc, cst(S.iref[s]), ns, nocc, e, lane, false);
   double *invn = w_inv(L, ws, s, 1), *detn = w_detv(L, ws, s, 1);
   for (int u = lane; u < S.ndetu[s]; u += G) {
     int k = cst(S.ord[s])[u];
