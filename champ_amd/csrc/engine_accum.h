@@ -26,10 +26,10 @@ typedef double acc_d4 __attribute__((ext_vector_type(4)));
 
 __host__ __device__ inline int64_t accum_doubles(int P) { return 3 + 3 * (int64_t)P + 3 * (int64_t)P * P; }
 
-// der: [W][ldd] rows of dpsi[P] followed by deloc[P]; E_L of walker w at
+// der: dpsi [W][P]; del: deloc [W][P]; E_L of walker w at
 // st[w * lst + eoff].  part: [nchunk][3][P][P].
-__global__ __launch_bounds__(64) void k_accum_gemm(const double *__restrict__ der, int ldd, int P,
-                                                   const double *__restrict__ st, int64_t lst,
+__global__ __launch_bounds__(64) void k_accum_gemm(const double *__restrict__ der, const double *__restrict__ del,
+                                                   int P, const double *__restrict__ st, int64_t lst,
                                                    int64_t eoff, int W, double *__restrict__ part) {
   const int nb = (P + kAccBlk - 1) / kAccBlk;
   const int bi = blockIdx.x / nb, bj = blockIdx.x % nb, c = blockIdx.y;
@@ -52,7 +52,7 @@ __global__ __launch_bounds__(64) void k_accum_gemm(const double *__restrict__ de
     const int ww = w + kq;
     const double ok = ww < w1 ? 1.0 : 0.0;             // walkers past the chunk add zero
     const int wc = min(ww, w1 - 1);                    // and read an in-range row
-    const double *row = der + (int64_t)wc * ldd;
+    const double *row = der + (int64_t)wc * P, *rol = del + (int64_t)wc * P;
     const double e = ok * st[(int64_t)wc * lst + eoff];
     double a[2], b[2], l[2];
 #pragma unroll
@@ -60,7 +60,7 @@ __global__ __launch_bounds__(64) void k_accum_gemm(const double *__restrict__ de
       const int ii = i0 + 16 * t + r, jj = j0 + 16 * t + r;
       a[t] = ii < P ? ok * row[ii] : 0.0;
       b[t] = jj < P ? ok * row[jj] : 0.0;
-      l[t] = jj < P ? ok * row[P + jj] : 0.0;
+      l[t] = jj < P ? ok * rol[jj] : 0.0;
     }
 #pragma unroll
     for (int t = 0; t < 2; t++)
@@ -86,8 +86,8 @@ __global__ __launch_bounds__(64) void k_accum_gemm(const double *__restrict__ de
 }
 
 // Vector sums of one chunk: partv[c][3 + 3P] as the accumulator's head.
-__global__ __launch_bounds__(64) void k_accum_vec(const double *__restrict__ der, int ldd, int P,
-                                                  const double *__restrict__ st, int64_t lst,
+__global__ __launch_bounds__(64) void k_accum_vec(const double *__restrict__ der, const double *__restrict__ del,
+                                                  int P, const double *__restrict__ st, int64_t lst,
                                                   int64_t eoff, int W, double *__restrict__ partv) {
   const int t = blockIdx.x * 64 + threadIdx.x, c = blockIdx.y;
   const int w0 = c * kAccChunk, w1 = min(W, w0 + kAccChunk);
@@ -96,11 +96,10 @@ __global__ __launch_bounds__(64) void k_accum_vec(const double *__restrict__ der
     double sd = 0.0, sde = 0.0, sl = 0.0;
 #pragma unroll 8
     for (int w = w0; w < w1; w++) {
-      const double *row = der + (int64_t)w * ldd;
-      const double d = row[t], e = st[(int64_t)w * lst + eoff];
+      const double d = der[(int64_t)w * P + t], e = st[(int64_t)w * lst + eoff];
       sd += d;
       sde += d * e;
-      sl += row[P + t];
+      sl += del[(int64_t)w * P + t];
     }
     o[3 + t] = sd;
     o[3 + P + t] = sde;

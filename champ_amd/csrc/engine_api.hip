@@ -53,7 +53,9 @@ struct qmcw_handle {
   std::vector<int> csf_det_off, csf_det;
   std::vector<double> csf_det_coef;
   int nparm = 0;
-  double *der = nullptr;     // [Wp][2 nparm] dpsi, deloc of the last derivative evaluation
+  double *der = nullptr;     // [2][Wp][nparm] dpsi, then deloc, of the last derivative evaluation
+  double *del() const { return der + (size_t)Wp * nparm; }   // deloc, after dpsi
+  double *pin = nullptr;      // pinned host memory of a call's results and inputs (pin_*)
   int sample_derivs = 0;     // VMC steps evaluate derivatives (CHAMP's ideriv)
   int der_valid = 0;
   // one VMC step captured as a HIP graph (qmcw_vmc_run_device) and its key
@@ -489,17 +491,36 @@ __global__ void k_init_walkers(KArgs A, int W) {
   }
 }
 
-__global__ void k_gather_full(KArgs A, double *out, int W) {
-  int w = blockIdx.x * blockDim.x + threadIdx.x;
-  if (w >= W) return;
-  const int N = A.S.N, stride = 8 + 4 * N;
+// The full evaluation's results in the caller's layout: grad [W][N][3] and
+// lap [W][N] on the device, the walkers' five scalars [5][W] and the error
+// flags (1 set for each bit that any walker has) in pinned host memory.
+__global__ void k_gather_full(KArgs A, double *grad, double *lap, double *sc5, int *fl, int W,
+                              int nflag) {
+  const int N = A.S.N, n = 4 * N + 1;
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= (int64_t)W * n) return;
+  const int w = (int)(t / n), q = (int)(t % n);
   const double *ws = A.st + (int64_t)w * A.L.stride;
   const double *ss = A.sc + (int64_t)w * A.SL.stride;
-  double *o = out + (int64_t)w * stride;
-  o[0] = ws[A.L.logpsid]; o[1] = ws[A.L.sgn]; o[2] = ws[A.L.psij]; o[3] = ws[A.L.eloc];
-  o[4] = ws[A.L.epot]; o[5] = ss[A.SL.phs + 60]; o[6] = ss[A.SL.phs + 61]; o[7] = ss[A.SL.phs + 62];
-  for (int q = 0; q < 3 * N; q++) o[8 + q] = ss[A.SL.vj + q] + ss[A.SL.vd + q];
-  for (int i = 0; i < N; i++) o[8 + 3 * N + i] = ss[A.SL.divv + i];
+  if (q < 3 * N) {
+    grad[(int64_t)w * 3 * N + q] = ss[A.SL.vj + q] + ss[A.SL.vd + q];
+  } else if (q < 4 * N) {
+    lap[(int64_t)w * N + q - 3 * N] = ss[A.SL.divv + q - 3 * N];
+  } else {
+    sc5[w] = ws[A.L.logpsid]; sc5[W + w] = ws[A.L.sgn]; sc5[2 * W + w] = ws[A.L.psij];
+    sc5[3 * W + w] = ws[A.L.eloc]; sc5[4 * W + w] = ws[A.L.epot];
+    const int f = w < nflag ? A.flags[w] : 0;
+    for (int b = 0; b < 3; b++)
+      if (f & (1 << b)) fl[b] = 1;
+  }
+}
+
+// the error flags alone
+__global__ void k_gather_flags(const int *flags, int *fl, int W) {
+  const int w = blockIdx.x * blockDim.x + threadIdx.x;
+  if (w >= W) return;
+  for (int b = 0; b < 3; b++)
+    if (flags[w] & (1 << b)) fl[b] = 1;
 }
 
 __global__ void k_trace_eloc(KArgs A, double *trace, int step, int W) {
@@ -552,7 +573,7 @@ static void launch_fin(qmcw_handle *h, const KArgs &A) {
 template <int G>
 static void launch_derivs_asm(qmcw_handle *h, const KArgs &A) {
   const dim3 grid(h->Wl / (kWave / G)), block(kWave);
-  hipLaunchKernelGGL((k_derivs<G, false>), grid, block, 0, h->stream, A, h->der);
+  hipLaunchKernelGGL((k_derivs<G, false>), grid, block, 0, h->stream, A, h->der, h->del());
 }
 
 #define DISPATCH_GW(gw, fn, ...)                  \
@@ -761,7 +782,7 @@ static void launch_eval(qmcw_handle *h, bool derivs) {
     // its intermediates in LDS while four blocks fit a compute unit's 160 KB
     const size_t lds = sizeof(double) * derivs_lds_doubles(A.S);
     if (h->use_lds && lds <= 40 * 1024)
-      hipLaunchKernelGGL((k_derivs<64, true>), dim3(h->Wl), dim3(kWave), lds, h->stream, A, h->der);
+      hipLaunchKernelGGL((k_derivs<64, true>), dim3(h->Wl), dim3(kWave), lds, h->stream, A, h->der, h->del());
     else
       DISPATCH_GW(gd, launch_derivs_asm, h, A);
     prof_end(h);
@@ -1387,6 +1408,8 @@ extern "C" int qmcw_create(const qmcw_system *s, int32_t nwalk, int32_t precisio
   h->io_doubles = (size_t)h->Wp * std::max(8 + 4 * N, 8);
   if (hipMalloc(&p, h->io_doubles * sizeof(double)) != hipSuccess) { qmcw_destroy(h); return fail(nullptr, QMCW_ERR_NOMEM, "io alloc"); }
   h->allocs.push_back(p); h->io = (double *)p;
+  if (hipHostMalloc(&p, (size_t)h->Wp * 12 * sizeof(double) + 64) != hipSuccess) { qmcw_destroy(h); return fail(nullptr, QMCW_ERR_NOMEM, "pinned alloc"); }
+  h->pin = (double *)p;
   (void)hipMemsetAsync(h->A.st, 0, stb, h->stream);
   (void)hipMemsetAsync(h->A.sc, 0, scb, h->stream);
   (void)hipMemsetAsync(h->A.rng, 0, (size_t)h->Wp * 4 * sizeof(int), h->stream);
@@ -1427,6 +1450,7 @@ extern "C" int qmcw_destroy(qmcw_handle *h) {
   for (hipEvent_t e : h->ev) (void)hipEventDestroy(e);
   for (void *p : h->allocs) (void)hipFree(p);
   if (h->trace) (void)hipFree(h->trace);
+  if (h->pin) (void)hipHostFree(h->pin);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
   return QMCW_OK;
@@ -1555,17 +1579,31 @@ extern "C" int qmcw_get_rng(const qmcw_handle *hc, int32_t *seed) {
   return QMCW_OK;
 }
 
+// The per-call results and inputs in pinned host memory that the kernels read
+// and write themselves: out [8][Wp], the given positions [3][Wp], the
+// decisions [Wp] bytes and three error flags.  Without a copy command each way
+// a cycle of nine one-electron calls took 332 instead of 395 us for 64
+// four-electron walkers, 1,464 instead of 1,742 for 4,099 C2-like ones.
+static double *pin_x(const qmcw_handle *h) { return h->pin + (size_t)h->Wp * 8; }
+static uint8_t *pin_acc(const qmcw_handle *h) { return (uint8_t *)(h->pin + (size_t)h->Wp * 11); }
+static int *pin_flags(const qmcw_handle *h) { return (int *)(h->pin + (size_t)h->Wp * 12); }
+
+static int flags_status(qmcw_handle *h) {
+  const int *f = pin_flags(h);
+  if (f[0]) return fail(h, QMCW_ERR_SINGULAR, "a Slater matrix is singular");
+  if (f[1]) return fail(h, QMCW_ERR_NAN, "non-finite local energy");
+  if (f[2]) return fail(h, QMCW_ERR_ARG, "an electron is in range of more pseudopotential centres than the T-move record holds");
+  return QMCW_OK;
+}
+
 static int check_flags(qmcw_handle *h) {
   const int n = h->dmc_on ? h->nact : h->W;
-  std::vector<int> fl(n);
-  HIPCHK(h, hipMemcpyAsync(fl.data(), h->A.flags, n * sizeof(int), hipMemcpyDeviceToHost, h->stream));
+  int *f = pin_flags(h);
+  f[0] = f[1] = f[2] = 0;
+  hipLaunchKernelGGL(k_gather_flags, dim3((n + 255) / 256), dim3(256), 0, h->stream, (const int *)h->A.flags, f, n);
+  HIPCHK(h, hipGetLastError());
   HIPCHK(h, hipStreamSynchronize(h->stream));
-  int any = 0;
-  for (int f : fl) any |= f;
-  if (any & 1) return fail(h, QMCW_ERR_SINGULAR, "a Slater matrix is singular");
-  if (any & 2) return fail(h, QMCW_ERR_NAN, "non-finite local energy");
-  if (any & 4) return fail(h, QMCW_ERR_ARG, "an electron is in range of more pseudopotential centres than the T-move record holds");
-  return QMCW_OK;
+  return flags_status(h);
 }
 
 extern "C" int qmcw_eval_full(qmcw_handle *h, double *logpsid, double *sgn, double *psij,
@@ -1573,38 +1611,34 @@ extern "C" int qmcw_eval_full(qmcw_handle *h, double *logpsid, double *sgn, doub
   if (!h) return QMCW_ERR_ARG;
   launch_eval(h, false);
   HIPCHK(h, hipGetLastError());
-  int N = h->A.S.N, stride = 8 + 4 * N;
-  hipLaunchKernelGGL(k_gather_full, dim3((h->W + 63) / 64), dim3(64), 0, h->stream, h->A, h->io, h->W);
-  std::vector<double> o((size_t)h->W * stride);
-  HIPCHK(h, hipMemcpyAsync(o.data(), h->io, o.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+  const int N = h->A.S.N;
+  const size_t W = h->W;
+  double *dg = h->io, *dl = h->io + W * 3 * N;
+  int *f = pin_flags(h);
+  f[0] = f[1] = f[2] = 0;
+  hipLaunchKernelGGL(k_gather_full, dim3((unsigned)((W * (4 * N + 1) + 255) / 256)), dim3(256), 0, h->stream,
+                     h->A, dg, dl, h->pin, f, h->W, h->dmc_on ? h->nact : h->W);
+  HIPCHK(h, hipGetLastError());
+  if (grad) HIPCHK(h, hipMemcpyAsync(grad, dg, W * 3 * N * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+  if (lap) HIPCHK(h, hipMemcpyAsync(lap, dl, W * N * sizeof(double), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
-  for (int w = 0; w < h->W; w++) {
-    const double *r = o.data() + (size_t)w * stride;
-    if (logpsid) logpsid[w] = r[0];
-    if (sgn) sgn[w] = r[1];
-    if (psij) psij[w] = r[2];
-    if (eloc) eloc[w] = r[3];
-    if (epot) epot[w] = r[4];
-    if (grad) memcpy(grad + (size_t)w * 3 * N, r + 8, 3 * N * sizeof(double));
-    if (lap) memcpy(lap + (size_t)w * N, r + 8 + 3 * N, N * sizeof(double));
-  }
-  return check_flags(h);
+  double *const dst[5] = {logpsid, sgn, psij, eloc, epot};
+  for (int q = 0; q < 5; q++)
+    if (dst[q]) memcpy(dst[q], h->pin + q * W, W * sizeof(double));
+  return flags_status(h);
 }
 
 extern "C" int qmcw_ratio_1e(qmcw_handle *h, int32_t ie, const double *xnew, double *ratio,
                              double *grad_new, double *lap_new) {
   if (!h || !xnew || ie < 0 || ie >= h->A.S.N) return QMCW_ERR_ARG;
-  // xnew staged after the 8*Wp output block
-  double *xin = h->io + (size_t)h->Wp * 8;
-  std::vector<double> xp((size_t)h->Wp * 3);
-  for (int w = 0; w < h->Wp; w++)
-    for (int q = 0; q < 3; q++) xp[3 * w + q] = xnew[3 * std::min(w, h->W - 1) + q];
-  HIPCHK(h, hipMemcpyAsync(xin, xp.data(), xp.size() * sizeof(double), hipMemcpyHostToDevice, h->stream));
-  launch_ratio(h, ie, 0, (const double *)xin, 1.0, 1.0, h->io);
+  double *xp = pin_x(h);
+  memcpy(xp, xnew, (size_t)h->W * 3 * sizeof(double));
+  for (int w = h->W; w < h->Wp; w++)
+    for (int q = 0; q < 3; q++) xp[3 * w + q] = xnew[3 * (h->W - 1) + q];
+  launch_ratio(h, ie, 0, (const double *)xp, 1.0, 1.0, h->pin);
   HIPCHK(h, hipGetLastError());
-  std::vector<double> o((size_t)h->W * 8);
-  HIPCHK(h, hipMemcpyAsync(o.data(), h->io, o.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
+  const double *o = h->pin;
   for (int w = 0; w < h->W; w++) {
     if (ratio) ratio[w] = o[8 * w];
     if (grad_new) for (int q = 0; q < 3; q++) grad_new[3 * w + q] = o[8 * w + 4 + q];
@@ -1615,10 +1649,10 @@ extern "C" int qmcw_ratio_1e(qmcw_handle *h, int32_t ie, const double *xnew, dou
 
 extern "C" int qmcw_accept_1e(qmcw_handle *h, int32_t ie, const uint8_t *accept) {
   if (!h || !accept || ie < 0 || ie >= h->A.S.N) return QMCW_ERR_ARG;
-  std::vector<uint8_t> a(h->Wp, 0);
-  for (int w = 0; w < h->W; w++) a[w] = accept[w];
-  HIPCHK(h, hipMemcpyAsync(h->acc_buf, a.data(), h->Wp, hipMemcpyHostToDevice, h->stream));
-  DISPATCH_MOVE(h, launch_accept, ie, 0, (const uint8_t *)h->acc_buf, 1.0, 1.0, (long long *)nullptr);
+  uint8_t *a = pin_acc(h);
+  memcpy(a, accept, h->W);
+  memset(a + h->W, 0, h->Wp - h->W);
+  DISPATCH_MOVE(h, launch_accept, ie, 0, (const uint8_t *)a, 1.0, 1.0, (long long *)nullptr);
   HIPCHK(h, hipGetLastError());
   HIPCHK(h, hipStreamSynchronize(h->stream));
   return QMCW_OK;
@@ -1626,11 +1660,10 @@ extern "C" int qmcw_accept_1e(qmcw_handle *h, int32_t ie, const uint8_t *accept)
 
 extern "C" int qmcw_grad_1e(qmcw_handle *h, int32_t ie, double *grad, double *lap) {
   if (!h || ie < 0 || ie >= h->A.S.N) return QMCW_ERR_ARG;
-  DISPATCH_MOVE(h, launch_grad, ie, h->io);
+  DISPATCH_MOVE(h, launch_grad, ie, h->pin);
   HIPCHK(h, hipGetLastError());
-  std::vector<double> o((size_t)h->W * 4);
-  HIPCHK(h, hipMemcpyAsync(o.data(), h->io, o.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
+  const double *o = h->pin;
   for (int w = 0; w < h->W; w++) {
     if (grad) for (int q = 0; q < 3; q++) grad[3 * w + q] = o[4 * w + q];
     if (lap) lap[w] = o[4 * w + 3];
@@ -1663,10 +1696,10 @@ static void launch_accum(qmcw_handle *h) {
   const int64_t n = accum_doubles(P);
   prof_begin(h, QMCW_PROF_ACCUM);
   hipLaunchKernelGGL(k_accum_gemm, dim3(nb * nb, nch), dim3(64), 0, h->stream, (const double *)h->der,
-                     2 * P, P, (const double *)h->A.st, (int64_t)h->A.L.stride, (int64_t)h->A.L.eloc,
+                     (const double *)h->del(), P, (const double *)h->A.st, (int64_t)h->A.L.stride, (int64_t)h->A.L.eloc,
                      h->W, h->acc_part);
   hipLaunchKernelGGL(k_accum_vec, dim3((P + 1 + 63) / 64, nch), dim3(64), 0, h->stream,
-                     (const double *)h->der, 2 * P, P, (const double *)h->A.st,
+                     (const double *)h->der, (const double *)h->del(), P, (const double *)h->A.st,
                      (int64_t)h->A.L.stride, (int64_t)h->A.L.eloc, h->W, h->acc_partv);
   hipLaunchKernelGGL(k_accum_reduce, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h->stream,
                      (const double *)h->acc_part, (const double *)h->acc_partv, nch, P, h->acc);
@@ -2253,16 +2286,13 @@ extern "C" int qmcw_get_eloc(const qmcw_handle *hc, double *eloc) {
   return QMCW_OK;
 }
 
+// (straight into the caller's arrays, whose layout the kernels write: by way
+// of a vector the copies took a third of a linear-method block's 13.3 ms)
 static int copy_derivs(qmcw_handle *h, double *dpsi, double *deloc) {
-  const int P = h->nparm;
-  std::vector<double> o((size_t)h->W * 2 * P);
-  HIPCHK(h, hipMemcpyAsync(o.data(), h->der, o.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+  const size_t n = (size_t)h->W * h->nparm * sizeof(double);
+  if (dpsi) HIPCHK(h, hipMemcpyAsync(dpsi, h->der, n, hipMemcpyDeviceToHost, h->stream));
+  if (deloc) HIPCHK(h, hipMemcpyAsync(deloc, h->del(), n, hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
-  for (int w = 0; w < h->W; w++) {
-    const double *r = o.data() + (size_t)w * 2 * P;
-    if (dpsi) memcpy(dpsi + (size_t)w * P, r, P * sizeof(double));
-    if (deloc) memcpy(deloc + (size_t)w * P, r + P, P * sizeof(double));
-  }
   return QMCW_OK;
 }
 
@@ -2370,10 +2400,10 @@ extern "C" int qmcw_accum_add_static(qmcw_handle *h, double *acc) {
   const int nb = (P + kAccBlk - 1) / kAccBlk;
   const int64_t n = accum_doubles(P);
   hipLaunchKernelGGL(k_accum_gemm, dim3(nb * nb, nch), dim3(64), 0, h->stream, (const double *)h->der,
-                     2 * P, P, (const double *)h->A.st, (int64_t)h->A.L.stride, (int64_t)h->A.L.eloc,
+                     (const double *)h->del(), P, (const double *)h->A.st, (int64_t)h->A.L.stride, (int64_t)h->A.L.eloc,
                      h->W, part);
   hipLaunchKernelGGL(k_accum_vec, dim3((P + 1 + 63) / 64, nch), dim3(64), 0, h->stream,
-                     (const double *)h->der, 2 * P, P, (const double *)h->A.st,
+                     (const double *)h->der, (const double *)h->del(), P, (const double *)h->A.st,
                      (int64_t)h->A.L.stride, (int64_t)h->A.L.eloc, h->W, partv);
   hipLaunchKernelGGL(k_accum_reduce, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h->stream,
                      (const double *)part, (const double *)partv, nch, P, acc);

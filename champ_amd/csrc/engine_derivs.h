@@ -545,7 +545,7 @@ __global__ QMCW_HEAVY void k_deriv_nlpp(KArgs A) {
 // alpha_deloc_bld, dy_bld, dg_bld, csf_derivs_bld
 // (qmc/deriv_fast_mod.f90:174-823), dpsi_orb_bld / deloc_orb_bld
 // (qmc/deriv_orb_mod.f90:1486-1630) and the Jastrow denergy of
-// qmc/vmc/hpsi.f90:366-374.  out[w * 2P + p] = dpsi, out[w * 2P + P + p] = deloc.
+// qmc/vmc/hpsi.f90:366-374.  dpsi[w * P + p] and deloc[w * P + p].
 // With LDS the intermediates (derivs_lds_doubles of them) stay in LDS, a
 // wavefront per walker: each of the dozen dependent phases then waits for LDS
 // instead of L2, which bounded the kernel (37 of 600 VALU instructions per
@@ -558,7 +558,7 @@ __host__ __device__ inline int derivs_lds_doubles(const DevSys &S) {
   return n;
 }
 template <int G, bool LDS>
-__global__ QMCW_HEAVY void k_derivs(KArgs A, double *out) {
+__global__ QMCW_HEAVY void k_derivs(KArgs A, double *dpsi, double *deloc) {
   QMCW_GROUP_SETUP
   const int N = S.N, NO = S.NO, P = S.nparm;
   const WLayout &L = A.L;
@@ -746,7 +746,7 @@ __global__ QMCW_HEAVY void k_derivs(KArgs A, double *out) {
     __syncthreads();
   }
   // ---- outputs
-  double *o1 = out + (int64_t)w * 2 * P, *o2 = o1 + P;
+  double *o1 = dpsi + (int64_t)w * P, *o2 = deloc + (int64_t)w * P;
   for (int ip = lane; ip < S.npcsf; ip += G) {
     const int icsf = cst(S.pcsf)[ip];
     double dd = 0.0, de = 0.0;
