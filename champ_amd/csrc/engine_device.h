@@ -821,12 +821,12 @@ __device__ __forceinline__ T jas_point_val(const DevSys &S, int i, const double 
 // e-n Pade + polynomial of one electron summed over centres
 template <typename T>
 __device__ void jas_en(const DevSys &S, const double *ri_v, const double *rvi, T &f,
-                       T *g, T &lap) {
+                       T *g, T &lap, int ic0 = 0, int dic = 1) {
   const T k = T(S.scalek);
   f = 0;
   g[0] = g[1] = g[2] = 0;
   lap = 0;
-  for (int ic = 0; ic < S.M; ic++) {
+  for (int ic = ic0; ic < S.M; ic += dic) {
     int it = cst(S.iwctype)[ic];
     const cptr<double> a = cst(S.a4) + it * (S.norda + 1);
     T r = (T)ri_v[ic], u, d1, d2;

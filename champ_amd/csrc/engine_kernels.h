@@ -141,7 +141,8 @@ __device__ __forceinline__ float bf16r(float x) {
 // pseudopotential projection, group_gproj).
 // The coefficients come from L2 (a lane an orbital): the next eight are on
 // their way while eight are used; with four loaded and waited for at a time
-// this loop was half of the orbitals' 31,000 cycles of a 38-electron move.
+// the orbitals took 31,000 cycles of a 38-electron move (21,500 here, fewer
+// with contract5_rows).
 template <typename T>
 __device__ __forceinline__ void contract5(cptr<double> coefT, int NO, int NB, int lab,
                                           const T *__restrict__ ph, double *o) {
@@ -174,6 +175,71 @@ __device__ __forceinline__ void contract5(cptr<double> coefT, int NO, int NB, in
     a3 += cf * (double)p[3]; a4 += cf * (double)p[4];
   }
   o[0] = a0; o[1] = a1; o[2] = a2; o[3] = a3; o[4] = a4;
+}
+
+// contract5 of the orbitals j0 .. j0 + 16 R - 1 (those below NO) by a wide group:
+// sixteen lanes take R orbitals each, the sixteens share the basis.  With an
+// orbital per lane every basis function was read by all 64 lanes for one
+// orbital each, and the LDS's return path (20 clocks per function in FP64, of
+// eight wavefronts) bounded the contraction of the 98-electron chain's move;
+// 19 orbitals left most lanes idle.  With the e-n term a centre per lane: DMC
+// generation of the chain 143.5 -> 136.8 ms, its mixed block 37.9 -> 34.8, a
+// 38-electron block 9.07 -> 8.53.
+constexpr int kRowLanes = 16;
+template <typename T, int G, int R>
+__device__ __forceinline__ void contract5_rows(cptr<double> coef, int NO, int NB, int j0,
+                                               const T *__restrict__ ph, double *orbe, int lane) {
+  constexpr int P = G / kRowLanes, U = R == 4 ? 2 : 4;
+  const int jl = lane % kRowLanes, nb = (NB + P - 1) / P;
+  const int b0 = min(NB, (lane / kRowLanes) * nb), b1 = min(NB, b0 + nb);
+  int lab[R];
+  double a[R][5];
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    lab[r] = min(j0 + r * kRowLanes + jl, NO - 1);
+#pragma unroll
+    for (int c = 0; c < 5; c++) a[r][c] = 0.0;
+  }
+  double cf[U][R];
+#pragma unroll
+  for (int u = 0; u < U; u++)
+#pragma unroll
+    for (int r = 0; r < R; r++) cf[u][r] = coef[(int64_t)min(b0 + u, NB - 1) * NO + lab[r]];
+  for (int b = b0; b < b1; b += U) {
+    double nx[U][R];           // the next functions' coefficients, on their way meanwhile
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int r = 0; r < R; r++) nx[u][r] = coef[(int64_t)min(b + U + u, NB - 1) * NO + lab[r]];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const T *p = ph + 5 * min(b + u, NB - 1);
+      const bool in = b + u < b1;
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        const double k = in ? cf[u][r] : 0.0;
+#pragma unroll
+        for (int c = 0; c < 5; c++) a[r][c] += k * (double)p[c];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int r = 0; r < R; r++) cf[u][r] = nx[u][r];
+  }
+#pragma unroll
+  for (int d = kRowLanes; d < G; d *= 2)
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+      for (int c = 0; c < 5; c++) a[r][c] += __shfl_xor(a[r][c], d);
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const int j = j0 + r * kRowLanes + jl;
+    if (lane < kRowLanes && j < NO)
+#pragma unroll
+      for (int c = 0; c < 5; c++) orbe[5 * j + c] = a[r][c];
+  }
 }
 
 // contract5 of NB more functions onto o, in the same order as one call would add them
@@ -1518,19 +1584,15 @@ __device__ __forceinline__ void orbitals_1e(const KArgs &A, int s, int nocc, con
     eval_shell<T>(S, sh, (T)rven[3 * ic], (T)rven[3 * ic + 1], (T)rven[3 * ic + 2], (T)ren[ic], 1, phi);
   }
   __syncthreads();
-  // half as many orbitals as lanes, or fewer: the lanes share the basis too
-  const int parts = nocc <= G / 4 ? 4 : nocc <= G / 2 ? 2 : 1;
-  if (G >= 32 && parts > 1) {
-    const int wd = G / parts, j = lane % wd, nb = (S.NB + parts - 1) / parts;
-    const int b0 = min(S.NB, (lane / wd) * nb), b1 = min(S.NB, b0 + nb);
-    double o[5] = {0, 0, 0, 0, 0};
-    if (j < nocc) contract5<T>(cst(S.coef_occ[s]) + (int64_t)b0 * nocc, nocc, b1 - b0, j, phi + 5 * b0, o);
-    for (int d = wd; d < G; d *= 2)
-#pragma unroll
-      for (int c = 0; c < 5; c++) o[c] += __shfl_xor(o[c], d);
-    if (lane < nocc)
-#pragma unroll
-      for (int c = 0; c < 5; c++) orbe[5 * j + c] = o[c];
+  // wide groups: see contract5_rows
+  if (G >= 32) {
+    for (int j0 = 0; j0 < nocc; j0 += 4 * kRowLanes) {
+      const int left = nocc - j0;
+      const cptr<double> co = cst(S.coef_occ[s]);
+      if (left <= kRowLanes) contract5_rows<T, G, 1>(co, nocc, S.NB, j0, phi, orbe, lane);
+      else if (left <= 2 * kRowLanes) contract5_rows<T, G, 2>(co, nocc, S.NB, j0, phi, orbe, lane);
+      else contract5_rows<T, G, 4>(co, nocc, S.NB, j0, phi, orbe, lane);
+    }
     return;
   }
   for (int j = lane; j < nocc; j += G)
@@ -1632,18 +1694,35 @@ __device__ __forceinline__ void ratio_1e_b(const KArgs &A, int bid_, int ie, int
       een_tables<T, ORD, G>(S, ren, rven, etab, lane);
     __syncthreads();
   }
+  // The e-n diagonal term, wide groups a centre per lane: summed on the one
+  // lane that the pair list leaves free, with the others waiting, it took
+  // about 1,000 cycles a centre (50 in a 98-electron chain's move of 640,000).
+  constexpr bool kEnLanes = G >= 32;
+  double en[5] = {0, 0, 0, 0, 0};
+  if (kEnLanes) {
+    T f, g[3], lp;
+    jas_en<T>(S, ren, rven, f, g, lp, lane, G);
+    en[0] = gsum<G>((double)f);
+    for (int q = 0; q < 3; q++) en[1 + q] = gsum<G>((double)g[q]);
+    en[4] = gsum<G>((double)lp);
+  }
   for (int j = lane; j < N; j += G) {
     if (j == ie) {  // e-n diagonal term, on the lane the pair list leaves free
-      T f, g[3], lp;
-      jas_en<T>(S, ren, rven, f, g, lp);
-      fsn[ie] = f;
-      for (int q = 0; q < 3; q++) fijn_i[3 * ie + q] = g[q];
-      lapn[ie] = lp;
-      dsum += (double)f - fso[ie * N + ie];
-      gix += (double)g[0] - fijo[3 * (ie * N + ie)];
-      giy += (double)g[1] - fijo[3 * (ie * N + ie) + 1];
-      giz += (double)g[2] - fijo[3 * (ie * N + ie) + 2];
-      lapi += lp;
+      if (!kEnLanes) {
+        T f, g[3], lp;
+        jas_en<T>(S, ren, rven, f, g, lp);
+        en[0] = f;
+        for (int q = 0; q < 3; q++) en[1 + q] = g[q];
+        en[4] = lp;
+      }
+      fsn[ie] = en[0];
+      for (int q = 0; q < 3; q++) fijn_i[3 * ie + q] = en[1 + q];
+      lapn[ie] = en[4];
+      dsum += en[0] - fso[ie * N + ie];
+      gix += en[1] - fijo[3 * (ie * N + ie)];
+      giy += en[2] - fijo[3 * (ie * N + ie) + 1];
+      giz += en[3] - fijo[3 * (ie * N + ie) + 2];
+      lapi += en[4];
       continue;
     }
     int hi = j < ie ? ie : j, lo = j < ie ? j : ie;
