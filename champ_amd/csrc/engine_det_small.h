@@ -79,8 +79,8 @@ void k_det_small(KArgs A) {
   for (int i = 0; i < nmax; i++) {
     const int col = i * ns;
     const bool on = i < ns;
-    double am = -1.0, vm = 0.0;
-    int km = ns;
+    double am = -1.0, vm = __builtin_nan("");
+    int km = i;
     if (on)
       for (int k = i + l; k < ns; k += H) {
         const double v = a[ipiv[k] + col];

@@ -269,9 +269,10 @@ __device__ double group_matinv(double *a, double *tmp, int n, int lane, int *ipi
   bool singular = false;
   for (int i = 0; i < n; i++) {
     const int col = i * n;
-    // matinv scans k = i..n-1 keeping the first strictly larger |a(ipiv(k), i)|
-    double am = -1.0, vm = 0.0;
-    int km = n;
+    // matinv scans k = i..n-1 keeping the first strictly larger |a(ipiv(k), i)|;
+    // where no element compares (all NaN) it stays on row i with a NaN pivot
+    double am = -1.0, vm = __builtin_nan("");
+    int km = i;
     for (int k = i + lane; k < n; k += G) {
       double v = a[ipiv[k] + col];
       if (fabs(v) > am) { am = fabs(v); vm = v; km = k; }
@@ -339,8 +340,8 @@ __device__ double group_gj_lds(double *la, int n, int lane, int *ipiv, bool *sin
   bool singular = false;
   for (int i = 0; i < n; i++) {
     const int col = i * n;
-    double am = -1.0, vm = 0.0;
-    int km = n;
+    double am = -1.0, vm = __builtin_nan("");
+    int km = i;
     for (int k = i + lane; k < n; k += G) {
       double v = la[ipiv[k] + col];
       if (fabs(v) > am) { am = fabs(v); vm = v; km = k; }

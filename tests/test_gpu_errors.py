@@ -46,3 +46,33 @@ def test_singular_slater_matrix_is_reported(name):
     e.set_walkers(x)
     g = e.psi_at()
     assert np.isfinite(g["logpsid"]).all() and np.isfinite(g["eloc"]).all()
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf], ids=["nan", "inf"])
+@pytest.mark.parametrize("name,switch", [("be", None), ("c2", None), ("c2", "QMCW_NO_DET_SMALL"), ("mol", None),
+                                         ("mol", "QMCW_NO_LDS")])
+def test_non_finite_walker_is_reported(monkeypatch, name, switch, bad):
+    """A coordinate that is no number leaves no pivot that compares in its
+    walker's Slater matrix (k_det_small, group_matinv and group_gj_lds): the
+    call reports QMCW_ERR_NAN and the other walkers keep their values."""
+    if switch:
+        monkeypatch.setenv(switch, "1")
+    s = {"be": lambda: system.be_atom(1), "c2": lambda: system.c2_dimer(2),
+         "mol": lambda: system.random_molecule(77, nelec=34, ncent=3, zeff=6.0)}[name]()
+    W = 11
+    x = system.random_walkers(s, W, seed=17)
+    e = Engine(s, W)
+    e.set_walkers(x)
+    ref = e.psi_at()
+    N = s.nelec
+    x[4, N - 1, 1] = bad
+    e.set_walkers(x)
+    out = {k: np.zeros_like(ref[k]) for k in ref}
+    p = lambda a: a.ctypes.data_as(C.POINTER(C.c_double))
+    st = e.lib.qmcw_eval_full(e.h, *[p(out[k]) for k in ("logpsid", "sign", "psij", "grad", "divv", "eloc", "epot")])
+    assert st == abi.QMCW_ERR_NAN
+    assert not np.isfinite(out["eloc"][4])
+    ok = [w for w in range(W) if w != 4]
+    for k in ref:
+        assert np.array_equal(out[k][ok], ref[k][ok]), k
+    e.close()
