@@ -1171,14 +1171,16 @@ __device__ void eval_shell(const DevSys &S, int s, T x, T y, T z, T r, int want,
 // scalar load of a shell's description and of its primitives serves all of
 // the type's centres and the exponentials of two centres are independent.
 // Shell by shell over the centres, each with its own chain of dependent
-// scalar loads, the wavefront waited for those most of the time.
+// scalar loads, the wavefront waited for those most of the time.  The sum over
+// a type's centres is FP64 in every engine: in FP32 its error grew with the
+// centres (128 of a type: 7.7e-8 of the nonlocal energy, 2.1e-8 so).
 template <typename T, int L, typename GP>
-__device__ __forceinline__ T type_shell_dot(const DevSys &S, const TypeShell &d, int c0, int c1,
+__device__ __forceinline__ double type_shell_dot(const DevSys &S, const TypeShell &d, int c0, int c1,
                                             const double *xn, const GP *gp) {
   const cptr<TypeCent> tc = (cptr<TypeCent>)S.tcent;
   const cptr<double> tp = cst(S.tprim);
   const bool gauss = (S.basis_type == QMCW_BASIS_GAUSSIAN);
-  T acc = 0;
+  double acc = 0;
   for (int c = c0; c < c1; c += 2) {
     const int cs[2] = {c, c + 1 < c1 ? c + 1 : c};
     T x[2], y[2], z[2], arg[2], g[2] = {T(0), T(0)};
@@ -1218,7 +1220,7 @@ __device__ __forceinline__ T type_shell_dot(const DevSys &S, const TypeShell &d,
 #pragma unroll
       for (int q = 0; q < 2 * L + 1; q++)
         if (d.bas[q] >= 0) a += T(gp[b0[u] + d.bas[q]]) * Sv[q];
-      acc += a * g[u];
+      acc += (double)(a * g[u]);
     }
   }
   return acc;
@@ -1235,7 +1237,7 @@ __device__ __forceinline__ double point_ratio(const DevSys &S, const double *xn,
       d.l = w[0]; d.a = w[1]; d.num = w[2]; d.p0 = w[3]; d.p1 = w[4];
 #pragma unroll
       for (int q = 0; q < kMaxShellM; q++) d.bas[q] = w[5 + q];
-      T v;
+      double v;
       switch (d.l) {
         case 0: v = type_shell_dot<T, 0, GP>(S, d, c0, c1, xn, gp); break;
         case 1: v = type_shell_dot<T, 1, GP>(S, d, c0, c1, xn, gp); break;
@@ -1244,7 +1246,7 @@ __device__ __forceinline__ double point_ratio(const DevSys &S, const double *xn,
         case 4: v = type_shell_dot<T, 4, GP>(S, d, c0, c1, xn, gp); break;
         default: v = type_shell_dot<T, 5, GP>(S, d, c0, c1, xn, gp); break;
       }
-      rd += (double)v;
+      rd += v;
     }
   }
   return rd;

@@ -1,0 +1,64 @@
+"""The determinant ratio of a quadrature point in the mixed engines, whose
+basis values are FP32 and whose sums are FP64: two electrons in one orbital
+that adds the same s function of 128 centres, so that the values'
+roundings (a few units of 2^-24 each) average to 2^-24 / sqrt(centres) and
+what is left shows how the sum was formed.  No Jastrow factor; the nonlocal
+pseudopotential's energy against the FP64 engine's."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+from champ_amd import system
+from champ_amd.engine import Engine
+
+pytestmark = pytest.mark.gpu
+
+M = 128
+
+
+def _sum_of_centres():
+    s = system.random_molecule(11, nelec=2, ncent=M, zeff=4.0)
+    s.prim_zeta = s.prim_zeta * 0.01           # wide: every centre counts everywhere
+    nb = s.coef.shape[1] // M
+    s.coef = np.zeros_like(s.coef[:1])
+    s.coef[0, ::nb] = 1.0
+    s.a4, s.b, s.c = np.zeros_like(s.a4), np.zeros_like(s.b), np.zeros_like(s.c)
+    return s
+
+
+def _local_only(s):
+    """The same system without its nonlocal channels."""
+    off, keep = np.asarray(s.ecp_off), np.asarray(s.lpotp1)
+    coef = np.array(s.ecp_coef, float)
+    lmax = (len(off) - 1) // len(keep)
+    for t in range(len(keep)):
+        for l in range(lmax):
+            if l != keep[t] - 1:
+                coef[off[t * lmax + l]:off[t * lmax + l + 1]] = 0.0
+    return dataclasses.replace(s, ecp_coef=coef)
+
+
+def _epot(s, x, prec):
+    e = Engine(s, len(x), prec)
+    e.set_walkers(x)
+    v = e.psi_at()["epot"]
+    e.close()
+    return v
+
+
+@pytest.mark.parametrize("tiles", ["0", "2"])
+def test_sum_over_centres_is_fp64(monkeypatch, tiles):
+    monkeypatch.setenv("QMCW_NLPP_TILES", tiles)
+    s = _sum_of_centres()
+    x = system.random_walkers(s, 64, seed=3, sigma=0.6)
+    v = _epot(s, x, "fp64")
+    vnl = v - _epot(_local_only(s), x, "fp64")
+    near = np.abs(vnl) > 1e-2
+    assert near.sum() >= 32
+    err = ((_epot(s, x, "mixed") - v) / vnl)[near]
+    rms = float(np.sqrt(np.mean(err ** 2)))
+    print("relative error of the nonlocal energy", rms, np.abs(err).max())
+    # one FP32 rounding of the common factor gp (2^-24 at most) and the
+    # averaged ones of the values
+    assert rms < 2.0 ** -24
