@@ -2,7 +2,8 @@
 // (the optimisation sample): Jastrow parameter derivatives, the
 // pseudopotential pieces (psp_nonloc_orb over all orbitals, dpe), the
 // orbital-resolved local energy and the CSF / Jastrow / orbital-rotation
-// blocks.  Everything here runs in FP64.
+// blocks.  All sums here are FP64; in the mixed engines the basis values and
+// the points' Jastrow factors that they take are FP32.
 #pragma once
 #include "engine_kernels.h"
 

@@ -1171,9 +1171,11 @@ __device__ void eval_shell(const DevSys &S, int s, T x, T y, T z, T r, int want,
 // scalar load of a shell's description and of its primitives serves all of
 // the type's centres and the exponentials of two centres are independent.
 // Shell by shell over the centres, each with its own chain of dependent
-// scalar loads, the wavefront waited for those most of the time.  The sum over
-// a type's centres is FP64 in every engine: in FP32 its error grew with the
-// centres (128 of a type: 7.7e-8 of the nonlocal energy, 2.1e-8 so).
+// scalar loads, the wavefront waited for those most of the time.  The products
+// with gp and all sums are FP64 in every engine (the points' weights of the
+// derivatives come from here): with FP32 products and sums the nonlocal energy
+// of 128 centres of a type was 7.7e-8 from 64 bits, with FP32 products alone
+// 2.1e-8, so it is 4.4e-9.
 template <typename T, int L, typename GP>
 __device__ __forceinline__ double type_shell_dot(const DevSys &S, const TypeShell &d, int c0, int c1,
                                             const double *xn, const GP *gp) {
@@ -1215,12 +1217,13 @@ __device__ __forceinline__ double type_shell_dot(const DevSys &S, const TypeShel
     if (c + 1 >= c1) g[1] = T(0);
 #pragma unroll
     for (int u = 0; u < 2; u++) {
-      T Sv[2 * L + 1], Sg[2 * L + 1][3], a = 0;
+      T Sv[2 * L + 1], Sg[2 * L + 1][3];
+      double a = 0;
       solid_harm<T>(L, x[u], y[u], z[u], Sv, Sg);
 #pragma unroll
       for (int q = 0; q < 2 * L + 1; q++)
-        if (d.bas[q] >= 0) a += T(gp[b0[u] + d.bas[q]]) * Sv[q];
-      acc += (double)(a * g[u]);
+        if (d.bas[q] >= 0) a += gp[b0[u] + d.bas[q]] * (double)Sv[q];
+      acc += a * (double)g[u];
     }
   }
   return acc;

@@ -59,6 +59,28 @@ def test_sum_over_centres_is_fp64(monkeypatch, tiles):
     err = ((_epot(s, x, "mixed") - v) / vnl)[near]
     rms = float(np.sqrt(np.mean(err ** 2)))
     print("relative error of the nonlocal energy", rms, np.abs(err).max())
-    # one FP32 rounding of the common factor gp (2^-24 at most) and the
-    # averaged ones of the values
-    assert rms < 2.0 ** -24
+    # what the averaged roundings of the values may come to, and less than
+    # one FP32 rounding of the factor gp that all centres share
+    assert rms < 2.0 ** -26
+
+
+@pytest.mark.parametrize("tiles", ["0", "2"])
+def test_derivative_weights_are_fp64(monkeypatch, tiles):
+    """The points' factors of the pseudopotential derivatives: dE_L/dp of
+    the e-n parameters of the type with the pseudopotential, whose nonlocal
+    part is the weighted sum over the points."""
+    monkeypatch.setenv("QMCW_NLPP_TILES", tiles)
+    s = system.molecule_derivs(_sum_of_centres())
+    x = system.random_walkers(s, 64, seed=3, sigma=0.6)
+    de = {}
+    for prec, t in (("fp64", s), ("mixed", s), ("local64", _local_only(s)), ("local", _local_only(s))):
+        e = Engine(t, 64, "mixed" if prec in ("mixed", "local") else "fp64")
+        e.set_walkers(x)
+        de[prec] = e.derivs()[1]
+        e.close()
+    dv = de["fp64"] - de["local64"]
+    err = (de["mixed"] - de["local"]) - dv
+    live = np.abs(dv).max(axis=0) > 1e-3 * np.abs(dv).max()
+    rms = np.sqrt(np.mean(err[:, live] ** 2, axis=0) / np.mean(dv[:, live] ** 2, axis=0))
+    print("relative error of the nonlocal derivatives", rms.max(), np.median(rms), live.sum(), dv.shape)
+    assert live.any() and rms.max() < 2.0 ** -26
