@@ -81,6 +81,7 @@ struct qmcw_handle {
   int split_forced = 0;      // QMCW_SPLIT_MOVE set: the autotuner keeps split_move
   int lds_y = 1;             // LDS staging of eval_y in the move kernels
   int ncu = 256;             // compute units of the device (set at create)
+  int lds_max = 64 * 1024;   // LDS bytes a block may have (set at create)
   double *acc = nullptr, *acc_part = nullptr, *acc_partv = nullptr;  // product sums and chunk partials
   int acc_nch = 0;
   // DMC population (qmcw_dmc_begin / qmcw_dmc_step)
@@ -615,11 +616,13 @@ static void det_lds_inv(const qmcw_handle *h, KArgs &A, size_t &smem) {
 // 6,660, FP64); below it the lane groups fill the GPU when there are many
 // walkers (8, 2, 16,384: 555 against 1,041) and the tiles when there are few
 // (8, 2, 1,024: 235 against 104), which the autotuner finds out.  A block
-// gets as many wavefronts as leave two on every SIMD.
+// gets as many wavefronts as leave two on every SIMD.  Systems whose pair
+// flags outgrow a block's LDS (some 700,000 pairs) keep the lane groups.
 constexpr int kNlppTilePairs = 160;
 static int nlpp_tile_waves(const qmcw_handle *h) {
   const DevSys &S = h->A.S;
   if (S.nloc == 0 || S.nordc < 2 || S.nctype * S.nterms > kMaxCtype * kMaxTerms) return 0;
+  if (kNlppTilesStatic + sizeof(double) * nlpp_tiles_lds((int64_t)S.N * S.M) > (size_t)h->lds_max) return 0;
   if (h->nlpp_tiles_env >= 0) return std::min(h->nlpp_tiles_env, kNlppWaves);
   if (h->nlpp_waves >= 0) return h->nlpp_waves;      // the autotuner's choice
   if (S.N * S.M < kNlppTilePairs) return 0;
@@ -1435,6 +1438,9 @@ extern "C" int qmcw_create(const qmcw_system *s, int32_t nwalk, int32_t precisio
     if (hipGetDevice(&dev) == hipSuccess &&
         hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
       h->ncu = n;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&n, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && n > 0)
+      h->lds_max = n;
   }
   if (hipStreamSynchronize(h->stream) != hipSuccess) { qmcw_destroy(h); return fail(nullptr, QMCW_ERR_HIP, "init sync"); }
   *out = h;

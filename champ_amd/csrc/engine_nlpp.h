@@ -207,7 +207,10 @@ __device__ __forceinline__ void nlpp_tile(const DevSys &S, NlppTile<T, ORD> &tl,
 
 // doubles of dynamic LDS of a block: the flags of the (electron, centre)
 // pairs in range, a bit each, and their running counts
-__host__ __device__ inline int nlpp_tiles_lds(int npairs) { return (npairs + 63) / 64 * 3 / 2 + 1; }
+__host__ __device__ inline int64_t nlpp_tiles_lds(int64_t npairs) { return (npairs + 63) / 64 * 3 / 2 + 1; }
+// most bytes of its other LDS (the largest order in FP64)
+constexpr size_t kNlppTilesStatic =
+    kNlppWaves * sizeof(NlppTile<double, 7>) + sizeof(double) * (kMaxCtype * kMaxTerms + 2 * kNlppWaves);
 
 // k_full_nlpp of one walker by a block of 64 to 64 kNlppWaves lanes
 template <typename T, int ORD>

@@ -6,6 +6,7 @@ shells.  FP64 against the oracle (bounds of the molecules' parity tests);
 mixed against the lane-group kernel of the same precision, whose FP32 sums
 run in another order (2^-24 per operation over the few thousand terms of a
 point's Jastrow, times |V_nl| of a few Ha, stays below 1e-4)."""
+import dataclasses
 import os
 import sys
 
@@ -77,3 +78,29 @@ def test_batch_of_tiles_and_lane_groups(monkeypatch):
     from test_gpu_batch import test_one_launch_batch_matches_oracle
     monkeypatch.setenv("QMCW_NLPP_TILES", "4")
     test_one_launch_batch_matches_oracle(monkeypatch, "0")
+
+
+@pytest.mark.parametrize("ncent", [1600, 2900])
+def test_pair_flags_beyond_the_lds(monkeypatch, ncent):
+    """256 electrons: the flags of 410,000 pairs take 77 KB of a block's
+    160 KB of LDS, those of 742,000 would take 139 KB beside the tiles' own 26
+    and stay in lane groups.  Against the lane groups, whose FP64 sums run in
+    another order."""
+    s = system.random_molecule(12, nelec=2, ncent=1, zeff=4.0)
+    side = int(np.ceil(ncent ** (1 / 3)))
+    grid = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3)[:ncent] * 2.5
+    g = np.random.default_rng(2)
+    types = np.where(np.arange(ncent) < 128, 1, 0).astype(np.int32)
+    nb = int(np.diff(s.ctype_bas_off)[types].sum())
+    s = dataclasses.replace(s, nelec=256, nup=128, cent=grid, iwctype=types,
+                            coef=g.normal(0.0, 0.3, (128, nb)), det_up=np.arange(128, dtype=np.int32)[None],
+                            det_dn=np.arange(128, dtype=np.int32)[None])
+    x = system.random_walkers(s, 1, seed=9, sigma=0.5)
+    out = []
+    for tiles in ("0", "4"):
+        monkeypatch.setenv("QMCW_NLPP_TILES", tiles)
+        e = Engine(s, 1)
+        e.set_walkers(x)
+        out.append(e.psi_at()["epot"][0])
+        e.close()
+    assert np.isfinite(out[0]) and abs(out[1] - out[0]) < 1e-9 * abs(out[0])
