@@ -73,8 +73,9 @@ def test_dmc_generations_on_tiles(monkeypatch, tmoves):
     test_dmc_generations_match_oracle("c2_dimer", 0.3, tmoves)
 
 
-def test_batch_of_tiles_and_lane_groups(monkeypatch):
-    """One launch sequence over systems on either side of the rule."""
+def test_batch_of_tiles(monkeypatch):
+    """One launch sequence with every pseudopotential on tiles (by the rule,
+    test_gpu_batch.py has systems on either side of it)."""
     from test_gpu_batch import test_one_launch_batch_matches_oracle
     monkeypatch.setenv("QMCW_NLPP_TILES", "4")
     test_one_launch_batch_matches_oracle(monkeypatch, "0")

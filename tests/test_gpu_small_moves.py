@@ -1,12 +1,16 @@
 """The fused move of few electrons with its pending record in LDS
 (k_move_small): electrons up to the lane group's width, one or several passes
-over the centres' basis functions, both movers, the last block partly empty.
+over the centres' basis functions, both movers, more occupied orbitals than
+its matrix tiles take, the last block partly empty.
 Against k_ratio_1e (QMCW_NO_MOVE_SMALL), whose operations it repeats up to
 the order of a matrix product's sums: identical decisions, local energies to
 1e-10."""
+import dataclasses
+
 import numpy as np
 import pytest
 
+import oracle
 from champ_amd import rng, system
 from champ_amd.engine import Engine
 
@@ -59,3 +63,48 @@ def test_equals_the_general_kernel(monkeypatch, name, G, imetro, prec):
     tol, floor = (1e-10, 1e-8) if prec == "fp64" else (1e-4, 10.0)
     assert np.max(np.abs(a[2] - b[2]) / (np.abs(b[2]) + floor)) < tol
 
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("name,G", [("c2", 8), ((8, 3), 8), ((15, 6), 16)], ids=str)
+def test_passes_over_the_centres(monkeypatch, name, G, prec):
+    """So many walkers that a block's LDS does not hold all basis values at
+    once (20 and 10 blocks to a compute unit): one centre a pass with two and
+    three centres, two centres a pass with six."""
+    s = _system(name)
+    W = 20011
+    a = _walk(s, W, G, prec)[2]
+    monkeypatch.setenv("QMCW_NO_MOVE_SMALL", "1")
+    b = _walk(s, W, G, prec)[2]
+    same = np.all(a[0] == b[0], axis=(1, 2)) & (a[1] == b[1])
+    # FP32 rows in another order: a decision turns where the ratio lies within
+    # some 1e-6 of the draw, up to 30 decisions a walker
+    assert same.all() if prec == "fp64" else same.sum() >= W - 20
+    assert np.array_equal(a[3][same], b[3][same])
+    tol, floor = (1e-10, 1.0) if prec == "fp64" else (1e-3, 10.0)
+    assert np.max((np.abs(a[2] - b[2]) / (np.abs(b[2]) + floor))[:, same]) < tol
+
+
+@pytest.mark.parametrize("G", [8, 16])
+@pytest.mark.parametrize("nvirt", [14, 32])
+def test_more_orbitals_than_tiles(monkeypatch, G, nvirt):
+    """18 and 36 occupied orbitals of a spin: beyond 16 at 8 lanes and 32 at
+    16 the orbitals are taken one per lane."""
+    s = system.c2_dimer(2)
+    ref, exc = [0, 1, 2, 3], [[0, 1, 2, a] for a in range(4, 4 + nvirt)]
+    n = 1 + 2 * nvirt
+    g = np.random.default_rng(nvirt)
+    s = dataclasses.replace(s, det_up=np.array([ref] + exc + [ref] * nvirt, np.int32),
+                            det_dn=np.array([ref] + [ref] * nvirt + exc, np.int32),
+                            csf_coef=np.concatenate([[1.0], g.normal(0, 0.1, n - 1)]),
+                            csf_det_off=np.arange(n + 1, dtype=np.int32), csf_det=np.arange(n, dtype=np.int32),
+                            csf_det_coef=np.ones(n))
+    x, seeds, a = _walk(s, 19, G)
+    o = oracle.Oracle(s).vmc_run(x, seeds, 2, 0.4)
+    monkeypatch.setenv("QMCW_NO_MOVE_SMALL", "1")
+    b = _walk(s, 19, G)[2]
+    for r in (b[:2], (o["x"], o["naccept"])):
+        assert np.array_equal(a[0], r[0]) and np.array_equal(a[1], r[1])
+    assert np.array_equal(a[3], b[3]) and np.array_equal(a[3], o["rng"])
+    assert np.max(np.abs(a[2] - b[2]) / (np.abs(b[2]) + 1e-8)) < 1e-10
+    assert np.max(np.abs(a[2] - o["eloc"]) / (np.abs(o["eloc"]) + 1e-8)) < 1e-9
