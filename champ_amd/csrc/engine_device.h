@@ -606,7 +606,8 @@ __device__ __forceinline__ void een_sum_tables(const DevSys &S, const double *rn
 }
 
 // jas_pair_tab for many centres.  The sum over centres of a polynomial in U is
-// a polynomial in U of sums over centres, so the centre loop only adds up, for each power of U, the value,
+// a polynomial in U of sums over centres, so the centre loop only adds up, for
+// each power of U, the value,
 // both electrons' gradient vectors and their laplacian parts; U's derivatives
 // and the cross terms (twice grad U . grad A, a product with the gradient
 // vectors) are formed once per pair.  Per (pair, centre) that is about 190

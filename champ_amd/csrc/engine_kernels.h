@@ -1605,13 +1605,16 @@ __device__ __forceinline__ void orbitals_1e(const KArgs &A, int s, int nocc, con
 // walker's rannyu stream) or take xnew (mode 0), then distancese +
 // jastrow4e + orbitals + dete_update + eval_grad into the pending buffers.
 // out[w][8]: ratio, ln|psid_new|, sign, psij_new, grad(3), lap
-// Whether the move of a system of M centres at lane-group width G takes
-// jas_pair_sum: always in FP32, where it costs nothing with few centres; in
-// FP64 from this many centres on, at the widths such systems run at.  Closing
-// the sums costs about 400 operations a pair, what seven centres save at some
-// 60 each: with two centres the move slowed from 115 to 128 us (registers),
-// with the chain's it quickened from 1,010 to 874.
-constexpr int kSumCentres = 8;
+// Whether k_ratio_1e of a system of M centres at lane-group width G takes
+// jas_pair_sum (k_move_small never does).  Closing the sums costs about 400
+// operations a pair, what seven centres save at some 60 each, and registers.
+// Measured jas_pair_tab -> jas_pair_sum, us per launch.  FP64, 64 lanes: 4
+// centres 39.4 -> 41.5, 8: 44.8 -> 46.3, 12: 52.4 -> 52.9, 14: 47.4 -> 46.6, 16:
+// 54.1 -> 53.3, 24: 66.4 -> 64.0, 40: 157 -> 144; at 8 and 16 lanes, where
+// systems have few centres, no difference.  FP32, 64 lanes: 2: 34.4 -> 33.8, 8:
+// 43.5 -> 42.1, 14: 45.9 -> 44.3, 40: 144 -> 136; at 8 to 32 lanes 2 centres
+// 38.1 -> 39.0, 8: 48.1 -> 47.9, which one kernel for all is worth.
+constexpr int kSumCentres = 14;
 template <typename T>
 __host__ __device__ constexpr bool een_sums(int G, int M) {
   return sizeof(T) == 4 || (G >= 32 && M >= kSumCentres);

@@ -15,7 +15,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
 @pytest.mark.parametrize("M,nordc,G", [(7, 4, 32), (8, 4, 32), (9, 4, 64), (8, 4, 16), (8, 2, 32), (8, 3, 64),
-                                       (8, 5, 32), (8, 6, 64), (8, 7, 32), (1, 4, 32)])
+                                       (8, 5, 32), (8, 6, 64), (8, 7, 32), (1, 4, 32),
+                                       (13, 4, 64), (14, 4, 32), (14, 4, 64), (15, 4, 32), (14, 4, 16), (14, 2, 32),
+                                       (14, 3, 64), (14, 5, 32), (14, 6, 64), (14, 7, 32)])
 def test_walks_match_oracle(M, nordc, G, prec):
     s = system.random_molecule(700 + M, nelec=21, ncent=M, zeff=4.0)
     g = np.random.default_rng(nordc)
