@@ -26,6 +26,8 @@ using namespace qmcw;
 
 static thread_local std::string g_lib_err;
 
+constexpr size_t kPinStage = 512 * 1024;   // doubles of a call's arrays that pinned memory takes (pin_stage)
+
 struct qmcw_handle {
   int W = 0, Wp = 0, G = 16, precision = QMCW_FP64, chunk = 1;
   // lane-group width of each kernel class (jastrow, determinants, pseudopotential, moves)
@@ -56,6 +58,7 @@ struct qmcw_handle {
   double *der = nullptr;     // [2][Wp][nparm] dpsi, then deloc, of the last derivative evaluation
   double *del() const { return der + (size_t)Wp * nparm; }   // deloc, after dpsi
   double *pin = nullptr;      // pinned host memory of a call's results and inputs (pin_*)
+  size_t pin_stage_doubles = 0;   // room for a call's arrays at its end (pin_stage)
   int sample_derivs = 0;     // VMC steps evaluate derivatives (CHAMP's ideriv)
   int der_valid = 0;
   // one VMC step captured as a HIP graph (qmcw_vmc_run_device) and its key
@@ -514,6 +517,12 @@ __global__ void k_gather_full(KArgs A, double *grad, double *lap, double *sc5, i
     for (int b = 0; b < 3; b++)
       if (f & (1 << b)) fl[b] = 1;
   }
+}
+
+// two arrays of m values, one after the other, in pinned host memory
+__global__ void k_gather_pair(const double *a, const double *b, double *out, int64_t m) {
+  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < 2 * m; t += (int64_t)gridDim.x * blockDim.x)
+    out[t] = t < m ? a[t] : b[t - m];
 }
 
 // the error flags alone
@@ -1411,7 +1420,8 @@ extern "C" int qmcw_create(const qmcw_system *s, int32_t nwalk, int32_t precisio
   h->io_doubles = (size_t)h->Wp * std::max(8 + 4 * N, 8);
   if (hipMalloc(&p, h->io_doubles * sizeof(double)) != hipSuccess) { qmcw_destroy(h); return fail(nullptr, QMCW_ERR_NOMEM, "io alloc"); }
   h->allocs.push_back(p); h->io = (double *)p;
-  if (hipHostMalloc(&p, (size_t)h->Wp * 12 * sizeof(double) + 64) != hipSuccess) { qmcw_destroy(h); return fail(nullptr, QMCW_ERR_NOMEM, "pinned alloc"); }
+  h->pin_stage_doubles = std::min(kPinStage, (size_t)h->Wp * std::max(4 * N, 2 * S.nparm));
+  if (hipHostMalloc(&p, ((size_t)h->Wp * 12 + 8 + h->pin_stage_doubles) * sizeof(double)) != hipSuccess) { qmcw_destroy(h); return fail(nullptr, QMCW_ERR_NOMEM, "pinned alloc"); }
   h->pin = (double *)p;
   (void)hipMemsetAsync(h->A.st, 0, stb, h->stream);
   (void)hipMemsetAsync(h->A.sc, 0, scb, h->stream);
@@ -1594,6 +1604,22 @@ static double *pin_x(const qmcw_handle *h) { return h->pin + (size_t)h->Wp * 8; 
 static uint8_t *pin_acc(const qmcw_handle *h) { return (uint8_t *)(h->pin + (size_t)h->Wp * 11); }
 static int *pin_flags(const qmcw_handle *h) { return (int *)(h->pin + (size_t)h->Wp * 12); }
 
+// A call's larger arrays also come through pinned memory while they fit
+// (pin_stage_doubles): a runtime copy into the caller's own pages has waited up
+// to 65 us per array of some 100 KB (psi_at of 1,024 C2-like walkers 371 us by
+// way of a vector, 500 with such copies, 280 so; get_derivs of 64, 242
+// parameters, 132, 264 and 23; psi_at of 16,384, 4 MB, 1,110 -> 1,040).
+static double *pin_stage(const qmcw_handle *h, size_t doubles) {
+  return doubles <= h->pin_stage_doubles ? h->pin + (size_t)h->Wp * 12 + 8 : nullptr;
+}
+
+// Into the caller's array, in pieces too short for memcpy's string and
+// streaming stores, which take twice as long on pages met for the first time
+// (4 MB: 824 -> 443 us; on pages in use 82 -> 70).
+static void copy_out(double *dst, const double *src, size_t n) {
+  for (size_t i = 0; i < n; i += 240) memcpy(dst + i, src + i, std::min<size_t>(240, n - i) * sizeof(double));
+}
+
 static int flags_status(qmcw_handle *h) {
   const int *f = pin_flags(h);
   if (f[0]) return fail(h, QMCW_ERR_SINGULAR, "a Slater matrix is singular");
@@ -1619,18 +1645,21 @@ extern "C" int qmcw_eval_full(qmcw_handle *h, double *logpsid, double *sgn, doub
   HIPCHK(h, hipGetLastError());
   const int N = h->A.S.N;
   const size_t W = h->W;
-  double *dg = h->io, *dl = h->io + W * 3 * N;
+  double *stage = grad || lap ? pin_stage(h, W * 4 * N) : nullptr;
+  double *dg = stage ? stage : h->io, *dl = dg + W * 3 * N;
   int *f = pin_flags(h);
   f[0] = f[1] = f[2] = 0;
   hipLaunchKernelGGL(k_gather_full, dim3((unsigned)((W * (4 * N + 1) + 255) / 256)), dim3(256), 0, h->stream,
                      h->A, dg, dl, h->pin, f, h->W, h->dmc_on ? h->nact : h->W);
   HIPCHK(h, hipGetLastError());
-  if (grad) HIPCHK(h, hipMemcpyAsync(grad, dg, W * 3 * N * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-  if (lap) HIPCHK(h, hipMemcpyAsync(lap, dl, W * N * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+  if (grad && !stage) HIPCHK(h, hipMemcpyAsync(grad, dg, W * 3 * N * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+  if (lap && !stage) HIPCHK(h, hipMemcpyAsync(lap, dl, W * N * sizeof(double), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
+  if (grad && stage) copy_out(grad, dg, W * 3 * N);
+  if (lap && stage) copy_out(lap, dl, W * N);
   double *const dst[5] = {logpsid, sgn, psij, eloc, epot};
   for (int q = 0; q < 5; q++)
-    if (dst[q]) memcpy(dst[q], h->pin + q * W, W * sizeof(double));
+    if (dst[q]) copy_out(dst[q], h->pin + q * W, W);
   return flags_status(h);
 }
 
@@ -2292,13 +2321,23 @@ extern "C" int qmcw_get_eloc(const qmcw_handle *hc, double *eloc) {
   return QMCW_OK;
 }
 
-// (straight into the caller's arrays, whose layout the kernels write: by way
-// of a vector the copies took a third of a linear-method block's 13.3 ms)
+// (through pinned memory, or straight into the caller's arrays, whose layout
+// the kernels write: by way of a vector the copies took a third of a
+// linear-method block's 13.3 ms)
 static int copy_derivs(qmcw_handle *h, double *dpsi, double *deloc) {
-  const size_t n = (size_t)h->W * h->nparm * sizeof(double);
-  if (dpsi) HIPCHK(h, hipMemcpyAsync(dpsi, h->der, n, hipMemcpyDeviceToHost, h->stream));
-  if (deloc) HIPCHK(h, hipMemcpyAsync(deloc, h->del(), n, hipMemcpyDeviceToHost, h->stream));
+  const size_t m = (size_t)h->W * h->nparm, n = m * sizeof(double);
+  double *stage = pin_stage(h, 2 * m);
+  if (stage) {
+    hipLaunchKernelGGL(k_gather_pair, dim3((unsigned)std::min<size_t>(1024, (2 * m + 255) / 256)), dim3(256), 0,
+                       h->stream, (const double *)h->der, (const double *)h->del(), stage, (int64_t)m);
+    HIPCHK(h, hipGetLastError());
+  } else {
+    if (dpsi) HIPCHK(h, hipMemcpyAsync(dpsi, h->der, n, hipMemcpyDeviceToHost, h->stream));
+    if (deloc) HIPCHK(h, hipMemcpyAsync(deloc, h->del(), n, hipMemcpyDeviceToHost, h->stream));
+  }
   HIPCHK(h, hipStreamSynchronize(h->stream));
+  if (dpsi && stage) copy_out(dpsi, stage, m);
+  if (deloc && stage) copy_out(deloc, stage + m, m);
   return QMCW_OK;
 }
 
