@@ -150,7 +150,7 @@ struct SLayout {
   int64_t red;               // reduction scratch (matrix temporaries)
   int64_t phs;               // [64] scalars passed between the phase kernels
   int64_t cup;               // [ndetu0 + ndetu1] det-coefficient sums
-  int64_t qd;                // [G][4M] quadrature-point distances
+  int64_t qd;                // [G][M] quadrature-point distances
   int64_t vnl;               // [N*M][QMCW_MAX_LPOT+1] nonlocal channel values
   int64_t gproj;             // [N][NB] G(:,i)^T coef of the occupied orbitals
   int64_t bt;                // [M][N] e-e-n variable 1 - k scaled(r_j,ic) (as the kernel's T)

@@ -1367,7 +1367,7 @@ extern "C" int qmcw_create(const qmcw_system *s, int32_t nwalk, int32_t precisio
   SL.red = take(std::max(std::max(64, nsm * nsm), noccm * nsm) + 64);
   SL.cup = take(D.ndetu[0] + D.ndetu[1]);
   SL.phs = take(64);
-  SL.qd = take((int64_t)kWave * 4 * M);
+  SL.qd = take((int64_t)kWave * M);
   SL.vnl = take((int64_t)N * M * (QMCW_MAX_LPOT + 1));
   SL.gproj = take((int64_t)N * NB);
   SL.bt = take((int64_t)N * M);
