@@ -1586,7 +1586,7 @@ __device__ __forceinline__ void orbitals_1e(const KArgs &A, int s, int nocc, con
   }
   __syncthreads();
   // wide groups: see contract5_rows
-  if (G >= 32) {
+  if constexpr (G >= 32) {
     for (int j0 = 0; j0 < nocc; j0 += 4 * kRowLanes) {
       const int left = nocc - j0;
       const cptr<double> co = cst(S.coef_occ[s]);
@@ -1594,10 +1594,10 @@ __device__ __forceinline__ void orbitals_1e(const KArgs &A, int s, int nocc, con
       else if (left <= 2 * kRowLanes) contract5_rows<T, G, 2>(co, nocc, S.NB, j0, phi, orbe, lane);
       else contract5_rows<T, G, 4>(co, nocc, S.NB, j0, phi, orbe, lane);
     }
-    return;
+  } else {
+    for (int j = lane; j < nocc; j += G)
+      contract5<T>(cst(S.coef_occ[s]), nocc, S.NB, j, phi, orbe + 5 * j);
   }
-  for (int j = lane; j < nocc; j += G)
-    contract5<T>(cst(S.coef_occ[s]), nocc, S.NB, j, phi, orbe + 5 * j);
 }
 
 // ---------------------------------------------------------------------------
